@@ -8,8 +8,6 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <utility>
-
 #include "common.hpp"
 #include "geom.hpp"
 #include "graph.hpp"
@@ -538,451 +536,6 @@ __global__ void k_cc_final(int32_t* parent, int32_t* labels, int N)
     if (k < N) labels[k] = uf_root(parent, k);
 }
 
-// Border chains (extractBorderPoints cc_functions.cu:348-503) of one frame.
-// The scan: a walk starts at each node, in row-major order, that is neither
-// internal (90) nor without links nor listed; it leaves by the node's first
-// link clockwise from up-left and at each node turns clockwise from the link
-// it came in by.  It is a chain when it comes back to its start through the
-// link just counter-clockwise of the first one; it is abandoned on an
-// internal, listed or discarded node, discarding the node it stepped from.
-// Chain nodes are listed; an abandoned walk leaves its start unlisted (the
-// behaviour that reproduces the chains recorded in alex_png.txt:1-21).
-//
-// Which walks become chains depends on every earlier walk, but where a walk
-// goes does not: the turn rule gives each directed link (node s, link e) one
-// successor (the neighbour t, its first link clockwise after 7 - e), and on
-// a symmetric graph that is a permutation of the directed links whose
-// cycles are the faces of the graph's plane embedding.  A walk from s runs
-// along the cycle of s's first link and closes where that cycle comes back
-// to it; a link into an internal node has no successor (the walk stops
-// there), which cuts some cycles into paths.  So the cycles and paths are
-// laid out first, all links in parallel: list ranking by pointer jumping
-// (Wyllie) finds each link's distance to the end of its path and, on a
-// cycle, the smallest link of the cycle, where the cycle is then cut; each
-// path is written as an array of its links' nodes in walk order.  The scan
-// itself (one wave) then needs, per walk, only the marks of the nodes of a
-// contiguous range of that array, 64 at a time.
-//
-// Directed link id = node * 8 + link.  State per link (uint4): x = next
-// link 2^k steps on (kEnd past the end, kNoLink for slots that are not
-// links of a walkable node), y = steps to it, z = the furthest link reached
-// (the path's last link once x = kEnd), w = the smallest link seen (cycle
-// search) or flags (bit 0: on a cycle, bit 1: first link of its path).
-constexpr int kEnd = -1, kNoLink = -2;
-
-inline size_t round256(size_t v) { return (v + 255) / 256 * 256; }
-
-// successor of directed link (s, e) of a walkable node, or kEnd when the
-// neighbour is internal
-__device__ inline int bc_succ(const uint8_t* g, int W, int s, int e)
-{
-    const int t = s + edy(e) * W + edx(e);
-    const uint32_t vt = g[t];
-    return vt == 90u ? kEnd : t * 8 + cw_turn(vt, 7 - e, +1);
-}
-
-__global__ void k_bc_clear(int* ctr)
-{
-    if (threadIdx.x < 4) ctr[threadIdx.x] = 0;
-}
-
-// ctr[0]: status (DPX_EINVAL: a link leaves the frame or has no reverse
-// link), ctr[1]: entries of the path arrays handed out
-__global__ __launch_bounds__(256) void k_bc_init(const uint8_t* __restrict__ g, int W, int H, uint4* __restrict__ S,
-                                                 int* ctr)
-{
-    const uint32_t id = blockIdx.x * 256u + threadIdx.x, E = 8u * (uint32_t)W * (uint32_t)H;
-    if (id >= E) return;
-    const int s = (int)(id >> 3), e = (int)(id & 7u);
-    const uint32_t v = g[s];
-    if (!((v >> e) & 1u) || v == 90u) {
-        S[id] = make_uint4((uint32_t)kNoLink, 0u, id, 0u);
-        return;
-    }
-    const int ni = s % W + edx(e), nj = s / W + edy(e);
-    if (!in_frame(ni, nj, W, H) || !((g[nj * W + ni] >> (7 - e)) & 1u)) {
-        ctr[0] = DPX_EINVAL;
-        S[id] = make_uint4((uint32_t)kNoLink, 0u, id, 0u);
-        return;
-    }
-    const int nx = bc_succ(g, W, s, e);
-    S[id] = make_uint4((uint32_t)nx, nx >= 0 ? 1u : 0u, nx >= 0 ? (uint32_t)nx : id, id);
-}
-
-// pointer jumping, in -> out; MIN: also the smallest link seen.  A link's
-// state in `in` covers 2^k steps; composed with the state it points to
-// HOPS times it covers (HOPS + 1) 2^k: HOPS = 1 is one doubling round,
-// HOPS = 3 two rounds and HOPS = 7 three in one launch (dependent reads of
-// `in` in place of launches that each read and write every state).
-template <bool MIN, int HOPS>
-__global__ __launch_bounds__(256) void k_bc_jump(const uint4* __restrict__ in, uint4* __restrict__ out, uint32_t E)
-{
-    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
-    if (id >= E) return;
-    uint4 st = in[id];
-#pragma unroll
-    for (int h = 0; h < HOPS; h++) {
-        if ((int)st.x >= 0) {
-            const uint4 x = in[st.x];
-            st = make_uint4(x.x, st.y + x.y, x.z, MIN ? (x.w < st.w ? x.w : st.w) : st.w);
-        }
-    }
-    out[id] = st;
-}
-
-// after the cycle search: links still jumping lie on cycles; each cycle is
-// cut before its smallest link, which becomes the first of its path.  A
-// link on a path is the first of its path when its predecessor (the link
-// that turns into it: from the neighbour across s's link just
-// counter-clockwise of e) is no walkable node's link.
-__global__ __launch_bounds__(256) void k_bc_cut(const uint8_t* __restrict__ g, int W, int H,
-                                                const uint4* __restrict__ F, uint4* __restrict__ G, uint32_t E)
-{
-    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
-    if (id >= E) return;
-    const uint4 st = F[id];
-    if ((int)st.x == kNoLink) {
-        G[id] = st;
-        return;
-    }
-    const int s = (int)(id >> 3), e = (int)(id & 7u);
-    if ((int)st.x >= 0) {
-        const int nx = bc_succ(g, W, s, e);
-        const uint32_t fl = 1u | (id == st.w ? 2u : 0u);
-        G[id] = (uint32_t)nx == st.w ? make_uint4((uint32_t)kEnd, 0u, id, fl) : make_uint4((uint32_t)nx, 1u, (uint32_t)nx, fl);
-        return;
-    }
-    const int a = cw_turn(g[s], e, -1);
-    const int pi = s % W + edx(a), pj = s / W + edy(a);
-    const bool first = !in_frame(pi, pj, W, H) || g[pj * W + pi] == 90u;
-    G[id] = make_uint4((uint32_t)kEnd, st.y, st.z, first ? 2u : 0u);
-}
-
-// the first link of each path takes the path's range of the node array:
-// info[last link] = (offset, length, on a cycle)
-constexpr int kHeadsBlock = 1024;
-
-__global__ __launch_bounds__(kHeadsBlock) void k_bc_heads(const uint4* __restrict__ F, uint4* __restrict__ info,
-                                                          int* ctr, uint32_t E)
-{
-    const uint32_t id = blockIdx.x * (uint32_t)kHeadsBlock + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    const bool ok = id < E && ctr[0] == 0;
-    const uint4 st = ok ? F[id] : make_uint4((uint32_t)kNoLink, 0u, 0u, 0u);
-    const bool link = (int)st.x != kNoLink;
-    if (link && (int)st.x != kEnd) ctr[0] = DPX_EINVAL;  // not at the end: the links are no permutation
-    const bool head = link && (int)st.x == kEnd && (st.w & 2u);
-    // one atomic per block (one per wave made the counter the kernel's
-    // bottleneck): the block's paths take consecutive ranges
-    __shared__ uint64_t s_tot[kHeadsBlock / 64], s_base;
-    const int wave = threadIdx.x >> 6;
-    const uint64_t len = head ? (uint64_t)st.y + 1u : 0u;
-    uint64_t incl = len;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint64_t t = __shfl_up(incl, d);
-        if (lane >= d) incl += t;
-    }
-    if (lane == 63) s_tot[wave] = incl;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t total = 0;
-        for (int w = 0; w < kHeadsBlock / 64; w++) total += s_tot[w];
-        s_base = total == 0 ? 0u
-                 : total > E ? (uint64_t)E + 1u
-                             : (uint64_t)atomicAdd(reinterpret_cast<unsigned*>(&ctr[1]), (unsigned)total);
-    }
-    __syncthreads();
-    if (!head) return;
-    uint64_t base = s_base;
-    for (int w = 0; w < wave; w++) base += s_tot[w];
-    const uint64_t off = base + incl - len;
-    if (off + len > E) {
-        ctr[0] = DPX_EINVAL;
-        return;
-    }
-    info[st.z] = make_uint4((uint32_t)off, (uint32_t)len, st.w & 1u, 0u);
-}
-
-// each link writes its node at its place in its path's array; the first
-// link of a walkable node gives that node's walk (offset, length, place of
-// the start, on a cycle)
-__global__ __launch_bounds__(256) void k_bc_scatter(const uint8_t* __restrict__ g, const uint4* __restrict__ F,
-                                                    const uint4* __restrict__ info, int32_t* __restrict__ A,
-                                                    uint4* __restrict__ rec, const int* ctr, uint32_t E)
-{
-    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
-    if (id >= E || ctr[0] != 0) return;
-    const uint4 st = F[id];
-    if ((int)st.x == kNoLink) return;
-    const uint4 inf = info[st.z];
-    if (st.y >= inf.y || (uint64_t)inf.x + inf.y > E) return;  // (inconsistent only for graphs refused above)
-    const uint32_t pos = inf.y - 1u - st.y;
-    A[inf.x + pos] = (int32_t)(id >> 3);
-    if ((int)(id & 7u) == cw_first_link(g[id >> 3])) rec[id >> 3] = make_uint4(inf.x, inf.y, pos, inf.z);
-}
-
-// The scan, one wave (wave 0 of the block).  Marks are two bitmaps of
-// (N + 31) / 32 words each, in LDS when they fit, else in bits_g: listed
-// (nodes of chains: a candidate that is listed starts no walk) and marked
-// (listed or discarded: a walk stops at such a node), so that a walk's test
-// reads one bit per node.  Which walks run depends on the marks, but what a walk
-// reads does not, so the loads go out in groups and the wave waits once per
-// group, not once per load:
-// - the candidate flags and walk records of kBcBlk batches of 64 nodes are
-//   loaded into registers while the block before is scanned, then staged
-//   in LDS;
-// - the first kBcChunk nodes of the next kBcAhead walks of a batch are
-//   loaded together into registers (a walk whose start a chain lists
-//   meanwhile is skipped);
-// - the rest of a long walk, and a long chain's nodes, kBcChunk2 at a time.
-// The loads of records and of a walk's nodes are unconditional (an index
-// past an end is clamped, its value dropped): a load that the wave may skip
-// leaves the compiler unsure how many are in flight, and it then waits for
-// all of them at the next use.
-// The other three waves read the path arrays, the graph and the records
-// once, so that the scan's loads hit the L2 of its XCD.  The sizes are the
-// fastest of a sweep on 256x224 and 640x480 frames (groups of 1-8 walks,
-// first chunks of 64-256 nodes, later ones of 128-1024, blocks of 4-16
-// batches): 85% of walks end within 64 nodes, and each load the wave
-// issues for a slot it may not need costs more than the wait it saves.
-constexpr int kBcU = 1, kBcChunk = 64 * kBcU, kBcAhead = 2, kBcBlk = 8, kBcU2 = 4, kBcChunk2 = 64 * kBcU2;
-
-__device__ inline int lane_of(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
-
-// place of the node before the first marked one in a chunk of U slots of 64
-// (-1: the node before the chunk); -2 when no node of the chunk is marked
-template <int U>
-__device__ inline int bc_before_mark(const uint64_t (&bal)[U])
-{
-#pragma unroll
-    for (int u = 0; u < U; u++)
-        if (bal[u]) return 64 * u + __builtin_ctzll(bal[u]) - 1;
-    return -2;
-}
-
-// the node at place p (uniform) of a chunk held U per lane
-template <int U>
-__device__ inline int bc_node_at(const int (&nd)[U], int p)
-{
-    int x = 0;
-#pragma unroll
-    for (int u = 0; u < U; u++)
-        if ((p >> 6) == u) x = lane_of(nd[u], p & 63);
-    return x;
-}
-
-template <bool LDS>
-__global__ __launch_bounds__(256) void k_bc_scan(const uint8_t* __restrict__ g, int N, const uint4* __restrict__ rec,
-                                                 const int32_t* __restrict__ A, uint32_t* bits_g, int32_t* nodes,
-                                                 int32_t* sizes, int max_nodes, int max_chains, const int* ctr,
-                                                 int32_t* counts)
-{
-    extern __shared__ uint32_t s_bits[];
-    __shared__ uint4 s_rec[kBcBlk][64];
-    __shared__ uint64_t s_cand[kBcBlk];
-    uint32_t* bits = LDS ? s_bits : bits_g;
-    const int NW = (N + 31) >> 5, tid = threadIdx.x, lane = tid & 63;
-    uint32_t* listed = bits;
-    uint32_t* marked = bits + NW;
-    for (int k = tid; k < 2 * NW; k += 256) bits[k] = 0u;
-    if constexpr (!LDS) __threadfence();
-    __syncthreads();
-    if (tid >= 64) {  // the helper waves: read the path arrays, the graph and the records, then leave
-        const int total = ctr[0] == 0 ? ctr[1] : 0;
-        uint32_t acc = 0u;
-        for (int k = (tid - 64) * 16; k < total; k += 192 * 16) acc ^= (uint32_t)A[k];  // one read per 64 bytes
-        for (int k = (tid - 64) * 64; k < N; k += 192 * 64) acc ^= g[k];
-        for (int k = (tid - 64) * 4; k < N; k += 192 * 4) acc ^= rec[k].x;
-        asm volatile("" ::"v"(acc));  // (keeps the reads)
-        return;
-    }
-    auto get = [&](const uint32_t* b, int n) -> uint32_t {
-        uint32_t w;
-        if constexpr (LDS)
-            w = b[n >> 5];
-        else
-            w = __hip_atomic_load(b + (n >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return (w >> (n & 31)) & 1u;
-    };
-    auto put = [&](uint32_t* b, int n) { atomicOr(b + (n >> 5), 1u << (n & 31)); };
-    // the marks written so far are seen by the wave's next reads (one wave:
-    // its LDS operations complete in order)
-    auto settle = [&]() {
-        if constexpr (!LDS) __threadfence();
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    };
-    // node k (1-based) of a walk of n nodes from place pos of a path of L at
-    // off; past the walk (k > n) the path arrays' first entry, unused
-    auto walk_node = [&](int off, int L, int pos, int k, int n) -> int {
-        int q = pos + k;
-        if (q >= L) q -= L;
-        return A[k <= n ? off + q : 0];
-    };
-    int status = ctr[0], nc = 0, nn = 0;
-    // block k of kBcBlk batches: graph bytes and records into registers
-    // (nodes past the frame read its last node), then flags and records
-    // into LDS (the arrays stay in registers: both are inlined)
-    const int nblk = (N + 64 * kBcBlk - 1) / (64 * kBcBlk);
-    uint32_t vv[kBcBlk], rx[kBcBlk], ry[kBcBlk], rz[kBcBlk], rw[kBcBlk];  // (no uint4 array: it would go to scratch)
-    auto issue = [&](int k) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < kBcBlk; j++) {
-            const int n = (k * kBcBlk + j) * 64 + lane, c = n < N ? n : N - 1;
-            const uint4 t = rec[c];
-            vv[j] = g[c];
-            rx[j] = t.x;
-            ry[j] = t.y;
-            rz[j] = t.z;
-            rw[j] = t.w;
-        }
-    };
-    auto stage = [&](int k) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < kBcBlk; j++) {
-            const int n = (k * kBcBlk + j) * 64 + lane;
-            const uint64_t cm = __ballot(n < N && vv[j] != 90u && vv[j] != 0u);
-            if (lane == 0) s_cand[j] = cm;
-            s_rec[j][lane] = make_uint4(rx[j], ry[j], rz[j], rw[j]);
-        }
-    };
-    if (status == 0) issue(0);
-    for (int k = 0; k < nblk && status == 0; k++) {
-        stage(k);  // (the walks of block k - 1 are done with the LDS copy)
-        if (k + 1 < nblk) issue(k + 1);
-        for (int j = 0; j < kBcBlk && status == 0; j++) {
-            const int base = (k * kBcBlk + j) * 64;
-            if (base >= N) break;
-            const int me = base + lane;
-            const bool cand = (s_cand[j] >> lane) & 1u;
-            uint64_t m = __ballot(cand && !get(listed, me));
-            while (m && status == 0) {
-                // the next walks of the batch: their first chunks, all loads at once
-                int bs[kBcAhead], pv[kBcAhead][kBcU], ro[kBcAhead], rl[kBcAhead], rp[kBcAhead], rn[kBcAhead];
-                bool rc[kBcAhead];
-#pragma unroll
-                for (int a = 0; a < kBcAhead; a++) {
-                    bs[a] = m ? __builtin_ctzll(m) : -1;
-                    m &= m ? m - 1 : 0;
-                }
-#pragma unroll
-                for (int a = 0; a < kBcAhead; a++) {  // their records: path offset, length, place, on a cycle
-                    const uint4 rb = s_rec[j][bs[a] < 0 ? 0 : bs[a]];
-                    ro[a] = (int)rb.x;
-                    rl[a] = (int)rb.y;
-                    rp[a] = (int)rb.z;
-                    rc[a] = rb.w != 0u;
-                    rn[a] = bs[a] < 0 ? 0 : rc[a] ? rl[a] - 1 : rl[a] - 1 - rp[a];  // walk nodes after the start
-                }
-#pragma unroll
-                for (int a = 0; a < kBcAhead; a++)
-#pragma unroll
-                    for (int u = 0; u < kBcU; u++)
-                        pv[a][u] = walk_node(ro[a], rl[a], rp[a], 1 + lane + 64 * u, rn[a]);
-                uint64_t alive = ~0ull;  // candidates not listed by a chain of this batch
-#pragma unroll
-                for (int a = 0; a < kBcAhead; a++) {  // (unrolled: pv[a] stays in registers)
-                    if (status != 0) break;
-                    const int b = bs[a];
-                    if (b < 0) break;
-                    if (!((alive >> b) & 1u)) continue;
-                    const int s = base + b;
-                    const int off = ro[a], L = rl[a], pos = rp[a], n = rn[a];
-                    const bool cyc = rc[a];
-                    int prev = s, nd[kBcU];
-                    bool hit;
-                    {  // the first chunk, loaded above
-                        uint64_t bal[kBcU];
-#pragma unroll
-                        for (int u = 0; u < kBcU; u++) nd[u] = pv[a][u];
-#pragma unroll
-                        for (int u = 0; u < kBcU; u++) {
-                            const int kk = 1 + lane + 64 * u;
-                            bal[u] = 64 * u < n ? __ballot(kk <= n && get(marked, nd[u])) : 0ull;
-                        }
-                        const int f = bc_before_mark(bal);
-                        hit = f != -2;
-                        const int last = hit ? f : (n < kBcChunk ? n : kBcChunk) - 1;
-                        if (last >= 0) prev = bc_node_at(nd, last);
-                    }
-                    for (int c = kBcChunk; !hit && c < n; c += kBcChunk2) {  // the rest of a long walk
-                        int nd2[kBcU2];
-                        uint64_t bal[kBcU2];
-#pragma unroll
-                        for (int u = 0; u < kBcU2; u++) nd2[u] = walk_node(off, L, pos, c + 1 + lane + 64 * u, n);
-#pragma unroll
-                        for (int u = 0; u < kBcU2; u++) {
-                            const int kk = c + 1 + lane + 64 * u;
-                            bal[u] = c + 64 * u < n ? __ballot(kk <= n && get(marked, nd2[u])) : 0ull;
-                        }
-                        const int f = bc_before_mark(bal);
-                        hit = f != -2;
-                        const int last = hit ? f : (n - c < kBcChunk2 ? n - c : kBcChunk2) - 1;
-                        if (last >= 0) prev = bc_node_at(nd2, last);
-                    }
-                    if (hit || !cyc) {  // abandoned (a path ends at an internal node)
-                        if (lane == 0) put(marked, prev);
-                        settle();
-                        continue;
-                    }
-                    if (nc >= max_chains || (int64_t)nn + L > max_nodes) {
-                        status = DPX_ENOMEM;
-                        break;
-                    }
-                    if (n < kBcChunk) {  // the whole walk is in nd
-                        if (lane == 0) {
-                            nodes[nn] = s;
-                            put(listed, s);
-                            put(marked, s);
-                        }
-#pragma unroll
-                        for (int u = 0; u < kBcU; u++) {
-                            if (64 * u >= n) break;  // (uniform)
-                            const int kk = 1 + lane + 64 * u;
-                            if (kk <= n) {
-                                nodes[nn + kk] = nd[u];
-                                put(listed, nd[u]);
-                                put(marked, nd[u]);
-                            }
-                        }
-                    } else {
-                        for (int c = 0; c < L; c += kBcChunk2) {
-                            int v[kBcU2];
-#pragma unroll
-                            for (int u = 0; u < kBcU2; u++) {
-                                const int kk = c + lane + 64 * u;
-                                v[u] = c + 64 * u >= L ? 0 : kk == 0 ? s : walk_node(off, L, pos, kk, n);  // (uniform)
-                            }
-#pragma unroll
-                            for (int u = 0; u < kBcU2; u++) {
-                                const int kk = c + lane + 64 * u;
-                                if (kk < L) {
-                                    nodes[nn + kk] = v[u];
-                                    put(listed, v[u]);
-                                    put(marked, v[u]);
-                                }
-                            }
-                        }
-                    }
-                    if (lane == 0) sizes[nc] = L;
-                    nc++;
-                    nn += L;
-                    settle();
-                    const uint64_t still = __ballot(cand && !get(listed, me));
-                    alive &= still;
-                    m &= still;
-                }
-            }
-        }
-    }
-    if (lane == 0) {
-        counts[0] = nc;
-        counts[1] = nn;
-        counts[2] = status;
-    }
-}
-
 int check_img(const void* p, int W, int H, int stride, int ch, uint32_t flags)
 {
     DPX_CHECK(p != nullptr, DPX_EINVAL, "null image pointer");
@@ -1131,91 +684,6 @@ extern "C" int dpx_stage_components(const uint8_t* d_graph, int W, int H, int32_
     hipLaunchKernelGGL(k_cc_tile, tiles, dim3(256), 0, s, d_graph, W, H, d_labels);
     hipLaunchKernelGGL(k_cc_cross, grid2(W, H), dim3(kB, kB), 0, s, d_graph, W, H, d_labels);
     hipLaunchKernelGGL(k_cc_final, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, d_labels, d_labels, N);
-    DPX_HIP(hipGetLastError());
-    return DPX_OK;
-}
-
-extern "C" int dpx_stage_border_chains(const uint8_t* d_graph, int W, int H, uint8_t* d_scratch, int32_t* d_nodes,
-                                       int max_nodes, int32_t* d_sizes, int max_chains, int32_t* d_counts,
-                                       void* stream)
-{
-    DPX_CHECK(d_graph && d_scratch && d_nodes && d_sizes && d_counts && W > 0 && H > 0, DPX_EINVAL,
-              "bad arguments");
-    DPX_CHECK((int64_t)W * H <= (1 << 28), DPX_EINVAL, "frame too large (%dx%d)", W, H);
-    DPX_CHECK(max_nodes >= 0 && max_chains >= 0, DPX_EINVAL, "negative capacity");
-    const hipStream_t s = as_stream(stream);
-    const uint32_t N = (uint32_t)W * (uint32_t)H, E = 8u * N;
-    // the scan's marks in LDS when they fit a block, else in d_scratch
-    int dev = 0, lds_max = 0;
-    DPX_HIP(hipGetDevice(&dev));
-    DPX_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    const size_t lds = 8 * (size_t)((N + 31) / 32);
-    hipFuncAttributes fa{};
-    DPX_HIP(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(k_bc_scan<true>)));
-    bool use_lds = lds + fa.sharedSizeBytes <= (size_t)lds_max &&
-                   hipFuncSetAttribute(reinterpret_cast<const void*>(k_bc_scan<true>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-    if (!use_lds) {
-        (void)hipGetLastError();
-        DPX_CHECK(reinterpret_cast<uintptr_t>(d_scratch) % 4 == 0, DPX_EINVAL,
-                  "d_scratch must be 4-byte aligned for a frame of %dx%d", W, H);
-    }
-    int rounds = 0;
-    while ((1ull << rounds) < E) rounds++;
-    // working memory, stream-ordered: two link-state arrays, the path
-    // arrays, the per-node walk records and the counters
-    const size_t szS = round256((size_t)E * sizeof(uint4)), szA = round256((size_t)E * 4),
-                 szR = round256((size_t)N * sizeof(uint4));
-    uint8_t* work = nullptr;
-    DPX_HIP(hipMallocAsync(reinterpret_cast<void**>(&work), 2 * szS + szA + szR + 256, s));
-    struct FreeAfter {  // freed in stream order on every return below
-        void* p;
-        hipStream_t s;
-        ~FreeAfter() { (void)hipFreeAsync(p, s); }
-    } free_after{ work, s };
-    uint4* SA = reinterpret_cast<uint4*>(work);
-    uint4* SB = reinterpret_cast<uint4*>(work + szS);
-    int32_t* A = reinterpret_cast<int32_t*>(work + 2 * szS);
-    uint4* rec = reinterpret_cast<uint4*>(work + 2 * szS + szA);
-    int* ctr = reinterpret_cast<int*>(work + 2 * szS + szA + szR);
-    const dim3 grid((E + 255) / 256);
-    hipLaunchKernelGGL(k_bc_clear, dim3(1), dim3(64), 0, s, ctr);
-    hipLaunchKernelGGL(k_bc_init, grid, dim3(256), 0, s, d_graph, W, H, SA, ctr);
-    uint4 *cur = SA, *oth = SB;
-    for (int r = 0; r < rounds;) {  // (three rounds a launch while three are left)
-        const int m = rounds - r >= 3 ? 3 : rounds - r;
-        if (m == 3)
-            hipLaunchKernelGGL((k_bc_jump<true, 7>), grid, dim3(256), 0, s, cur, oth, E);
-        else if (m == 2)
-            hipLaunchKernelGGL((k_bc_jump<true, 3>), grid, dim3(256), 0, s, cur, oth, E);
-        else
-            hipLaunchKernelGGL((k_bc_jump<true, 1>), grid, dim3(256), 0, s, cur, oth, E);
-        r += m;
-        std::swap(cur, oth);
-    }
-    hipLaunchKernelGGL(k_bc_cut, grid, dim3(256), 0, s, d_graph, W, H, cur, oth, E);
-    std::swap(cur, oth);
-    for (int r = 0; r < rounds;) {
-        const int m = rounds - r >= 3 ? 3 : rounds - r;
-        if (m == 3)
-            hipLaunchKernelGGL((k_bc_jump<false, 7>), grid, dim3(256), 0, s, cur, oth, E);
-        else if (m == 2)
-            hipLaunchKernelGGL((k_bc_jump<false, 3>), grid, dim3(256), 0, s, cur, oth, E);
-        else
-            hipLaunchKernelGGL((k_bc_jump<false, 1>), grid, dim3(256), 0, s, cur, oth, E);
-        r += m;
-        std::swap(cur, oth);
-    }
-    hipLaunchKernelGGL(k_bc_heads, dim3((E + kHeadsBlock - 1) / kHeadsBlock), dim3(kHeadsBlock), 0, s, cur, oth, ctr, E);
-    hipLaunchKernelGGL(k_bc_scatter, grid, dim3(256), 0, s, d_graph, cur, oth, A, rec, ctr, E);
-    if (use_lds) {
-        hipLaunchKernelGGL(k_bc_scan<true>, dim3(1), dim3(256), lds, s, d_graph, (int)N, rec, A, nullptr, d_nodes,
-                           d_sizes, max_nodes, max_chains, ctr, d_counts);
-    } else {
-        hipLaunchKernelGGL(k_bc_scan<false>, dim3(1), dim3(256), 0, s, d_graph, (int)N, rec, A,
-                           reinterpret_cast<uint32_t*>(d_scratch), d_nodes, d_sizes, max_nodes, max_chains, ctr,
-                           d_counts);
-    }
     DPX_HIP(hipGetLastError());
     return DPX_OK;
 }
