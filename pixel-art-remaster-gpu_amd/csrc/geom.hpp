@@ -186,7 +186,9 @@ __host__ __device__ inline int cell_hull(uint32_t key, int* hx, int* hy)
 // Subdivision helpers (subdivision_functions.cu).  Inputs in quarter units,
 // outputs in 1/64 units.
 // ---------------------------------------------------------------------------
-__host__ __device__ inline int mod_n(int i, int n) { return (n + (i % n)) % n; }
+// index i of a polygon of n vertices, -1 <= i <= n (a remainder by a variable
+// costs some 35 instructions, and a cell takes dozens)
+__host__ __device__ inline int wrap_n(int i, int n) { return i < 0 ? i + n : i >= n ? i - n : i; }
 
 // The functions below take a polygon as any indexable type (a pointer to
 // int, or an accessor whose operator[] reads packed storage).
@@ -196,7 +198,7 @@ __host__ __device__ inline int mod_n(int i, int n) { return (n + (i % n)) % n; }
 template <class HX, class HY>
 __host__ __device__ inline int linked_edge(const HX& hx, const HY& hy, int n, uint32_t node, int idx)
 {
-    int b = mod_n(idx + 1, n);
+    int b = wrap_n(idx + 1, n);
     int ax = hx[idx], ay = hy[idx], bx = hx[b], by = hy[b];
     int dx = bx - ax, dy = by - ay;
     bool sp = dx != 0 && dy == dx;
@@ -218,9 +220,7 @@ __host__ __device__ inline int linked_edge(const HX& hx, const HY& hy, int n, ui
 template <class HX, class HY>
 __host__ __device__ inline void q_point(const HX& hx, const HY& hy, int n, int i, int* qx, int* qy)
 {
-    int p = i % n;
-    if (p < 0) p += n;
-    int q = (i + 1) % n;
+    const int p = wrap_n(i, n), q = wrap_n(i + 1, n);
     int x0 = hx[p], y0 = hy[p], x1 = hx[q], y1 = hy[q];
     int dx = x1 - x0, dy = y1 - y0;
     if (dx * dx + dy * dy <= 16) { *qx = 4 * (3 * x0 + x1); *qy = 4 * (3 * y0 + y1); }
@@ -230,9 +230,7 @@ __host__ __device__ inline void q_point(const HX& hx, const HY& hy, int n, int i
 template <class HX, class HY>
 __host__ __device__ inline void r_point(const HX& hx, const HY& hy, int n, int i, int* rx, int* ry)
 {
-    int p = i % n;
-    if (p < 0) p += n;
-    int q = (i + 1) % n;
+    const int p = wrap_n(i, n), q = wrap_n(i + 1, n);
     int x0 = hx[p], y0 = hy[p], x1 = hx[q], y1 = hy[q];
     int dx = x1 - x0, dy = y1 - y0;
     if (dx * dx + dy * dy <= 16) { *rx = 4 * (x0 + 3 * x1); *ry = 4 * (y0 + 3 * y1); }
@@ -267,7 +265,7 @@ __host__ __device__ inline void subdivide_cell_emit(const HX& hx, const HY& hy, 
     for (int e = 0; e < n; e++) links |= (uint64_t)(linked_edge(hx, hy, n, node, e) & 15) << (4 * e);
     auto link = [&](int e) { return (int)((links >> (4 * e)) & 15u); };
     for (int k = 0; k < n; k++) {
-        int prev = mod_n(k - 1, n);
+        int prev = wrap_n(k - 1, n);
         const int lk = link(k), lp = link(prev);
         bool sk = lk != 15, sp = lp != 15;
         if (!sk && !sp) {
@@ -390,6 +388,129 @@ __host__ __device__ inline int ear_clip(const int* x, const int* y, int n, uint8
         }
     }
     return ntri;
+}
+
+// ear_clip on at most MAXN <= 16 vertices in counter-clockwise order, for
+// one lane of a wave: vertex k at P[stride * k], x | y << 16.  ear(A, B, C)
+// receives each triangle as it is cut; returns the number of vertices left (2
+// when the polygon is cut wholly).  The vertices stay where they are: a mask
+// holds those not cut off yet, and the three at hand move along it (after an
+// ear the walk goes on at its third corner, else at its second, which is
+// where ear_clip's index stands in its shortened list).  The test of the
+// other vertices is unrolled over registers, two multiply-adds an edge: a
+// loop over a list in LDS costs a read, two unpackings and three comparisons
+// of indices a vertex more.  Products are taken modulo 2^32, as ear_clip's
+// are; coordinates are 16 bits.
+__host__ __device__ inline int mad24(int a, int b, int c);
+
+// Shape of a polygon (vertex k at P[stride * k], x | y << 16): twice its
+// signed area, and whether it is convex once it stands counter-clockwise: no
+// corner turns right or back and the edges' directions go round once
+// (`convex`: straight corners allowed, `strict`: none).
+struct PolyShape {
+    int area2;
+    bool convex, strict;
+};
+__host__ __device__ inline PolyShape poly_shape(const uint32_t* P, int stride, int n)
+{
+    PolyShape s;
+    int a2 = 0, left = 0, right = 0, back = 0, straight = 0, rounds = 0;
+    const uint32_t L = P[stride * (n - 1)], K = P[stride * (n - 2)];
+    int px = (int)(int16_t)(L & 0xFFFFu), py = (int)L >> 16;
+    int ex = px - (int)(int16_t)(K & 0xFFFFu), ey = py - ((int)K >> 16);
+    int half = ey > 0 || (ey == 0 && ex > 0);
+    for (int k = 0; k < n; k++) {  // edge from vertex k - 1 to k, and the corner before it
+        const uint32_t w = P[stride * k];
+        const int x = (int)(int16_t)(w & 0xFFFFu), y = (int)w >> 16, dx = x - px, dy = y - py;
+        a2 += mad24(px, y, mad24(-x, py, 0));
+        const int c = mad24(ex, dy, mad24(-ey, dx, 0)), d = mad24(ex, dx, mad24(ey, dy, 0));
+        left |= c > 0;
+        right |= c < 0;
+        straight |= c == 0;
+        back |= c == 0 && d <= 0;
+        const int h = dy > 0 || (dy == 0 && dx > 0);
+        rounds += h & ~half;
+        half = h;
+        px = x;
+        py = y;
+        ex = dx;
+        ey = dy;
+    }
+    s.area2 = a2;
+    // (a clockwise polygon's directions go round the other way, once as well)
+    s.convex = !(left && right) && !back && rounds == 1;
+    s.strict = s.convex && !straight;
+    return s;
+}
+
+__host__ __device__ inline int mad24(int a, int b, int c)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __mul24(a, b) + c;
+#else
+    return (int)((uint32_t)a * (uint32_t)b + (uint32_t)c);
+#endif
+}
+
+// With `test` false (the caller knows the polygon to be strictly convex) no
+// vertex can lie in another three's triangle, and none is looked at.
+template <int MAXN, class Ear>
+__host__ __device__ inline int ear_clip_ring(const uint32_t* P, int stride, int n, bool test, Ear ear)
+{
+    static_assert(MAXN <= 16, "coordinates are 16 bits");
+    int x[MAXN], y[MAXN];
+#pragma unroll
+    for (int k = 0; k < MAXN; k++) {
+        const uint32_t w = k < n ? P[stride * k] : 0u;
+        x[k] = (int)(int16_t)(w & 0xFFFFu);
+        y[k] = (int)w >> 16;
+    }
+    uint32_t alive = (1u << n) - 1u;
+    auto next = [&](int k) {
+        const uint32_t m = alive & (0xFFFFFFFEu << k);
+        return __builtin_ctz(m ? m : alive);
+    };
+    int nv = n, count = 2 * nv, u = n - 1, v = 0, w = 1;
+    uint32_t A = P[stride * u], B = P[stride * v], C = P[stride * w];
+    while (nv > 2) {
+        if (0 >= (count--)) break;  // the reference gives up; the triangles cut so far stand
+        const int ax = (int)(int16_t)(A & 0xFFFFu), ay = (int)A >> 16;
+        const int bx = (int)(int16_t)(B & 0xFFFFu), by = (int)B >> 16;
+        const int cx = (int)(int16_t)(C & 0xFFFFu), cy = (int)C >> 16;
+        // edges B -> C, A -> B, C -> A: cross = dx py - dy px + k
+        const int dx1 = cx - bx, dy1 = cy - by, dx2 = bx - ax, dy2 = by - ay, dx3 = ax - cx, dy3 = ay - cy;
+        bool cut = mad24(dx2, -dy3, mad24(dy2, dx3, 0)) > 0;
+        if (cut && test) {
+            const int k1 = mad24(dy1, bx, mad24(-dx1, by, 0)), k2 = mad24(dy2, ax, mad24(-dx2, ay, 0)),
+                      k3 = mad24(dy3, cx, mad24(-dx3, cy, 0));
+            uint32_t in = 0;  // vertices inside the triangle or on its edges
+#pragma unroll
+            for (int k = 0; k < MAXN; k++) {
+                const int c1 = mad24(dx1, y[k], mad24(-dy1, x[k], k1)), c2 = mad24(dx2, y[k], mad24(-dy2, x[k], k2)),
+                          c3 = mad24(dx3, y[k], mad24(-dy3, x[k], k3));
+                in |= (c1 | c2 | c3) >= 0 ? 1u << k : 0u;
+            }
+            cut = (in & alive & ~(1u << u | 1u << v | 1u << w)) == 0;
+        }
+        if (cut) {
+            ear(A, B, C);
+            alive &= ~(1u << v);
+            nv--;
+            count = 2 * nv;
+            u = w;
+            A = C;
+            v = next(u);
+            B = P[stride * v];
+        } else {
+            u = v;
+            A = B;
+            v = w;
+            B = C;
+        }
+        w = next(v);
+        C = P[stride * w];
+    }
+    return nv;
 }
 
 // ---------------------------------------------------------------------------

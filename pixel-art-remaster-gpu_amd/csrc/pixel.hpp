@@ -226,4 +226,48 @@ __host__ __device__ inline bool tjunction(const TjView& v, int i, int j, int x4,
     return false;
 }
 
+// tjunction for the four corners of cell (i, j) at once: bits 0..3 for (0,
+// 0), (4, 0), (4, 4), (0, 4), bit 4: every vertex is kept.  The eight colours
+// are read side by side (one after another, and per vertex, each is a round
+// trip to memory), and the virtual buffer's index arithmetic is done once.
+__host__ __device__ inline uint32_t tj_corners(const TjView& v, int i, int j)
+{
+    const long long ws = v.ws, index = (long long)j * ws + 3LL * i;
+    if ((index - ws - 1) < 0 || (index + v.im.W + 1) > (v.im.H * ws - 1)) return 0x1Fu;
+    const int cc = colour_channels(v.im);
+    uint32_t col[8], ok = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        // c0 .. c7: up-left, up, up-right, left, right, down-left, down, down-right
+        const int dx = (k == 0 || k == 3 || k == 5) ? -1 : ((k == 1 || k == 6) ? 0 : 1);
+        const int dy = k <= 2 ? 1 : (k <= 4 ? 0 : -1);
+        col[k] = 0;
+        const uint8_t* q;
+        if (v.raw) {
+            const long long a = index + dy * ws + 3 * dx;
+            if (a < 0 || a + 2 >= v.size) continue;
+            q = v.im.p + a;
+        } else {
+            int x = i + dx, y = j + dy;  // pixel j W + i of the packed view: rows run on into each other
+            if (x < 0) { x += v.im.W; y--; }
+            if (x >= v.im.W) { x -= v.im.W; y++; }
+            if (y < 0 || y >= v.im.H) continue;
+            q = px_ptr(v.im, x, y);
+        }
+        ok |= 1u << k;
+        col[k] = (uint32_t)q[0] | (uint32_t)q[1] << 8 | (uint32_t)q[2] << 16 | (cc == 4 ? (uint32_t)q[3] << 24 : 0u);
+    }
+    auto differ = [&](int a, int b) { return !((ok >> a) & (ok >> b) & 1u) || col[a] != col[b]; };
+    return (differ(3, 5) || differ(5, 6) ? 1u : 0u) | (differ(4, 7) || differ(7, 6) ? 2u : 0u) |
+           (differ(1, 2) || differ(2, 4) ? 4u : 0u) | (differ(0, 1) || differ(1, 3) ? 8u : 0u);
+}
+
+// tjunction's answer for hull vertex (x4, y4) from the cell's tj_corners
+__host__ __device__ inline bool tj_kept(uint32_t corners, int x4, int y4)
+{
+    if (corners & 16u) return true;
+    if ((x4 != 0 && x4 != 4) || (y4 != 0 && y4 != 4)) return false;
+    return (corners >> (y4 == 0 ? (x4 == 0 ? 0 : 1) : (x4 == 4 ? 2 : 3))) & 1u;
+}
+
 }  // namespace dpx

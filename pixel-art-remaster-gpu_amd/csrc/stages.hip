@@ -2,11 +2,15 @@
 // sequence, intermediates in HBM in the reference's formats), the stage entry
 // points of the C ABI, the plain per-frame path and the launch_kernel drop-in.
 //
-// Launch shape: 16x16 threads, one thread per pixel (or per output pixel for
-// the raster).  These kernels favour a direct mapping of the reference's data
-// formats over speed; the batched path in fused.hip is the fast one.
+// The graph kernels take 16x16 threads, one per pixel; the kernels that read
+// and write whole cells (45 slots, 360 bytes) take runs or tiles of cells,
+// staged in LDS and written as contiguous ranges; the raster and the window
+// take tiles of output pixels.  The formats are the reference's; the batched
+// path in fused.hip, which has none of them in HBM, is the fast one.
 #include <stdlib.h>
 #include <string.h>
+
+#include <algorithm>
 
 #include "common.hpp"
 #include "geom.hpp"
@@ -81,27 +85,53 @@ __global__ void k_heuristic(uint8_t* __restrict__ graph, const uint8_t* __restri
     graph[idx] = (uint8_t)(c & ~heuristic_clear_mask(get, i, j, c, nb));
 }
 
-// cells_Kernel (kernel.cu:192-213): hull points in 45-slot cells.  Slots past
-// the closing point are written as (0,0).
-__global__ void k_cells(const uint8_t* __restrict__ graph, int W, int H, dpx_point* __restrict__ diagram,
-                        int32_t* __restrict__ edge_count)
+// The hulls of the 4096 cell keys (gen_hull_table.cpp): 32 KB, one word each.
+__device__ const uint64_t kHullTable[4096] = {
+#include "hull_table.inc"
+};
+
+// The kernels below write whole cells of 45 slots (360 bytes).  A thread
+// that writes its own cell's slots puts every lane of a store on a line of
+// its own, so the cells' values go to LDS first and a block then writes its
+// kRun cells as one contiguous range, adjacent lanes adjacent slots.
+constexpr int kRun = 64;
+
+__device__ inline dpx_point hull_point(uint64_t h, int t)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int j = blockIdx.y * blockDim.y + threadIdx.y;
-    if (i >= W || j >= H) return;
-    size_t N = (size_t)W * H, idx = (size_t)j * W + i;
-    uint32_t left = idx > 0 ? graph[idx - 1] : 0u;
-    uint32_t right = idx + 1 < N ? graph[idx + 1] : 0u;
-    int hx[2 * kMaxPts], hy[2 * kMaxPts];
-    int n = cell_hull(cell_key(graph[idx], left, right), hx, hy);
-    dpx_point* c = &diagram[idx * kCellSize];
-    for (int t = 0; t < kCellSize; t++) {
-        dpx_point p;
-        p.x = t <= n ? 0.25f * (float)hx[t] : 0.0f;
-        p.y = t <= n ? 0.25f * (float)hy[t] : 0.0f;
-        c[t] = p;
+    dpx_point p;
+    p.x = 0.25f * (float)((int)((h >> (6 * t)) & 7u) - 1);
+    p.y = 0.25f * (float)((int)((h >> (6 * t + 3)) & 7u) - 1);
+    return p;
+}
+
+// cells_Kernel (kernel.cu:192-213): hull points in 45-slot cells.  Slots past
+// the closing point are written as (0,0).  Bound by its writes (20.6 MB for
+// 256x224); 8 us there; the
+// hulls computed in per-thread arrays took 59.
+__global__ __launch_bounds__(256) void k_cells(const uint8_t* __restrict__ graph, size_t N,
+                                               dpx_point* __restrict__ diagram, int32_t* __restrict__ edge_count)
+{
+    __shared__ uint64_t s_h[kRun];
+    const size_t c0 = (size_t)blockIdx.x * kRun;
+    const int t = threadIdx.x, cells = (int)(N - c0 < kRun ? N - c0 : kRun);
+    if (t < cells) {
+        const size_t idx = c0 + t;
+        const uint32_t left = idx > 0 ? graph[idx - 1] : 0u;
+        const uint32_t right = idx + 1 < N ? graph[idx + 1] : 0u;
+        const uint64_t h = kHullTable[cell_key(graph[idx], left, right)];
+        s_h[t] = h;
+        edge_count[idx] = (int)(h >> 48);
     }
-    edge_count[idx] = n;
+    __syncthreads();
+    dpx_point* d = diagram + c0 * kCellSize;
+    for (int k = t; k < cells * kCellSize; k += 256) {
+        const int c = k / kCellSize, q = k - c * kCellSize;
+        const uint64_t h = s_h[c];
+        const int n = (int)(h >> 48);
+        dpx_point p = { 0.0f, 0.0f };
+        if (q <= n) p = hull_point(h, q == n ? 0 : q);
+        d[k] = p;
+    }
 }
 
 __device__ inline int load_quarter(const dpx_point* c, int n, int* x, int* y)
@@ -113,29 +143,23 @@ __device__ inline int load_quarter(const dpx_point* c, int n, int* x, int* y)
     return n;
 }
 
-// subdivision_Kernel (kernel.cu:216-261) on the snapshots daux/eaux.
-__global__ void k_subdivide(ImgView im, const uint8_t* __restrict__ graph, dpx_point* __restrict__ diagram,
-                            const dpx_point* __restrict__ daux, int32_t* __restrict__ edge_count,
-                            const int32_t* __restrict__ eaux)
+// One cell of subdivision_Kernel in per-thread arrays: any vertex counts and
+// coordinates that a caller's diagram may hold.
+__device__ __noinline__ int subdivide_any(ImgView im, uint32_t node, int i, int j, int n,
+                                          dpx_point* __restrict__ diagram, const dpx_point* __restrict__ daux,
+                                          const int32_t* __restrict__ eaux)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int j = blockIdx.y * blockDim.y + threadIdx.y;
-    int W = im.W;
-    if (i >= W || j >= im.H) return;
-    int idx = j * W + i;
-    uint32_t node = graph[idx];
-    if (node == 90) return;  // internal node (kernel.cu:231)
-    int n = eaux[idx];
-    // subdivide_cell emits up to 2n points into kMaxPoly slots; real hulls
-    // have at most 8 vertices, larger caller-supplied counts leave the cell
-    if (n < 3 || n > kMaxPoly / 2) return;
+    const int W = im.W, idx = j * W + i;
     int hx[2 * kMaxPts], hy[2 * kMaxPts];
     load_quarter(&daux[(size_t)idx * kCellSize], n, hx, hy);
     TjView tv = tj_view(im);
     auto nbr = [&](int e, int* lx, int* ly) -> int {
         int q = idx + edy(e) * W + edx(e);
+        lx[0] = ly[0] = 0;
+        if (q < 0 || q >= W * im.H) return 1;  // (a link that leaves the frame)
         int ln = eaux[q];
         if (ln > 2 * kMaxPts - 1) ln = 2 * kMaxPts - 1;
+        if (ln < 1) return 1;
         return load_quarter(&daux[(size_t)q * kCellSize], ln, lx, ly);
     };
     auto tj = [&](int x4, int y4) -> bool { return tjunction(tv, i, j, x4, y4); };
@@ -148,20 +172,128 @@ __global__ void k_subdivide(ImgView im, const uint8_t* __restrict__ graph, dpx_p
         p.y = (float)oy[t] * (1.0f / 64.0f);
         c[t] = p;
     }
-    edge_count[idx] = m;
+    return m;
 }
 
-// triangulate_Kernel (kernel.cu:264-282): ear clipping, then every slot gets
-// the pixel offset; unwritten slots stay at the pixel origin.
-__global__ void k_triangulate(dpx_point* __restrict__ diagram, const int32_t* __restrict__ edge_count, int W,
-                              int H)
+// x | y << 16; false when one lies outside -limit .. limit (at most 32767)
+__device__ inline bool pack_point(int x, int y, int limit, uint32_t* w)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int j = blockIdx.y * blockDim.y + threadIdx.y;
-    if (i >= W || j >= H) return;
-    size_t idx = (size_t)j * W + i;
-    dpx_point* c = &diagram[idx * kCellSize];
-    int n = edge_count[idx];
+    *w = ((uint32_t)x & 0xFFFFu) | ((uint32_t)y << 16);
+    return x >= -limit && x <= limit && y >= -limit && y <= limit;
+}
+__device__ inline int point_x(uint32_t w) { return (int)(int16_t)(w & 0xFFFFu); }
+__device__ inline int point_y(uint32_t w) { return (int)w >> 16; }
+
+// subdivision_Kernel (kernel.cu:216-261) on the snapshots daux/eaux, a tile
+// of 32x8 cells per block: the hulls of the tile and the cells around it in
+// LDS (up to 8 vertices, as the cells stage makes them), the new points from
+// LDS to the diagram.  A cell with other hulls around it, or a link that
+// leaves the frame, takes subdivide_any.  (All cells through per-thread
+// arrays: 58 us for 256x224; so 28.)
+constexpr int kSubX = 32, kSubY = 8, kSubPitch = 9;  // (9 words a hull: no bank is shared by adjacent cells)
+__global__ __launch_bounds__(256) void k_subdivide(ImgView im, const uint8_t* __restrict__ graph,
+                                                   dpx_point* __restrict__ diagram,
+                                                   const dpx_point* __restrict__ daux,
+                                                   int32_t* __restrict__ edge_count,
+                                                   const int32_t* __restrict__ eaux)
+{
+    constexpr int CX = kSubX + 2, CY = kSubY + 2;
+    constexpr uint8_t ANY = 255;
+    __shared__ uint32_t s_hull[CX * CY * kSubPitch];
+    __shared__ uint8_t s_n[CX * CY];
+    __shared__ uint32_t s_new[16 * 256];  // point k of cell t at [k * 256 + t]
+    __shared__ uint8_t s_m[256];
+    const int t = threadIdx.x, W = im.W, H = im.H;
+    const int x0 = blockIdx.x * kSubX, y0 = blockIdx.y * kSubY;
+    for (int k = t; k < CX * CY; k += 256) {
+        const int x = x0 - 1 + k % CX, y = y0 - 1 + k / CX;
+        int n = 1;  // (outside the frame: never asked for, see below)
+        if (in_frame(x, y, W, H)) n = eaux[y * W + x];
+        s_n[k] = n < 1 || n > 8 ? ANY : (uint8_t)n;
+    }
+    __syncthreads();
+    // (all of a thread's loads before the first is waited for)
+    constexpr int PER = (CX * CY * 8 + 255) / 256;
+    dpx_point p[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const int c = (t >> 3) + 32 * k, q = t & 7, x = x0 - 1 + c % CX, y = y0 - 1 + c / CX;
+        p[k] = dpx_point{ 0.0f, 0.0f };
+        if (c < CX * CY && in_frame(x, y, W, H) && s_n[c] != ANY && q < s_n[c])
+            p[k] = daux[(size_t)(y * W + x) * kCellSize + q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const int c = (t >> 3) + 32 * k, q = t & 7;
+        if (c < CX * CY) {
+            uint32_t w;
+            // (the new points are 16 times as large and have to fit as well)
+            if (!pack_point((int)(p[k].x * 4.0f), (int)(p[k].y * 4.0f), 1024, &w)) s_n[c] = ANY;
+            s_hull[c * kSubPitch + q] = w;
+        }
+    }
+    __syncthreads();
+    const int cx = t % kSubX, cy = t / kSubX, i = x0 + cx, j = y0 + cy;
+    const int own = (cy + 1) * CX + cx + 1;
+    s_m[t] = 0;
+    if (i < W && j < H) {
+        const int idx = j * W + i;
+        const uint32_t node = graph[idx];
+        const int n = eaux[idx];
+        // subdivide_cell emits up to 2n points into kMaxPoly slots; real hulls
+        // have at most 8 vertices, larger caller-supplied counts leave the
+        // cell, and so do internal nodes (kernel.cu:231)
+        if (node != 90 && n >= 3 && n <= kMaxPoly / 2) {
+            bool any = false;
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (bit(node, e))
+                    any = any || !in_frame(i + edx(e), j + edy(e), W, H) || s_n[own + edy(e) * CX + edx(e)] == ANY;
+            if (any || s_n[own] == ANY) {
+                edge_count[idx] = subdivide_any(im, node, i, j, n, diagram, daux, eaux);
+            } else {
+                struct HullX {
+                    const uint32_t* p;
+                    __device__ int operator[](int k) const { return point_x(p[k]); }
+                };
+                struct HullY {
+                    const uint32_t* p;
+                    __device__ int operator[](int k) const { return point_y(p[k]); }
+                };
+                const uint32_t corners = tj_corners(tj_view(im), i, j);
+                const uint32_t* h = s_hull + own * kSubPitch;
+                auto nbr = [&](int e, auto f) {
+                    const int c = own + edy(e) * CX + edx(e);
+                    const uint32_t* q = s_hull + c * kSubPitch;
+                    return f(HullX{ q }, HullY{ q }, (int)s_n[c]);
+                };
+                auto tj = [&](int x4, int y4) -> bool { return tj_kept(corners, x4, y4); };
+                int m = 0;
+                subdivide_cell_emit(HullX{ h }, HullY{ h }, n, node, nbr, tj, [&](int px, int py) {
+                    s_new[256 * m + t] = ((uint32_t)px & 0xFFFFu) | ((uint32_t)py << 16);
+                    m++;
+                });
+                edge_count[idx] = m;
+                s_m[t] = (uint8_t)m;
+            }
+        }
+    }
+    __syncthreads();
+    for (int k = t; k < 256 * 16; k += 256) {
+        const int c = k >> 4, q = k & 15;
+        if (q >= s_m[c]) continue;
+        const uint32_t w = s_new[256 * q + c];
+        dpx_point p;
+        p.x = (float)point_x(w) * (1.0f / 64.0f);
+        p.y = (float)point_y(w) * (1.0f / 64.0f);
+        diagram[(size_t)((y0 + c / kSubX) * W + x0 + c % kSubX) * kCellSize + q] = p;
+    }
+}
+
+// One cell of triangulate_Kernel in per-thread arrays: any vertex counts and coordinates.
+__device__ __noinline__ void triangulate_any(dpx_point* __restrict__ c, int n, float fi, float fj)
+{
     int x[kMaxPoly], y[kMaxPoly];
     uint8_t tri[3 * kMaxPoly];
     int nt = 0, ok = 0;
@@ -172,7 +304,6 @@ __global__ void k_triangulate(dpx_point* __restrict__ diagram, const int32_t* __
         }
         nt = ear_clip(x, y, n, tri, &ok);
     }
-    float fi = (float)i, fj = (float)j;
     for (int t = 0; t < kCellSize; t++) {
         dpx_point p;
         if (t < 3 * nt) {
@@ -186,85 +317,186 @@ __global__ void k_triangulate(dpx_point* __restrict__ diagram, const int32_t* __
     }
 }
 
-// color_kernel (kernel.cu:67-104) + position_kernel (kernel.cu:109-137)
-__global__ void k_export_vbo(ImgView im, const dpx_point* __restrict__ diagram, const int32_t* __restrict__ edge_count,
-                             dpx_point* __restrict__ pos, dpx_uchar4* __restrict__ color)
+// triangulate_Kernel (kernel.cu:264-282): ear clipping, then every slot gets
+// the pixel offset; unwritten slots stay at the pixel origin.  A block takes
+// kTriRun cells, a lane a cell; the polygons (up to 16 vertices, twice a
+// hull's) lie in LDS.  Cells go to the lanes by the work they are, so that a
+// wave's lanes end together: those that need the inside tests by their
+// vertices, then the strictly convex ones, whose waves skip the tests.
+// Other cells take triangulate_any.  Bound by the instructions of the tests.
+// (28 us for 256x224.  All cells through per-thread arrays: 109, every vertex
+// read a round trip to memory; vertices shifted in LDS: 56.)
+constexpr int kTriRun = 256, kTriBlock = 1024;  // (all threads read and write, the first kTriRun clip)
+struct alignas(16) TriSlots {
+    float x, y;  // the pixel
+    int n;       // slots of triangles; -1: the cell takes triangulate_any
+    int pad;
+};
+__global__ __launch_bounds__(kTriBlock) void k_triangulate(dpx_point* __restrict__ diagram,
+                                                         const int32_t* __restrict__ edge_count, int W, size_t N)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int j = blockIdx.y * blockDim.y + threadIdx.y;
-    if (i >= im.W || j >= im.H) return;
-    size_t idx = (size_t)j * im.W + i;
-    uint32_t rgba = cell_rgba(load_px(im, i, j), colour_channels(im));
-    dpx_uchar4 c4;
-    c4.x = (uint8_t)(rgba & 0xFF);
-    c4.y = (uint8_t)((rgba >> 8) & 0xFF);
-    c4.z = (uint8_t)((rgba >> 16) & 0xFF);
-    c4.w = (uint8_t)(rgba >> 24);
-    int valid = (edge_count[idx] - 2) * 3;
-    for (int t = 0; t < kCellSize; t++) {
-        size_t s = idx * kCellSize + t;
-        if (color) color[s] = c4;
+    constexpr int MAXN = 16, MAXV = 3 * (MAXN - 2);
+    __shared__ uint32_t s_poly[MAXN * kTriRun];  // vertex k of cell t at [k * kTriRun + t]
+    __shared__ uint32_t s_tri[MAXV * kTriRun];   // triangle corners likewise
+    __shared__ uint8_t s_n[kTriRun], s_any[kTriRun];
+    __shared__ uint16_t s_list[kTriRun];  // cell (| kStrict) of each lane
+    __shared__ int s_bin[64];
+    __shared__ TriSlots s_slots[kTriRun];
+    constexpr uint16_t kStrict = 0x8000;
+    const size_t c0 = (size_t)blockIdx.x * kTriRun;
+    const int t = threadIdx.x, cells = (int)(N - c0 < kTriRun ? N - c0 : kTriRun);
+    dpx_point* d = diagram + c0 * kCellSize;
+    int n_own = 0;
+    if (t < kTriRun) {
+        if (t < cells) n_own = edge_count[c0 + t];
+        s_n[t] = (uint8_t)(n_own >= 3 && n_own <= MAXN ? n_own : 0);
+        s_any[t] = n_own > MAXN;
+    }
+    if (t < 64) s_bin[t] = 0;
+    __syncthreads();
+    {
+        // (all of a thread's loads before the first is waited for: a loop
+        // that stores each waits a memory latency per vertex)
+        constexpr int PER = kTriRun * MAXN / kTriBlock;
+        dpx_point p[PER];
+        const int q = t % MAXN;
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int c = t / MAXN + k * (kTriBlock / MAXN);
+            p[k] = dpx_point{ 0.0f, 0.0f };
+            if (q < s_n[c]) p[k] = d[c * kCellSize + q];
+        }
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int c = t / MAXN + k * (kTriBlock / MAXN);
+            uint32_t w;
+            if (!pack_point((int)(p[k].x * 64.0f), (int)(p[k].y * 64.0f), 32767, &w)) s_any[c] = 1;
+            s_poly[q * kTriRun + c] = w;
+        }
+    }
+    __syncthreads();
+    int bin = 2 * MAXN + 1, rank = 0;  // (nothing to cut)
+    bool strict = false;
+    if (t < kTriRun) {
+        if (s_n[t] && !s_any[t]) {
+            uint32_t* P = s_poly + t;
+            const int n = s_n[t];
+            const PolyShape shape = poly_shape(P, kTriRun, n);
+            strict = shape.strict;
+            if (shape.area2 <= 0)
+                for (int lo = 0, hi = n - 1; lo < hi; lo++, hi--) {
+                    const uint32_t tmp = P[kTriRun * lo];
+                    P[kTriRun * lo] = P[kTriRun * hi];
+                    P[kTriRun * hi] = tmp;
+                }
+            bin = (strict ? MAXN : 0) + MAXN - n;
+        }
+        rank = atomicAdd(&s_bin[bin], 1);
+    }
+    __syncthreads();
+    if (t < 64) {
+        const int own = s_bin[t];
+        int at = own;
+#pragma unroll
+        for (int e = 1; e < 64; e <<= 1) {
+            const int v = __shfl_up(at, e);
+            if (t >= e) at += v;
+        }
+        s_bin[t] = at - own;
+    }
+    __syncthreads();
+    if (t < kTriRun) s_list[s_bin[bin] + rank] = (uint16_t)t | (strict ? kStrict : (uint16_t)0);
+    __syncthreads();
+    if (t < kTriRun) {
+        const int c = s_list[t] & 0xFF;
+        const bool test = !(s_list[t] & kStrict);
+        const int n = s_any[c] ? 0 : s_n[c];
+        uint32_t* T = s_tri + c;
+        int written = 0;
+        if (n)
+            ear_clip_ring<MAXN>(s_poly + c, kTriRun, n, test, [&](uint32_t A, uint32_t B, uint32_t C) {
+                T[kTriRun * written] = A;
+                T[kTriRun * (written + 1)] = B;
+                T[kTriRun * (written + 2)] = C;
+                written += 3;
+            });
+        const size_t idx = c0 + c, j = idx / (size_t)W;
+        s_slots[c] = TriSlots{ (float)(int)(idx - j * (size_t)W), (float)(int)j, s_any[c] ? -1 : written, 0 };
+    }
+    __syncthreads();
+    for (int k = t; k < cells * kCellSize; k += kTriBlock) {
+        const int c = k / kCellSize, q = k - c * kCellSize;
+        const TriSlots sl = s_slots[c];
+        if (sl.n < 0) continue;
+        dpx_point p = { sl.x, sl.y };
+        if (q < sl.n) {
+            const uint32_t w = s_tri[q * kTriRun + c];
+            p.x = (float)point_x(w) * (1.0f / 64.0f) + sl.x;
+            p.y = (float)point_y(w) * (1.0f / 64.0f) + sl.y;
+        }
+        d[k] = p;
+    }
+    if (t < cells && s_any[t]) triangulate_any(d + t * kCellSize, n_own, s_slots[t].x, s_slots[t].y);
+}
+
+// color_kernel (kernel.cu:67-104) + position_kernel (kernel.cu:109-137), a
+// run of cells per block, adjacent lanes adjacent slots (256x224: 9 us; a thread per
+// cell: 55)
+__global__ __launch_bounds__(256) void k_export_vbo(ImgView im, const dpx_point* __restrict__ diagram,
+                                                    const int32_t* __restrict__ edge_count,
+                                                    dpx_point* __restrict__ pos, dpx_uchar4* __restrict__ color)
+{
+    __shared__ uint32_t s_rgba[kRun];
+    __shared__ int s_valid[kRun];
+    const size_t N = (size_t)im.W * im.H, c0 = (size_t)blockIdx.x * kRun;
+    const int t = threadIdx.x, cells = (int)(N - c0 < kRun ? N - c0 : kRun);
+    if (t < cells) {
+        const size_t idx = c0 + t;
+        s_rgba[t] = cell_rgba(load_px(im, (int)(idx % (size_t)im.W), (int)(idx / (size_t)im.W)), colour_channels(im));
+        s_valid[t] = (edge_count[idx] - 2) * 3;
+    }
+    __syncthreads();
+    for (int k = t; k < cells * kCellSize; k += 256) {
+        const int c = k / kCellSize, q = k - c * kCellSize;
+        const size_t s = c0 * kCellSize + k;
+        if (color) {
+            const uint32_t rgba = s_rgba[c];
+            dpx_uchar4 c4;
+            c4.x = (uint8_t)(rgba & 0xFF);
+            c4.y = (uint8_t)((rgba >> 8) & 0xFF);
+            c4.z = (uint8_t)((rgba >> 16) & 0xFF);
+            c4.w = (uint8_t)(rgba >> 24);
+            color[s] = c4;
+        }
         if (pos) {
-            dpx_point p;
-            if (t < valid) p = diagram[s];
-            else { p.x = -100.0f; p.y = -100.0f; }
+            dpx_point p = { -100.0f, -100.0f };
+            if (q < s_valid[c]) p = diagram[s];
             pos[s] = p;
         }
     }
 }
 
-// glDrawArrays(GL_TRIANGLES) in VBO order (simpleVBO.cpp:281) as a gather:
-// each output pixel takes the colour of the highest-index cell (the last one
-// drawn) with a triangle covering its centre.  Cells reach at most 0.34 past
-// their unit square, so the 3x3 cells around the pixel are the candidates.
-__global__ void k_raster_tri(ImgView im, const dpx_point* __restrict__ diagram, const int32_t* __restrict__ edge_count,
-                             int scale, uint8_t* __restrict__ out, int out_stride)
-{
-    int X = blockIdx.x * blockDim.x + threadIdx.x;
-    int Y = blockIdx.y * blockDim.y + threadIdx.y;
-    int OW = im.W * scale, OH = im.H * scale;
-    if (X >= OW || Y >= OH) return;
-    int cx = X / scale, cy = Y / scale;
-    uint32_t color = 0xFF000000u;  // clear colour (0,0,0,1), main.cpp:260
-    bool done = false;
-    for (int dy = 1; dy >= -1 && !done; dy--)
-        for (int dx = 1; dx >= -1 && !done; dx--) {
-            int ci = cx + dx, cj = cy + dy;
-            if (!in_frame(ci, cj, im.W, im.H)) continue;
-            size_t k = (size_t)cj * im.W + ci;
-            int nt = edge_count[k] - 2;
-            if (nt > kCellSize / 3) nt = kCellSize / 3;
-            int sx = (2 * X + 1) * 64 - ci * 128 * scale, sy = (2 * Y + 1) * 64 - cj * 128 * scale;
-            const dpx_point* c = &diagram[k * kCellSize];
-            float fi = (float)ci, fj = (float)cj;
-            for (int t = 0; t < nt; t++) {
-                int v[6];
-#pragma unroll
-                for (int q = 0; q < 3; q++) {
-                    dpx_point p = c[3 * t + q];
-                    v[2 * q] = (int)((p.x - fi) * 64.0f) * 2 * scale;
-                    v[2 * q + 1] = (int)((p.y - fj) * 64.0f) * 2 * scale;
-                }
-                if (tri_covers(v[0], v[1], v[2], v[3], v[4], v[5], sx, sy)) {
-                    color = cell_rgba(load_px(im, ci, cj), colour_channels(im));
-                    done = true;
-                    break;
-                }
-            }
-        }
-    int row = out_topdown(im.flags) ? (OH - 1 - Y) : Y;
-    *reinterpret_cast<uint32_t*>(out + (size_t)row * out_stride + (size_t)X * 4) = color;
-}
-
 // ---------------------------------------------------------------------------
-// Presentation: the GLUT window (display() callbacks.cpp:39-72, renderCuda
-// simpleVBO.cpp:185-440).  Window point (X + ox/8, Y + oy/8) maps to image
-// point ((8 (X - tx) + ox) * 100) / (8 * sc), sc the scale in hundredths.  In
-// units of 1/(512 sc) of a cell that is (8 (X - tx) + ox) * 6400 and a
-// 1/64-lattice vertex v is 64 v * 8 sc: both integers, so coverage is exact.
+// glDrawArrays(GL_TRIANGLES) in VBO order (simpleVBO.cpp:281) as a gather,
+// for the frame's raster and for the GLUT window (display()
+// callbacks.cpp:39-72, renderCuda simpleVBO.cpp:185-440): a sample takes the
+// colour of the highest-index cell (the last one drawn) with a triangle that
+// covers it.  Cells reach at most 0.34 past their unit square, so the cells
+// around the sample's own are the candidates.
+//
+// All coordinates are whole numbers of a unit such that a cell is `unit` of
+// them: 1/(128 scale) of a cell for the raster, 1/(512 sc) for the window
+// (sc the scale in hundredths).  Sample s of output pixel (X, Y) lies at
+// (step X + ox[s], step Y + oy[s]) and a 1/64-lattice vertex v at v unit / 64.
+// Window point (X + ox/8, Y + oy/8) is image point ((8 (X - tx) + ox) * 100)
+// / (8 * sc), i.e. (8 (X - tx) + ox) * 6400 units.
 // ---------------------------------------------------------------------------
-struct ViewGeom {
-    int mode, sc, tx, ty, W, H, aa, topdown;
+struct TriGeom {
+    int unit, step;         // of a cell, of an output pixel
+    long long ox[4], oy[4]; // samples of pixel (0, 0)
+    int W, H;               // output pixels
+    int topdown;            // output row 0 is the top one
+    int quads;              // each image pixel as its square
 };
 
 __device__ inline long long floor_div(long long a, long long b)  // b > 0
@@ -273,64 +505,280 @@ __device__ inline long long floor_div(long long a, long long b)  // b > 0
     return (a % b != 0 && a < 0) ? q - 1 : q;
 }
 
-// colour of the sample at window position (8 X + ox, 8 Y + oy) / 8
-__device__ inline uint32_t present_sample(const ImgView& im, const dpx_point* __restrict__ diagram,
-                                          const int32_t* __restrict__ edge_count, const ViewGeom& v, int X, int Y,
-                                          int ox, int oy)
+// The colour of a pixel from its samples': averaged per channel, halves rounded up.
+template <int NS>
+__device__ inline uint32_t tri_average(const uint32_t* col)
 {
-    const long long unit = 512LL * v.sc;  // one cell
-    const long long px = (8LL * (X - v.tx) + ox) * 6400, py = (8LL * (Y - v.ty) + oy) * 6400;
-    const long long ci = floor_div(px, unit), cj = floor_div(py, unit);
-    const int cc = colour_channels(im);
-    if (v.mode == DPX_VIEW_QUADS) {
-        // the two triangles of pixel (ci, cj) cover [ci, ci+1) x [cj, cj+1)
-        // under the coverage rule (left and bottom edges in, right and top out)
-        if (ci < 0 || cj < 0 || ci >= im.W || cj >= im.H) return 0xFF000000u;
-        return cell_rgba(load_px(im, (int)ci, (int)cj), cc);
+    if constexpr (NS == 1) return col[0];
+    uint32_t color = 0;
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        uint32_t sum = NS / 2;
+#pragma unroll
+        for (int s = 0; s < NS; s++) sum += (col[s] >> (8 * b)) & 0xFFu;
+        color |= (sum / NS) << (8 * b);
     }
-    for (int dy = 1; dy >= -1; dy--)
-        for (int dx = 1; dx >= -1; dx--) {  // cells in reverse draw order: the first hit wins
-            long long i = ci + dx, j = cj + dy;
-            if (i < 0 || j < 0 || i >= im.W || j >= im.H) continue;
-            size_t k = (size_t)j * im.W + (size_t)i;
-            int nt = edge_count[k] - 2;
-            if (nt > kCellSize / 3) nt = kCellSize / 3;
-            const long long sx = px - i * unit, sy = py - j * unit;
+    return color;
+}
+
+// A sample's colour over the cells [i0, i1] x [j0, j1] in reverse draw order,
+// straight from the diagram and in 64 bits: any scale and any coordinates.
+__device__ __noinline__ uint32_t tri_sample_any(ImgView im, const dpx_point* __restrict__ diagram,
+                                                const int32_t* __restrict__ edge_count, int unit, int i0, int i1,
+                                                int j0, int j1, long long px, long long py)
+{
+    for (int j = j1; j >= j0; j--)
+        for (int i = i1; i >= i0; i--) {
+            const size_t k = (size_t)j * im.W + (size_t)i;
+            const int nt = min(edge_count[k] - 2, kCellSize / 3);
             const dpx_point* c = &diagram[k * kCellSize];
             const float fi = (float)i, fj = (float)j;
+            const long long sx = px - (long long)i * unit, sy = py - (long long)j * unit;
             for (int t = 0; t < nt; t++) {
                 long long w[6];
 #pragma unroll
                 for (int q = 0; q < 3; q++) {
-                    dpx_point p = c[3 * t + q];
-                    w[2 * q] = (long long)(int)((p.x - fi) * 64.0f) * 8 * v.sc;
-                    w[2 * q + 1] = (long long)(int)((p.y - fj) * 64.0f) * 8 * v.sc;
+                    const dpx_point p = c[3 * t + q];
+                    w[2 * q] = (long long)(int)((p.x - fi) * 64.0f) * (unit / 64);
+                    w[2 * q + 1] = (long long)(int)((p.y - fj) * 64.0f) * (unit / 64);
                 }
                 if (tri_covers(w[0], w[1], w[2], w[3], w[4], w[5], sx, sy))
-                    return cell_rgba(load_px(im, (int)i, (int)j), cc);
+                    return cell_rgba(load_px(im, i, j), colour_channels(im));
             }
         }
-    return 0xFF000000u;  // clear colour (main.cpp:260)
+    return 0xFF000000u;  // clear colour (0,0,0,1), main.cpp:260
 }
 
-// The four antialiasing samples of window pixel (X, Y) in one scan: the
-// cells around all four, in reverse draw order, each triangle read once and
-// tested against every sample not yet covered.  A cell reaches at most a
-// quarter cell beyond its square, so the cells outside a sample's own 3x3
-// never cover it and the first cover found is the sample's last in draw
-// order, as in present_sample.
-__device__ inline void present_samples4(const ImgView& im, const dpx_point* __restrict__ diagram,
-                                        const int32_t* __restrict__ edge_count, const ViewGeom& v, int X, int Y,
-                                        const int* sox, const int* soy, uint32_t* col)
+// 16 x TY output pixels per block.  The cells around them (`cap` of them fit
+// the LDS the launch gave) are read once: each triangle's three edge
+// functions e = dx sy - dy sx + k, counter-clockwise and with the tie of the
+// coverage rule in k (covered: all three above 0), so that a sample's test of
+// a triangle is six multiply-adds; and how far the cells reach beyond their
+// squares, which keeps most pixels to one to four of the cells around them.
+// A vertex within half a cell of its cell and a sample within three cells
+// keep every term in 31 bits and the factors in 24; a cell of a caller's
+// diagram beyond that, and scales with more cells, take tri_sample_any.
+// Bound by the instructions of the tests; straight from memory in 64 bits
+// the 1200x800 window of a smoothed 256x224 frame took 221 us, so 44.
+constexpr int kTris = kCellSize / 3;
+constexpr int kTriLow = -32, kTriHigh = 96;  // 1/64 units
+struct TriEdge {
+    uint32_t d;  // dx | dy << 16
+    int k;
+};
+constexpr size_t kTriCellBytes = 3 * kTris * sizeof(TriEdge) + sizeof(int);
+
+template <int NS, int TY>
+__global__ __launch_bounds__(16 * TY) void k_tri(ImgView im, const dpx_point* __restrict__ diagram,
+                                             const int32_t* __restrict__ edge_count, TriGeom v, int cap,
+                                             uint8_t* __restrict__ out, int out_stride)
 {
-    const long long unit = 512LL * v.sc;
-    long long px[4], py[4];
-    long long i0 = 0, i1 = 0, j0 = 0, j1 = 0;
+    extern __shared__ uint32_t s_dyn[];
+    TriEdge* s_edge = reinterpret_cast<TriEdge*>(s_dyn);
+    int* s_nt = reinterpret_cast<int*>(s_edge + (size_t)cap * 3 * kTris);
+    __shared__ int s_range[4], s_any;
+    __shared__ int s_lo, s_hi;  // the least and greatest vertex coordinate, 1/64 units of its cell
+    constexpr int NT = 16 * TY;
+    const int t = threadIdx.x, X = blockIdx.x * 16 + (t & 15), Y = blockIdx.y * TY + (t >> 4);
+    // The cell of the block's first sample (64-bit, one division a wave), and
+    // every sample relative to that cell in 32 bits.  A block far outside the
+    // image keeps only that it is (its 16 pixels reach at most 64 cells).
+    auto origin = [&](int first, const long long* o) {
+        long long p = o[0];
 #pragma unroll
-    for (int s = 0; s < 4; s++) {
-        px[s] = (8LL * (X - v.tx) + sox[s]) * 6400;
-        py[s] = (8LL * (Y - v.ty) + soy[s]) * 6400;
-        col[s] = 0xFF000000u;  // clear colour (main.cpp:260)
+        for (int s = 1; s < NS; s++) p = min(p, o[s]);
+        return floor_div(p + (long long)v.step * first, (long long)v.unit);
+    };
+    auto near_frame = [](long long c, int n) { return (int)(c < -128 ? -128 : c > n + 64 ? n + 64 : c); };
+    const long long oi = origin(X - (t & 15), v.ox), oj = origin(Y - (t >> 4), v.oy);
+    const int ni = near_frame(oi, im.W), nj = near_frame(oj, im.H);
+    int rx[NS], ry[NS], ci[NS], cj[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        rx[s] = (int)((long long)v.step * (X - (t & 15)) + v.ox[s] - oi * v.unit) + v.step * (t & 15);
+        ry[s] = (int)((long long)v.step * (Y - (t >> 4)) + v.oy[s] - oj * v.unit) + v.step * (t >> 4);
+        ci[s] = ni + floor_div(rx[s], v.unit);
+        cj[s] = nj + floor_div(ry[s], v.unit);
+    }
+    uint32_t col[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) col[s] = 0xFF000000u;  // clear colour (0,0,0,1), main.cpp:260
+    const bool mine = X < v.W && Y < v.H;
+    const int cc = colour_channels(im);
+    if (v.quads) {
+        // the two triangles of pixel (ci, cj) cover [ci, ci+1) x [cj, cj+1)
+        // under the coverage rule (left and bottom edges in, right and top out)
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+            if (mine && in_frame(ci[s], cj[s], im.W, im.H)) col[s] = cell_rgba(load_px(im, ci[s], cj[s]), cc);
+    } else {
+        int i0 = ci[0], i1 = ci[0], j0 = cj[0], j1 = cj[0];
+#pragma unroll
+        for (int s = 1; s < NS; s++) {
+            i0 = min(i0, ci[s]);
+            i1 = max(i1, ci[s]);
+            j0 = min(j0, cj[s]);
+            j1 = max(j1, cj[s]);
+        }
+        // this pixel's candidates, and (corner threads) the block's; pixels
+        // past the output's edge only widen the block's range
+        i0 = max(i0 - 1, 0);
+        j0 = max(j0 - 1, 0);
+        i1 = min(i1 + 1, im.W - 1);
+        j1 = min(j1 + 1, im.H - 1);
+        if (t == 0) {
+            s_range[0] = i0;
+            s_range[1] = j0;
+            s_any = 0;
+            s_lo = 0;
+            s_hi = 64;
+        }
+        if (t == NT - 1) {
+            s_range[2] = i1;
+            s_range[3] = j1;
+        }
+        __syncthreads();
+        const int bi = s_range[0], bj = s_range[1], nci = s_range[2] - bi + 1, ncj = s_range[3] - bj + 1;
+        if (nci > 0 && ncj > 0) {  // (uniform; else no cell lies near this block)
+            const int nc = nci * ncj, vs = v.unit / 64;
+            if (nc > cap) {
+                if (t == 0) s_any = 1;
+            } else {
+                for (int k = t; k < nc; k += NT)
+                    s_nt[k] = min(edge_count[(size_t)(bj + k / nci) * im.W + bi + k % nci] - 2, kTris);
+                __syncthreads();
+                int lo = 0, hi = 64;
+                bool wide = false;
+                for (int k = t; k < nc * kTris; k += NT) {
+                    const int c = k / kTris, q = k - c * kTris;
+                    if (q >= s_nt[c]) continue;
+                    const int i = bi + c % nci, j = bj + c / nci;
+                    const dpx_point* p = &diagram[((size_t)j * im.W + i) * kCellSize + 3 * q];
+                    int x[3], y[3];
+#pragma unroll
+                    for (int e = 0; e < 3; e++) {
+                        x[e] = (int)((p[e].x - (float)i) * 64.0f);
+                        y[e] = (int)((p[e].y - (float)j) * 64.0f);
+                        lo = min(lo, min(x[e], y[e]));
+                        hi = max(hi, max(x[e], y[e]));
+                    }
+                    if (lo < kTriLow || hi > kTriHigh) {
+                        wide = true;
+                        break;
+                    }
+                    // counter-clockwise; a degenerate triangle covers nothing: edges of zeros
+                    const int o = (x[1] - x[0]) * (y[2] - y[0]) - (y[1] - y[0]) * (x[2] - x[0]);
+                    if (o < 0) {
+                        swap2(&x[1], &x[2]);
+                        swap2(&y[1], &y[2]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 3; e++) {
+                        const int f = (e + 1) % 3, dx = o ? x[f] - x[e] : 0, dy = o ? y[f] - y[e] : 0;
+                        const int tie = dy < 0 || (dy == 0 && dx > 0) ? 1 : 0;
+                        s_edge[(c * kTris + q) * 3 + e] = TriEdge{ ((uint32_t)dx & 0xFFFFu) | ((uint32_t)dy << 16),
+                                                                   (dy * x[e] - dx * y[e]) * vs + tie };
+                    }
+                }
+                if (wide) s_any = 1;
+                if (lo < 0) atomicMin(&s_lo, lo);
+                if (hi > 64) atomicMax(&s_hi, hi);
+            }
+            __syncthreads();
+            if (mine && s_any) {
+#pragma unroll 1
+                for (int s = 0; s < NS; s++) {
+                    int sx = rx[0], sy = ry[0];
+#pragma unroll
+                    for (int q = 1; q < NS; q++)
+                        if (q == s) {
+                            sx = rx[q];
+                            sy = ry[q];
+                        }
+                    const uint32_t c = tri_sample_any(im, diagram, edge_count, v.unit, i0, i1, j0, j1,
+                                                      (long long)ni * v.unit + sx, (long long)nj * v.unit + sy);
+#pragma unroll
+                    for (int q = 0; q < NS; q++)
+                        if (q == s) col[q] = c;
+                }
+            } else if (mine) {
+                // cells whose reach ends before all of the pixel's samples
+                const int lo = s_lo * vs, hi = s_hi * vs;
+                int x_lo = rx[0], x_hi = rx[0], y_lo = ry[0], y_hi = ry[0];
+#pragma unroll
+                for (int s = 1; s < NS; s++) {
+                    x_lo = min(x_lo, rx[s]);
+                    x_hi = max(x_hi, rx[s]);
+                    y_lo = min(y_lo, ry[s]);
+                    y_hi = max(y_hi, ry[s]);
+                }
+                while (i0 <= i1 && x_lo - (i0 - ni) * v.unit > hi) i0++;
+                while (i1 >= i0 && x_hi - (i1 - ni) * v.unit < lo) i1--;
+                while (j0 <= j1 && y_lo - (j0 - nj) * v.unit > hi) j0++;
+                while (j1 >= j0 && y_hi - (j1 - nj) * v.unit < lo) j1--;
+                uint32_t left = (1u << NS) - 1u;
+                for (int j = j1; j >= j0 && left; j--)
+                    for (int i = i1; i >= i0 && left; i--) {
+                        const int c = (j - bj) * nci + i - bi, nt = s_nt[c];
+                        int sx[NS], sy[NS];
+#pragma unroll
+                        for (int s = 0; s < NS; s++) {
+                            sx[s] = rx[s] - (i - ni) * v.unit;
+                            sy[s] = ry[s] - (j - nj) * v.unit;
+                        }
+                        uint32_t hit = 0;
+                        const TriEdge* w = s_edge + c * kTris * 3;
+                        for (int q = 0; q < nt && (left & ~hit); q++, w += 3) {
+                            int low[NS];
+#pragma unroll
+                            for (int e = 0; e < 3; e++) {
+                                const TriEdge ed = w[e];
+                                const int dx = point_x(ed.d), dy = -point_y(ed.d);
+#pragma unroll
+                                for (int s = 0; s < NS; s++) {
+                                    const int f = mad24(dx, sy[s], mad24(dy, sx[s], ed.k));
+                                    low[s] = e == 0 ? f : min(low[s], f);
+                                }
+                            }
+#pragma unroll
+                            for (int s = 0; s < NS; s++) hit |= low[s] > 0 ? 1u << s : 0u;
+                        }
+                        hit &= left;
+                        if (hit) {
+                            const uint32_t rgba = cell_rgba(load_px(im, i, j), cc);
+#pragma unroll
+                            for (int s = 0; s < NS; s++)
+                                if ((hit >> s) & 1u) col[s] = rgba;
+                            left &= ~hit;
+                        }
+                    }
+            }
+        }
+    }
+    if (!mine) return;
+    const int row = v.topdown ? (v.H - 1 - Y) : Y;
+    *reinterpret_cast<uint32_t*>(out + (size_t)row * out_stride + (size_t)X * 4) = tri_average<NS>(col);
+}
+
+// Views that put so many cells into a block that they do not fit LDS (scales
+// below 1): a thread per pixel, the cells around all of its samples read
+// once from the diagram, each triangle tested against every sample that no
+// cell has covered yet.
+template <int NS>
+__global__ __launch_bounds__(256) void k_tri_far(ImgView im, const dpx_point* __restrict__ diagram,
+                                                 const int32_t* __restrict__ edge_count, TriGeom v,
+                                                 uint8_t* __restrict__ out, int out_stride)
+{
+    const int X = blockIdx.x * 16 + (threadIdx.x & 15), Y = blockIdx.y * 16 + (threadIdx.x >> 4);
+    if (X >= v.W || Y >= v.H) return;
+    const long long unit = v.unit;
+    long long px[NS], py[NS], i0 = 0, i1 = 0, j0 = 0, j1 = 0;
+    uint32_t col[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        px[s] = (long long)v.step * X + v.ox[s];
+        py[s] = (long long)v.step * Y + v.oy[s];
+        col[s] = 0xFF000000u;  // clear colour (0,0,0,1), main.cpp:260
         const long long ci = floor_div(px[s], unit), cj = floor_div(py[s], unit);
         if (s == 0 || ci < i0) i0 = ci;
         if (s == 0 || ci > i1) i1 = ci;
@@ -338,77 +786,66 @@ __device__ inline void present_samples4(const ImgView& im, const dpx_point* __re
         if (s == 0 || cj > j1) j1 = cj;
     }
     // the window may lie far outside the image: clamp to the frame
-    j0 = j0 - 1 < 0 ? 0 : j0 - 1;
     i0 = i0 - 1 < 0 ? 0 : i0 - 1;
-    j1 = j1 + 1 > im.H - 1 ? im.H - 1 : j1 + 1;
+    j0 = j0 - 1 < 0 ? 0 : j0 - 1;
     i1 = i1 + 1 > im.W - 1 ? im.W - 1 : i1 + 1;
+    j1 = j1 + 1 > im.H - 1 ? im.H - 1 : j1 + 1;
     const int cc = colour_channels(im);
-    uint32_t left = 0xFu;
+    uint32_t left = (1u << NS) - 1u;
     for (long long j = j1; j >= j0 && left; j--)
         for (long long i = i1; i >= i0 && left; i--) {
-            size_t k = (size_t)j * im.W + (size_t)i;
-            int nt = edge_count[k] - 2;
-            if (nt > kCellSize / 3) nt = kCellSize / 3;
+            const size_t k = (size_t)j * im.W + (size_t)i;
+            const int nt = min(edge_count[k] - 2, kCellSize / 3);
             const dpx_point* c = &diagram[k * kCellSize];
             const float fi = (float)i, fj = (float)j;
-            long long sx[4], sy[4];
-#pragma unroll
-            for (int s = 0; s < 4; s++) { sx[s] = px[s] - i * unit; sy[s] = py[s] - j * unit; }
             uint32_t hit = 0;
             for (int t = 0; t < nt && (left & ~hit); t++) {
                 long long w[6];
 #pragma unroll
                 for (int q = 0; q < 3; q++) {
-                    dpx_point p = c[3 * t + q];
-                    w[2 * q] = (long long)(int)((p.x - fi) * 64.0f) * 8 * v.sc;
-                    w[2 * q + 1] = (long long)(int)((p.y - fj) * 64.0f) * 8 * v.sc;
+                    const dpx_point p = c[3 * t + q];
+                    w[2 * q] = (long long)(int)((p.x - fi) * 64.0f) * (v.unit / 64);
+                    w[2 * q + 1] = (long long)(int)((p.y - fj) * 64.0f) * (v.unit / 64);
                 }
 #pragma unroll
-                for (int s = 0; s < 4; s++)
+                for (int s = 0; s < NS; s++)
                     if (((left & ~hit) >> s) & 1u)
-                        if (tri_covers(w[0], w[1], w[2], w[3], w[4], w[5], sx[s], sy[s])) hit |= 1u << s;
+                        if (tri_covers(w[0], w[1], w[2], w[3], w[4], w[5], px[s] - i * unit, py[s] - j * unit))
+                            hit |= 1u << s;
             }
             if (hit) {
                 const uint32_t rgba = cell_rgba(load_px(im, (int)i, (int)j), cc);
 #pragma unroll
-                for (int s = 0; s < 4; s++)
+                for (int s = 0; s < NS; s++)
                     if ((hit >> s) & 1u) col[s] = rgba;
                 left &= ~hit;
             }
         }
+    const int row = v.topdown ? (v.H - 1 - Y) : Y;
+    *reinterpret_cast<uint32_t*>(out + (size_t)row * out_stride + (size_t)X * 4) = tri_average<NS>(col);
 }
 
-__global__ void k_present(ImgView im, const dpx_point* __restrict__ diagram, const int32_t* __restrict__ edge_count,
-                          ViewGeom v, uint8_t* __restrict__ out, int out_stride)
+void launch_tri(const ImgView& im, const dpx_point* diagram, const int32_t* edge_count, const TriGeom& v, int samples,
+                uint8_t* out, int out_stride, hipStream_t stream)
 {
-    int X = blockIdx.x * blockDim.x + threadIdx.x;
-    int Y = blockIdx.y * blockDim.y + threadIdx.y;
-    if (X >= v.W || Y >= v.H) return;
-    uint32_t color;
-    if (!v.aa) {
-        color = present_sample(im, diagram, edge_count, v, X, Y, 4, 4);
-    } else {
-        // rotated 4x grid, averaged per channel with halves rounded up
-        const int sox[4] = { 3, 7, 1, 5 }, soy[4] = { 1, 3, 5, 7 };
-        uint32_t sum[4] = { 0, 0, 0, 0 }, cs[4];
-        if (v.mode == DPX_VIEW_QUADS) {
-#pragma unroll
-            for (int s = 0; s < 4; s++) cs[s] = present_sample(im, diagram, edge_count, v, X, Y, sox[s], soy[s]);
-        } else {
-            present_samples4(im, diagram, edge_count, v, X, Y, sox, soy, cs);
-        }
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const uint32_t c = cs[s];
-#pragma unroll
-            for (int b = 0; b < 4; b++) sum[b] += (c >> (8 * b)) & 0xFFu;
-        }
-        color = 0;
-#pragma unroll
-        for (int b = 0; b < 4; b++) color |= ((sum[b] + 2) >> 2) << (8 * b);
+    // cells that n output pixels reach on one axis: their own, a part at each
+    // end and one around each side
+    auto reach = [&](int n) { return ((long long)n * v.step - 1) / v.unit + 4; };
+    auto lds_of = [&](int ty) { return (size_t)(reach(16) * reach(ty)) * kTriCellBytes; };
+    // tiles of 16 rows where their cells leave room for several blocks a CU
+    // (from 2.5x up), else of 4 rows (from 1x up: 48 KB), else no LDS
+    const bool tall = v.quads || lds_of(16) <= 40 * 1024;
+    const int ty = tall ? 16 : 4, cap = v.quads ? 0 : (int)std::min(reach(16) * reach(ty), 1LL << 20);
+    const size_t lds = v.quads ? 0 : lds_of(ty);
+    const dim3 grid((unsigned)((v.W + 15) / 16), (unsigned)((v.H + ty - 1) / ty));
+    if (lds > 60 * 1024) {
+        const dim3 far((unsigned)((v.W + 15) / 16), (unsigned)((v.H + 15) / 16));
+        hipLaunchKernelGGL(samples == 4 ? k_tri_far<4> : k_tri_far<1>, far, dim3(256), 0, stream, im, diagram,
+                           edge_count, v, out, out_stride);
+        return;
     }
-    int row = v.topdown ? (v.H - 1 - Y) : Y;
-    *reinterpret_cast<uint32_t*>(out + (size_t)row * out_stride + (size_t)X * 4) = color;
+    auto fn = samples == 4 ? (tall ? k_tri<4, 16> : k_tri<4, 4>) : (tall ? k_tri<1, 16> : k_tri<1, 4>);
+    hipLaunchKernelGGL(fn, grid, dim3(16 * ty), lds, stream, im, diagram, edge_count, v, cap, out, out_stride);
 }
 
 // ---------------------------------------------------------------------------
@@ -584,8 +1021,9 @@ extern "C" int dpx_stage_cells(const uint8_t* d_graph, int W, int H, dpx_point* 
                                void* stream)
 {
     DPX_CHECK(d_graph && d_diagram && d_edge_count && W > 0 && H > 0, DPX_EINVAL, "bad arguments");
-    hipLaunchKernelGGL(k_cells, grid2(W, H), dim3(kB, kB), 0, as_stream(stream), d_graph, W, H, d_diagram,
-                       d_edge_count);
+    const size_t N = (size_t)W * H;
+    hipLaunchKernelGGL(k_cells, dim3((unsigned)((N + kRun - 1) / kRun)), dim3(256), 0, as_stream(stream), d_graph, N,
+                       d_diagram, d_edge_count);
     DPX_HIP(hipGetLastError());
     return DPX_OK;
 }
@@ -602,7 +1040,8 @@ extern "C" int dpx_stage_subdivide(const uint8_t* d_img, int W, int H, int strid
     DPX_HIP(hipMemcpyAsync(d_diagram_aux, d_diagram, N * kCellSize * sizeof(dpx_point), hipMemcpyDeviceToDevice, s));
     DPX_HIP(hipMemcpyAsync(d_edge_count_aux, d_edge_count, N * sizeof(int32_t), hipMemcpyDeviceToDevice, s));
     ImgView im{ d_img, W, H, stride, ch, flags };
-    hipLaunchKernelGGL(k_subdivide, grid2(W, H), dim3(kB, kB), 0, s, im, d_graph, d_diagram, d_diagram_aux,
+    const dim3 tiles((unsigned)((W + kSubX - 1) / kSubX), (unsigned)((H + kSubY - 1) / kSubY));
+    hipLaunchKernelGGL(k_subdivide, tiles, dim3(256), 0, s, im, d_graph, d_diagram, d_diagram_aux,
                        d_edge_count, d_edge_count_aux);
     DPX_HIP(hipGetLastError());
     return DPX_OK;
@@ -611,7 +1050,9 @@ extern "C" int dpx_stage_subdivide(const uint8_t* d_img, int W, int H, int strid
 extern "C" int dpx_stage_triangulate(dpx_point* d_diagram, const int32_t* d_edge_count, int W, int H, void* stream)
 {
     DPX_CHECK(d_diagram && d_edge_count && W > 0 && H > 0, DPX_EINVAL, "bad arguments");
-    hipLaunchKernelGGL(k_triangulate, grid2(W, H), dim3(kB, kB), 0, as_stream(stream), d_diagram, d_edge_count, W, H);
+    const size_t N = (size_t)W * H;
+    hipLaunchKernelGGL(k_triangulate, dim3((unsigned)((N + kTriRun - 1) / kTriRun)), dim3(kTriBlock), 0,
+                       as_stream(stream), d_diagram, d_edge_count, W, N);
     DPX_HIP(hipGetLastError());
     return DPX_OK;
 }
@@ -623,7 +1064,8 @@ extern "C" int dpx_stage_export_vbo(const uint8_t* d_img, int W, int H, int stri
     if (int rc = check_img(d_img, W, H, stride, ch, flags)) return rc;
     DPX_CHECK(d_diagram && d_edge_count && (d_pos || d_color), DPX_EINVAL, "bad arguments");
     ImgView im{ d_img, W, H, stride, ch, flags };
-    hipLaunchKernelGGL(k_export_vbo, grid2(W, H), dim3(kB, kB), 0, as_stream(stream), im, d_diagram, d_edge_count,
+    const size_t N = (size_t)W * H;
+    hipLaunchKernelGGL(k_export_vbo, dim3((unsigned)((N + kRun - 1) / kRun)), dim3(256), 0, as_stream(stream), im, d_diagram, d_edge_count,
                        d_pos, d_color);
     DPX_HIP(hipGetLastError());
     return DPX_OK;
@@ -639,8 +1081,14 @@ extern "C" int dpx_stage_rasterize(const uint8_t* d_img, int W, int H, int strid
     DPX_CHECK((long long)W * scale <= 65536 && (long long)H * scale <= 65536, DPX_EINVAL, "output too large");
     DPX_CHECK(out_stride >= 4 * W * scale && out_stride % 4 == 0, DPX_EINVAL, "bad out_stride %d", out_stride);
     ImgView im{ d_img, W, H, stride, ch, flags };
-    hipLaunchKernelGGL(k_raster_tri, grid2(W * scale, H * scale), dim3(kB, kB), 0, as_stream(stream), im, d_diagram,
-                       d_edge_count, scale, d_out, out_stride);
+    TriGeom v{};
+    v.unit = 128 * scale;
+    v.step = 128;
+    v.ox[0] = v.oy[0] = 64;
+    v.W = W * scale;
+    v.H = H * scale;
+    v.topdown = out_topdown(flags);
+    launch_tri(im, d_diagram, d_edge_count, v, 1, d_out, out_stride, as_stream(stream));
     DPX_HIP(hipGetLastError());
     return DPX_OK;
 }
@@ -666,10 +1114,21 @@ extern "C" int dpx_stage_present(const uint8_t* d_img, int W, int H, int stride,
               "unknown view flags");
     DPX_CHECK(out_stride >= 4 * view->width && out_stride % 4 == 0, DPX_EINVAL, "bad out_stride %d", out_stride);
     ImgView im{ d_img, W, H, stride, ch, flags };
-    ViewGeom v{ view->mode, view->scale_x100, view->translate_x, view->translate_y, view->width, view->height,
-                (view->flags & DPX_VIEW_AA) ? 1 : 0, (view->flags & DPX_VIEW_TOPDOWN) ? 1 : 0 };
-    hipLaunchKernelGGL(k_present, grid2(v.W, v.H), dim3(kB, kB), 0, as_stream(stream), im, d_diagram, d_edge_count, v,
-                       d_out, out_stride);
+    const bool aa = view->flags & DPX_VIEW_AA;
+    TriGeom v{};
+    v.unit = 512 * view->scale_x100;
+    v.step = 8 * 6400;
+    // rotated 4x grid, or the pixel's centre
+    const int sox[4] = { 3, 7, 1, 5 }, soy[4] = { 1, 3, 5, 7 };
+    for (int s = 0; s < 4; s++) {
+        v.ox[s] = ((aa ? sox[s] : 4) - 8LL * view->translate_x) * 6400;
+        v.oy[s] = ((aa ? soy[s] : 4) - 8LL * view->translate_y) * 6400;
+    }
+    v.W = view->width;
+    v.H = view->height;
+    v.topdown = (view->flags & DPX_VIEW_TOPDOWN) ? 1 : 0;
+    v.quads = view->mode == DPX_VIEW_QUADS;
+    launch_tri(im, d_diagram, d_edge_count, v, aa ? 4 : 1, d_out, out_stride, as_stream(stream));
     DPX_HIP(hipGetLastError());
     return DPX_OK;
 }
