@@ -10,6 +10,7 @@
 #include "common.hpp"
 #include "geom.hpp"
 #include "graph.hpp"
+#include "hull_table.hpp"
 #include "pixel.hpp"
 
 namespace dpx {
@@ -19,7 +20,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 [[maybe_unused]] constexpr int kMaxScale = 15;
 [[maybe_unused]] constexpr int kKeys = 4096;
-constexpr int kHullBytes = 32;  // n, x[8], y[8] (quarter units), padding
 
 __host__ __device__ constexpr int mask_kmin(int S) { return -(S / 2) - 1; }
 __host__ __device__ constexpr int mask_w(int S) { return 2 * S + 2; }
@@ -354,38 +354,52 @@ __device__ inline void tile_resolved_load(const DevItem& it, const uint8_t* __re
 
 // ---------------------------------------------------------------------------
 // kf_smooth: crossing resolution, cells and corner-cutting subdivision of a
-// 32x8-cell tile (subdivision_Kernel kernel.cu:216-261 on the cells_Kernel
+// tile of cells (subdivision_Kernel kernel.cu:216-261 on the cells_Kernel
 // hulls, then triangulate_Kernel's ear clipping, kernel.cu:264-282), each
 // own cell once.  Writes the tile's resolved graph bytes to gfin and, for
 // every smoothed (non-internal) cell, the coverage rows of its triangles at
 // scale S with their summary to `rows` (rows_words(S) words per cell).
 // Internal cells (node 90) keep their hull (kernel.cu:231): the raster takes
-// their rows from the table.  The cells that need smoothing are listed first
-// so that every lane of a wave works on one; each lane's polygon lives in
-// LDS (a column of s_poly), where ear clipping scans and shifts it.
+// their rows from the table.
+//
+// Bound by instructions, so each part does the least a lane can do: hulls
+// are one table word each, held in registers; a cell's T-junction colours
+// are read side by side; the rows come from the polygon's edges, only where
+// an edge crosses a row, toggled into an LDS column; and the ear clipping,
+// which is needed only to know that it cuts the whole polygon (else the
+// triangles cut so far are the cell), runs for the few polygons for which
+// that is not plain, gathered into the first lanes.  The cells are listed by
+// the size of their hull, so that the lanes of a wave end together.  16 frames
+// of 640x480 at 8x: 335 us (606 with every row of every edge visited, every
+// cell clipped, and hulls and colours read per vertex); 64 of 251x223 at 4x:
+// 145 (334).
 // ---------------------------------------------------------------------------
 template <int S, int TX, bool WALK>
-__global__ __launch_bounds__(256, 4) void kf_smooth(const DevItem* __restrict__ items, const uint2* __restrict__ tile_map,
+__global__ __launch_bounds__(256, 3) void kf_smooth(const DevItem* __restrict__ items, const uint2* __restrict__ tile_map,
                                                  int grid3d, const uint8_t* __restrict__ in,
                                                  const uint8_t* __restrict__ gaux, uint8_t* __restrict__ gfin,
-                                                 const int8_t* __restrict__ hull_table, uint32_t* __restrict__ rows)
+                                                 uint32_t* __restrict__ rows)
 {
     DPX_TILE_NAMES(TX);
     constexpr int MW = mask_w(S), KMIN = mask_kmin(S), RW = rows_words(S);
-    constexpr int HB = 20;  // LDS bytes per hull: n, x[8], y[8] (quarter units), 3 bytes of padding
+    constexpr int PITCH = 257;  // of the rows: adjacent rows of a cell in adjacent banks
     __shared__ uint32_t s_aux32[AY * RWW];
     __shared__ uint32_t s_p32[(GY + 1) * RWW];
     __shared__ uint16_t s_blk[(GY + 1) * RDB];
     __shared__ int s_nblk;
     __shared__ uint32_t s_g32[GY * RWW];
-    __shared__ uint32_t s_hull32[RCX * RCY * HB / 4];
-    const int8_t* s_hull = reinterpret_cast<const int8_t*>(s_hull32);
+    __shared__ HullBits s_hull[RCX * RCY];
     __shared__ uint16_t s_list[RTX * RTY];
-    __shared__ int s_nlist;
-    __shared__ int s_bin[16];  // own cells to smooth per hull size, then the first list place of each size
-    // point k of lane t at [k * 256 + t]: x | y << 16 (1/64 units); a hull has
-    // at most 8 vertices (the table's), its smoothed polygon at most 16
-    __shared__ uint32_t s_poly[16 * 256];
+    __shared__ int s_bin[16];  // own cells to smooth per hull size
+    __shared__ int s_nlist, s_nclip;
+    __shared__ uint8_t s_clip[RTX * RTY];  // columns whose polygon is clipped
+    __shared__ uint8_t s_m[RTX * RTY];     // vertices of a column's polygon; 0 once its clipping has failed
+    // vertex k of column t at [k * 256 + t]; a hull has at most 8 vertices,
+    // its smoothed polygon at most 16, within the cells around (-64 .. 127)
+    __shared__ uint16_t s_poly[16 * 256];
+    // sample row r of column t at [r * PITCH + t], then the summary; first the walk window
+    constexpr int COV = RW * PITCH, WALK_WORDS = WALK ? WalkWindow<TX>::BYTES / 4 : 0;
+    __shared__ uint32_t s_cov[COV > WALK_WORDS ? COV : WALK_WORDS];
     const uint8_t* s_g = reinterpret_cast<const uint8_t*>(s_g32);
 
     const int t = threadIdx.x;
@@ -395,161 +409,126 @@ __global__ __launch_bounds__(256, 4) void kf_smooth(const DevItem* __restrict__ 
     const uint8_t* aux = gaux + it.g_off;
     const int ay0 = y0 - 2;
     if (t == 0) {
-        s_nlist = 0;
+        s_nclip = 0;
         s_nblk = 0;
     }
     if (t < 16) s_bin[t] = 0;
     if (t < (GY + 1) * RWW) s_p32[t] = 0;
     tile_snapshot_load<TX>(it, aux, x0, ay0, s_aux32, t);
     __syncthreads();
-    static_assert(16 * 256 * 4 >= WalkWindow<TX>::BYTES, "the polygon buffer holds the walk window first");
-    tile_resolve<TX, WALK>(it, aux, gfin, x0, y0, ay0, s_aux32, s_p32, s_blk, &s_nblk, s_g32, s_poly, t);
+    tile_resolve<TX, WALK>(it, aux, gfin, x0, y0, ay0, s_aux32, s_p32, s_blk, &s_nblk, s_g32, s_cov, t);
     __syncthreads();
     // hulls of the own cells and of their neighbours: cell (x0 - 1 + lx,
     // y0 - 1 + ly) at resolved row ly, byte lx + 7
-    for (int k = t; k < RCX * RCY; k += 256) {
+#pragma unroll
+    for (int q = 0; q < (RCX * RCY + 255) / 256; q++) {
+        const int k = t + 256 * q;
+        if (k >= RCX * RCY) break;
         const int lx = k % RCX, ly = k / RCX;
         const int c = ly * RWB + lx + 7;
-        const uint32_t key = cell_key(s_g[c], s_g[c - 1], s_g[c + 1]);
-        // the first HB bytes of the table's 32-byte entry, as words
-        const uint32_t* e = reinterpret_cast<const uint32_t*>(hull_table + (size_t)key * kHullBytes);
-#pragma unroll
-        for (int q = 0; q < HB / 4; q++) s_hull32[k * (HB / 4) + q] = e[q];
+        s_hull[k] = kHullTable[cell_key(s_g[c], s_g[c - 1], s_g[c + 1])];
     }
-    // own cells to smooth: in the frame and not internal, listed by the size
-    // of their hull (a cell's work grows with it), largest first, so that
-    // the lanes of a wave smooth polygons of about the same size
+    __syncthreads();
+    // own cells to smooth: in the frame and not internal, largest hulls first
     int my_n = -1, my_rank = 0;
     {
         const int cx = t % RTX, cy = t / RTX;
-        const int c = (cy + 1) * RWB + cx + 8;
-        const uint32_t node = s_g[c];
-        if (x0 + cx < it.W && y0 + cy < it.H && node != 90) {
-            my_n = hull_table[(size_t)cell_key(node, s_g[c - 1], s_g[c + 1]) * kHullBytes];
-            my_rank = atomicAdd(&s_bin[my_n], 1);
+        if (x0 + cx < it.W && y0 + cy < it.H && s_g[(cy + 1) * RWB + cx + 8] != 90) {
+            my_n = hull_count(s_hull[(cy + 1) * RCX + cx + 1]);
+            my_rank = atomicAdd(&s_bin[15 - my_n], 1);
         }
     }
     __syncthreads();
-    if (t == 0) {
-        int acc = 0;
-        for (int b = 15; b >= 0; b--) {
-            const int v = s_bin[b];
-            s_bin[b] = acc;
-            acc += v;
+    if (t < 16) {
+        const int own = s_bin[t];
+        int acc = own;
+#pragma unroll
+        for (int d = 1; d < 16; d <<= 1) {
+            const int v = __shfl_up(acc, d);
+            if (t >= d) acc += v;
         }
-        s_nlist = acc;
+        s_bin[t] = acc - own;
+        if (t == 15) s_nlist = acc;
     }
     __syncthreads();
-    if (my_n >= 0) s_list[s_bin[my_n] + my_rank] = (uint16_t)t;
+    if (my_n >= 0) s_list[s_bin[15 - my_n] + my_rank] = (uint16_t)t;
     __syncthreads();
-    if (t >= s_nlist) return;
-    const int own = s_list[t];
-    const int cx = own % RTX, cy = own / RTX;
-    const int x = x0 + cx, y = y0 + cy;
-    const uint32_t node = s_g[(cy + 1) * RWB + cx + 8];
-    const int hk = (cy + 1) * RCX + cx + 1;
-    const int8_t* h = s_hull + hk * HB;
-    const int n = h[0];
-    struct HullX {
-        const int8_t* p;
-        __device__ int operator[](int k) const { return p[1 + k]; }
-    };
-    struct HullY {
-        const int8_t* p;
-        __device__ int operator[](int k) const { return p[9 + k]; }
-    };
-    ImgView im{ in + it.in_off, it.W, it.H, it.stride, it.ch, it.flags,
-                (it.flags & DPX_INDEXED) ? in + it.pal_off : nullptr };
-    const TjView tv = tj_view(im);
-    auto nbr = [&](int e, auto f) {
-        const int8_t* q = s_hull + (hk + edy(e) * RCX + edx(e)) * HB;
-        return f(HullX{ q }, HullY{ q }, (int)q[0]);
-    };
-    auto tj = [&](int x4, int y4) -> bool { return tjunction(tv, x, y, x4, y4); };
-    uint32_t* P = s_poly + t;  // this lane's column
-    auto px_of = [](uint32_t p) { return (int)(int16_t)(p & 0xFFFFu); };
-    auto py_of = [](uint32_t p) { return (int)p >> 16; };
-    // Ear clipping (process, triangulate_functions.cu:108-217) as ear_clip
-    // does it: vertices in counter-clockwise order (reversed when the
-    // signed area is not positive), first ear tried at (m-1, 0, 1), an ear
-    // needs a positive cross and no other vertex inside or on it, a failure
-    // counter of 2 nv.  The coverage is the union of the ears' rows.  Pass 0
-    // takes it from the polygon's edges (poly_rows_xor: exact when the
-    // clipping cuts the whole polygon and the winding sum certifies it) and
-    // clips only to learn that; a lane where either fails (none in the
-    // synthetic workloads) takes pass 1, which subdivides again and
-    // accumulates each ear's rows as it is cut.
-    uint32_t cov[MW];
-    bool need = true;
-#pragma clang loop unroll(disable)
-    for (int pass = 0; pass < 2; pass++) {
-        if (!need) continue;
-        int m = 0;
-        subdivide_cell_emit(HullX{ h }, HullY{ h }, n, node, nbr, tj, [&](int px, int py) {
-            P[256 * m] = ((uint32_t)px & 0xFFFFu) | ((uint32_t)py << 16);
+    const int nlist = s_nlist;
+    if (nlist == 0) return;  // (uniform)
+    uint16_t* P = s_poly + t;  // this lane's columns
+    uint32_t* C = s_cov + t;
+    int m = 0, wsum = 0;
+    if (t < nlist) {
+        const int own = s_list[t];
+        const int cx = own % RTX, cy = own / RTX;
+        const int x = x0 + cx, y = y0 + cy;
+        const uint32_t node = s_g[(cy + 1) * RWB + cx + 8];
+        const int hk = (cy + 1) * RCX + cx + 1;
+        const HullBits h = s_hull[hk];
+        const ImgView im{ in + it.in_off, it.W, it.H, it.stride, it.ch, it.flags,
+                          (it.flags & DPX_INDEXED) ? in + it.pal_off : nullptr };
+        const uint32_t corners = tj_corners(tj_view(im), x, y);
+        auto nbr = [&](int e) { return s_hull[hk + edy(e) * RCX + edx(e)]; };
+        auto tj = [&](int x4, int y4) -> bool { return tj_kept(corners, x4, y4); };
+        subdivide_hull_emit(h, node, nbr, tj, [&](int px, int py) {
+            P[256 * m] = (uint16_t)(((uint32_t)px & 0xFFu) | ((uint32_t)py << 8));
             m++;
         });
 #pragma unroll
-        for (int r = 0; r < MW; r++) cov[r] = 0;
-        need = false;
-        if (m < 3) continue;
-        int a2 = 0;
-        for (int p = m - 1, q = 0; q < m; p = q++) {
-            const uint32_t A = P[256 * p], B = P[256 * q];
-            a2 += px_of(A) * py_of(B) - px_of(B) * py_of(A);
-        }
-        if (a2 <= 0)
-            for (int lo = 0, hi = m - 1; lo < hi; lo++, hi--) {
-                const uint32_t tmp = P[256 * lo];
-                P[256 * lo] = P[256 * hi];
-                P[256 * hi] = tmp;
-            }
-        int wsum = 0;
-        if (pass == 0) wsum = poly_rows_xor<MW>(P, 256, m, 2 * S, KMIN, cov);
-        int nv = m, count = 2 * nv;
-        for (int v = nv - 1; nv > 2;) {
-            if (0 >= (count--)) break;  // the reference gives up; the triangles cut so far stand
-            int u = v;
-            if (nv <= u) u = 0;
-            v = u + 1;
-            if (nv <= v) v = 0;
-            int w = v + 1;
-            if (nv <= w) w = 0;
-            const uint32_t A = P[256 * u], B = P[256 * v], Cc = P[256 * w];
-            const int ax = px_of(A), ay = py_of(A), bx = px_of(B), by = py_of(B), cx_ = px_of(Cc), cy_ = py_of(Cc);
-            bool ear = ((bx - ax) * (cy_ - ay) - (by - ay) * (cx_ - ax)) > 0;
-            if (ear) {
-                for (int p = 0; p < nv; p++) {
-                    if (p == u || p == v || p == w) continue;
-                    const uint32_t Q = P[256 * p];
-                    if (inside_tri(ax, ay, bx, by, cx_, cy_, px_of(Q), py_of(Q))) {
-                        ear = false;
-                        break;
-                    }
+        for (int r = 0; r < MW; r++) C[PITCH * r] = 0;
+        // seen from its pixel's centre almost every cell goes round once
+        // (no clipping is needed to know that it is cut wholly); the others
+        // are clipped, their vertices counter-clockwise as ear_clip takes them
+        if (!poly_star(P, 256, m, 32, 32)) {
+            if (poly_shape(P, 256, m).area2 <= 0)
+                for (int lo = 0, hi = m - 1; lo < hi; lo++, hi--) {
+                    const uint16_t tmp = P[256 * lo];
+                    P[256 * lo] = P[256 * hi];
+                    P[256 * hi] = tmp;
                 }
-            }
-            if (ear) {
-                // coverage of triangle (A, B, C) in units of 1/(128 S) of a
-                // cell; it is counter-clockwise (positive cross)
-                if (pass == 1)
-                    tri_rows_or<MW>(ax * 2 * S, ay * 2 * S, bx * 2 * S, by * 2 * S, cx_ * 2 * S, cy_ * 2 * S, KMIN,
-                                    cov);
-                for (int s2 = v, t2 = v + 1; t2 < nv; s2++, t2++) P[256 * s2] = P[256 * t2];
-                nv--;
-                count = 2 * nv;
-            }
+            s_clip[atomicAdd(&s_nclip, 1)] = (uint8_t)t;
         }
-        if (pass == 0) {
-            int bits = 0;
-#pragma unroll
-            for (int r = 0; r < MW; r++) bits += __builtin_popcount(cov[r]);
-            need = nv > 2 || wsum != bits;
-        }
+        wsum = poly_rows_cross<MW>(P, 256, m, 2 * S, KMIN,
+                                   [&](int r, uint32_t mask) { atomicXor(&C[PITCH * r], mask); });
+        s_m[t] = (uint8_t)m;
     }
-    uint32_t* dst = rows + it.rows_off / 4 + (size_t)((uint32_t)y * (uint32_t)it.W + (uint32_t)x) * RW;
+    __syncthreads();
+    if (t < s_nclip) {
+        const int c = s_clip[t];
+        if (ear_clip_ring<16>(s_poly + c, 256, (int)s_m[c], true, [](uint16_t, uint16_t, uint16_t) {}) > 2) s_m[c] = 0;
+    }
+    __syncthreads();
+    if (t < nlist) {
+        int bits = 0;
 #pragma unroll
-    for (int r = 0; r < MW; r++) dst[r] = cov[r];
-    dst[MW] = coverage_info(cov, S);
+        for (int r = 0; r < MW; r++) bits += __builtin_popcount(C[PITCH * r]);
+        if (s_m[t] == 0 || wsum != bits) {
+            // not cut wholly, or a winding other than 0 and 1 (none in the
+            // synthetic workloads): the rows of each ear as it is cut
+            uint32_t cov[MW];
+#pragma unroll
+            for (int r = 0; r < MW; r++) cov[r] = 0;
+            ear_clip_ring<16>(P, 256, m, true, [&](uint16_t A, uint16_t B, uint16_t E) {
+                // units of 1/(128 S) of a cell; counter-clockwise (an ear's cross is positive)
+                tri_rows_or<MW>(vert_x(A) * 2 * S, vert_y(A) * 2 * S, vert_x(B) * 2 * S, vert_y(B) * 2 * S,
+                                vert_x(E) * 2 * S, vert_y(E) * 2 * S, KMIN, cov);
+            });
+#pragma unroll
+            for (int r = 0; r < MW; r++) C[PITCH * r] = cov[r];
+        }
+        uint32_t cov[MW];
+#pragma unroll
+        for (int r = 0; r < MW; r++) cov[r] = C[PITCH * r];
+        C[PITCH * MW] = coverage_info(cov, S);
+    }
+    __syncthreads();
+    // the rows of a cell by adjacent lanes
+    uint32_t* dst = rows + it.rows_off / 4;
+    for (int k = t; k < nlist * RW; k += 256) {
+        const int c = k / RW, r = k - c * RW, own = s_list[c];
+        const uint32_t cell = (uint32_t)(y0 + own / RTX) * (uint32_t)it.W + (uint32_t)(x0 + own % RTX);
+        dst[(size_t)cell * RW + r] = s_cov[PITCH * r + c];
+    }
 }
 
 // `items` are the items of one (scale, subdivision) group, in launch order.
@@ -1046,8 +1025,7 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
 
 using RasterFn = void (*)(const DevItem*, const uint2*, int, const uint8_t*, const uint8_t*, uint8_t*,
                           const uint32_t*, const uint32_t*, const uint16_t*, uint8_t*);
-using SmoothFn = void (*)(const DevItem*, const uint2*, int, const uint8_t*, const uint8_t*, uint8_t*,
-                          const int8_t*, uint32_t*);
+using SmoothFn = void (*)(const DevItem*, const uint2*, int, const uint8_t*, const uint8_t*, uint8_t*, uint32_t*);
 
 // The raster and smoothing kernels of scale S (1..15), per tile shape (one
 // translation unit each: raster_tiles.hip).

@@ -46,20 +46,6 @@ namespace dpx {
 // ---------------------------------------------------------------------------
 // tables
 // ---------------------------------------------------------------------------
-__global__ void kt_hull(int8_t* __restrict__ table)
-{
-    int key = blockIdx.x * blockDim.x + threadIdx.x;
-    if (key >= kKeys) return;
-    int hx[2 * kMaxPts], hy[2 * kMaxPts];
-    int n = cell_hull((uint32_t)key, hx, hy);
-    int8_t* e = table + (size_t)key * kHullBytes;
-    e[0] = (int8_t)n;
-    for (int t = 0; t < 8; t++) {
-        e[1 + t] = (int8_t)(t < n ? hx[t] : 0);
-        e[9 + t] = (int8_t)(t < n ? hy[t] : 0);
-    }
-}
-
 // Coverage bits of one sample row of a polygon given in 1/64 units and
 // already ear-clipped (tri, nt).  Units of the test: 1/(128 S) of a cell.
 __device__ inline uint32_t coverage_row(const int* x, const int* y, const uint8_t* tri, int nt, int S, int r)
@@ -81,16 +67,16 @@ __device__ inline uint32_t coverage_row(const int* x, const int* y, const uint8_
     return bits;
 }
 
-__global__ void kt_mask(const int8_t* __restrict__ hull_table, int S, uint32_t* __restrict__ mask)
+__global__ void kt_mask(int S, uint32_t* __restrict__ mask)
 {
     int gid = blockIdx.x * blockDim.x + threadIdx.x;
     const int mw = mask_w(S);
     if (gid >= kKeys * mw) return;
     int key = gid / mw, r = gid % mw;
-    const int8_t* e = hull_table + (size_t)key * kHullBytes;
-    int n = e[0];
+    const HullBits h = kHullTable[key];
+    const int n = hull_count(h);
     int x[kMaxPoly], y[kMaxPoly];
-    for (int t = 0; t < n; t++) { x[t] = 16 * e[1 + t]; y[t] = 16 * e[9 + t]; }
+    for (int t = 0; t < n; t++) { x[t] = 16 * hull_x(h, t); y[t] = 16 * hull_y(h, t); }
     uint8_t tri[3 * kMaxPoly];
     int ok;
     int nt = ear_clip(x, y, n, tri, &ok);
@@ -328,7 +314,6 @@ struct BatchPlan {
 struct dpx_context {
     BatchPlan plan;
     int device = 0;
-    int8_t* d_hull = nullptr;
     uint32_t* d_mask[dpx::kMaxScale + 1] = {};
     uint16_t* d_info[dpx::kMaxScale + 1] = {};
     uint8_t *d_gaux = nullptr, *d_gfin = nullptr;
@@ -448,7 +433,7 @@ int ensure_mask(dpx_context* ctx, int S)
     const size_t cell_bytes = S <= kMaxCellScale ? (size_t)kKeys * 9 * sizeof(uint16_t) : 0;
     if (!ctx->d_mask[S]) DPX_HIP(hipMalloc(&ctx->d_mask[S], n * sizeof(uint32_t) + cell_bytes));
     if (!ctx->d_info[S]) DPX_HIP(hipMalloc(&ctx->d_info[S], kKeys * sizeof(uint16_t)));
-    hipLaunchKernelGGL(kt_mask, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, ctx->d_hull, S, ctx->d_mask[S]);
+    hipLaunchKernelGGL(kt_mask, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, S, ctx->d_mask[S]);
     if (cell_bytes)
         hipLaunchKernelGGL(kt_cell, dim3((unsigned)((kKeys * 9 + 255) / 256)), dim3(256), 0, 0, ctx->d_mask[S], S,
                            reinterpret_cast<uint16_t*>(ctx->d_mask[S] + n));
@@ -570,11 +555,6 @@ extern "C" int dpx_context_create(int device, dpx_context** out)
         dpx_context_destroy(ctx);
         return rc;
     };
-    if (hipMalloc(&ctx->d_hull, (size_t)kKeys * kHullBytes) != hipSuccess)
-        return cleanup(fail(DPX_ENOMEM, "table allocation failed"));
-    hipLaunchKernelGGL(kt_hull, dim3(kKeys / 256), dim3(256), 0, 0, ctx->d_hull);
-    if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess)
-        return cleanup(fail(DPX_EHIP, "cell table build failed"));
     if (hipEventCreateWithFlags(&ctx->upload_done, hipEventDisableTiming) != hipSuccess)
         return cleanup(fail(DPX_EHIP, "event creation failed"));
     load_tuning(ctx, tuning_path().c_str());
@@ -587,7 +567,6 @@ extern "C" void dpx_context_destroy(dpx_context* ctx)
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     (void)hipDeviceSynchronize();
-    (void)hipFree(ctx->d_hull);
     for (auto* m : ctx->d_mask) (void)hipFree(m);
     for (auto* m : ctx->d_info) (void)hipFree(m);
     (void)hipFree(ctx->d_gaux);
@@ -858,7 +837,7 @@ static int launch_plan(dpx_context* ctx, const BatchPlan& plan, const LaunchArgs
             SmoothFn sf = pick_smooth(pg.scale, pg.tx, pg.walk);
             DPX_CHECK(sf && la.gfin && la.rows, DPX_EINVAL, "no smoothing buffers for scale %d", pg.scale);
             hipLaunchKernelGGL(sf, pg.grid, dim3(256), 0, stream, d_gitems, d_rmap, pg.grid3d, d_in, la.gaux, la.gfin,
-                               ctx->d_hull, la.rows);
+                               la.rows);
         }
         hipLaunchKernelGGL(fn, pg.grid, dim3(256), 0, stream, d_gitems, d_rmap, pg.grid3d, d_in, la.gaux,
                            (pg.sub || la.keep) ? la.gfin : nullptr, la.rows, ctx->d_mask[pg.scale],
@@ -948,7 +927,6 @@ struct NodeArgs {
     const uint8_t* gaux_c;
     uint8_t* gaux;
     uint8_t* gfin;
-    const int8_t* hull;
     const uint32_t* rows_c;
     uint32_t* rows;
     const uint32_t* mask;
@@ -983,8 +961,7 @@ hipKernelNodeParams node_params(dpx_plan* p, int kind, int group, const uint8_t*
         a.rows = p->d_rows;
         a.rows_c = p->d_rows;
         if (kind == 1) {
-            a.hull = p->ctx->d_hull;
-            void* v[8] = { &a.items, &a.map, &a.g3d, &a.in, &a.gaux_c, &a.gfin, &a.hull, &a.rows };
+            void* v[7] = { &a.items, &a.map, &a.g3d, &a.in, &a.gaux_c, &a.gfin, &a.rows };
             memcpy(a.ptrs, v, sizeof(v));
             np.func = reinterpret_cast<void*>(pick_smooth(pg.scale, pg.tx, pg.walk));
         } else {
@@ -1150,9 +1127,9 @@ extern "C" int dpx_batch_timing_read(dpx_context* ctx, dpx_batch_times* out)
 // dpx_batch_run_noalloc: the batched path with every buffer beyond the
 // caller's input and output in one static device array, `scratch`, so that a
 // call allocates nothing.  Layout (all offsets 256-byte aligned):
-//   tables     the hull table, and per scale 1..15 the coverage rows (with
-//              the cell masks at 1x and 2x) and the coverage summaries,
-//              built on the first call on each device;
+//   tables     per scale 1..15 the coverage rows (with the cell masks at 1x
+//              and 2x) and the coverage summaries, built on the first call
+//              on each device;
 //   items      the batch's device items, in item order and grouped by
 //              (scale, subdivision);
 //   tile maps  block -> (item, tile) of the graph launch and of the raster
@@ -1171,7 +1148,7 @@ constexpr size_t na_mask_bytes(int S)
 constexpr size_t na_info_bytes() { return na_align((size_t)kKeys * 2); }
 constexpr size_t na_mask_off(int S)
 {
-    size_t o = na_align((size_t)kKeys * kHullBytes);
+    size_t o = 0;
     for (int s = 1; s < S; s++) o += na_mask_bytes(s) + na_info_bytes();
     return o;
 }
@@ -1240,12 +1217,10 @@ int na_setup(int dev, hipStream_t stream, uint8_t** out)
         uint8_t* ptr = nullptr;
         DPX_HIP(hipGetSymbolAddress((void**)&ptr, HIP_SYMBOL(scratch)));
         DPX_CHECK(ptr, DPX_EHIP, "no device address for the scratch array");
-        int8_t* hull = reinterpret_cast<int8_t*>(ptr);
-        hipLaunchKernelGGL(kt_hull, dim3(kKeys / 256), dim3(256), 0, stream, hull);
         for (int S = 1; S <= kMaxScale; S++) {
             uint32_t* mask = reinterpret_cast<uint32_t*>(ptr + na_mask_off(S));
             const size_t n = (size_t)kKeys * mask_w(S);
-            hipLaunchKernelGGL(kt_mask, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, hull, S, mask);
+            hipLaunchKernelGGL(kt_mask, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, S, mask);
             if (S <= kMaxCellScale)
                 hipLaunchKernelGGL(kt_cell, dim3((unsigned)((kKeys * 9 + 255) / 256)), dim3(256), 0, stream, mask, S,
                                    reinterpret_cast<uint16_t*>(mask + n));

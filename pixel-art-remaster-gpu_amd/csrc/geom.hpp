@@ -335,6 +335,117 @@ __host__ __device__ inline int subdivide_cell(const int* hx, const int* hy, int 
 }
 
 // ---------------------------------------------------------------------------
+// A cell's hull in two words: vertex k at bits 3k of xs (x + 1) and of ys (y +
+// 1), in quarter units; the vertex count (3..8) at bit 24 of xs; fields past
+// the count hold 7, which is no coordinate.
+// ---------------------------------------------------------------------------
+struct HullBits {
+    uint32_t xs, ys;
+};
+
+__host__ __device__ inline int hull_count(HullBits h) { return (int)(h.xs >> 24); }
+__host__ __device__ inline int hull_x(HullBits h, int k) { return (int)((h.xs >> (3 * k)) & 7u) - 1; }
+__host__ __device__ inline int hull_y(HullBits h, int k) { return (int)((h.ys >> (3 * k)) & 7u) - 1; }
+
+__host__ __device__ inline HullBits hull_pack(const int* hx, const int* hy, int n)
+{
+    HullBits h{ (uint32_t)n << 24 | 0xFFFFFFu, 0xFFFFFFu };
+    for (int k = 0; k < n; k++) {
+        h.xs ^= (7u ^ (uint32_t)(hx[k] + 1)) << (3 * k);
+        h.ys ^= (7u ^ (uint32_t)(hy[k] + 1)) << (3 * k);
+    }
+    return h;
+}
+
+// point_index on a packed hull: all fields compared at once
+__host__ __device__ inline int hull_find(HullBits h, int x, int y)
+{
+    if ((unsigned)(x + 1) > 6u || (unsigned)(y + 1) > 6u) return 0;
+    const uint32_t d = ((h.xs ^ ((uint32_t)(x + 1) * 0x249249u)) | (h.ys ^ ((uint32_t)(y + 1) * 0x249249u)));
+    const uint32_t hit = ~(d | d >> 1 | d >> 2) & 0x249249u;  // bit 3k: vertex k
+    return hit ? __builtin_ctz(hit) / 3 : 0;
+}
+
+// linked_edge of the edge (ax, ay) -> (bx, by): its link direction when the
+// cell has that link, else -1.  The direction is the edge's (horizontal,
+// vertical, rising, falling) and the side of the cell's middle it lies on.
+__host__ __device__ inline int hull_link(int ax, int ay, int bx, int by, uint32_t node)
+{
+    const int dx = bx - ax, dy = by - ay;
+    const int kind = dy == 0 ? 0 : dx == 0 ? 1 : dy == dx ? 2 : dy == -dx ? 3 : 4;
+    const int t = (dx == 0 ? ax + bx : ay + by) - 4;  // twice the middle's distance from the cell's
+    if (kind == 4 || t == 0) return -1;
+    // (beyond, before) the middle: 1, 6; 4, 3; 0, 7; 2, 5
+    const int e = (int)((0x52703461u >> (8 * kind + (t > 0 ? 0 : 4))) & 7u);
+    return bit(node, e) ? e : -1;
+}
+
+// The point of a cut edge nearer to its end (nx, ny) (q_point and r_point
+// alike: a quarter of an edge of length up to 1, else an eighth), 1/64 units.
+__host__ __device__ inline void near_point(int nx, int ny, int fx, int fy, int* x, int* y)
+{
+    const int dx = fx - nx, dy = fy - ny;
+    const bool near = dx * dx + dy * dy <= 16;
+    *x = near ? 4 * (3 * nx + fx) : 2 * (7 * nx + fx);
+    *y = near ? 4 * (3 * ny + fy) : 2 * (7 * ny + fy);
+}
+
+// subdivide_cell_emit on packed hulls; nbr(e): the packed hull of the
+// neighbour across graph edge e.  A corner with a link on one of its edges
+// takes that side's cut point from the neighbour and blends; all corners run
+// the same instructions, so that a wave whose cells are at different kinds of
+// corners takes them once and not in turn.
+template <class NbrHull, class TJunction, class Emit>
+__host__ __device__ inline void subdivide_hull_emit(HullBits h, uint32_t node, NbrHull nbr, TJunction tjunction,
+                                                    Emit emit)
+{
+    const int n = hull_count(h);
+    int px = hull_x(h, n - 1), py = hull_y(h, n - 1), vx = hull_x(h, 0), vy = hull_y(h, 0);
+    int lp = hull_link(px, py, vx, vy, node);
+    for (int k = 0; k < n; k++) {
+        const int kn = k + 1 == n ? 0 : k + 1;
+        const int wx = hull_x(h, kn), wy = hull_y(h, kn);
+        const int lk = hull_link(vx, vy, wx, wy, node);
+        const bool sp = lp >= 0, sk = lk >= 0;
+        // linked on both sides: kept; on none: kept if it is a T-junction's
+        if ((sp && sk) || (!sp && !sk && tjunction(vx, vy))) {
+            emit(16 * vx, 16 * vy);
+        } else {
+            // Q: the cut of the edge after the corner, R: of the edge before
+            int rnx = vx, rny = vy, rfx = px, rfy = py, qnx = vx, qny = vy, qfx = wx, qfy = wy, ox = 0, oy = 0;
+            if (sp || sk) {
+                const int e = sk ? lk : lp;
+                ox = edx(e);
+                oy = edy(e);
+                const HullBits o = nbr(e);
+                const int on = hull_count(o), at = hull_find(o, vx - 4 * ox, vy - 4 * oy);
+                const int to = sk ? (at + 1 == on ? 0 : at + 1) : (at == 0 ? on - 1 : at - 1);
+                const int nx = hull_x(o, at), ny = hull_y(o, at), fx = hull_x(o, to), fy = hull_y(o, to);
+                (sk ? qnx : rnx) = nx;
+                (sk ? qny : rny) = ny;
+                (sk ? qfx : rfx) = fx;
+                (sk ? qfy : rfy) = fy;
+            }
+            int qx, qy, rx, ry;
+            near_point(qnx, qny, qfx, qfy, &qx, &qy);
+            near_point(rnx, rny, rfx, rfy, &rx, &ry);
+            qx += sk ? 64 * ox : 0;
+            qy += sk ? 64 * oy : 0;
+            rx += sp ? 64 * ox : 0;
+            ry += sp ? 64 * oy : 0;
+            const int mx = (qx + rx) / 2, my = (qy + ry) / 2;
+            emit(sp ? mx : rx, sp ? my : ry);
+            emit(sk ? mx : qx, sk ? my : qy);
+        }
+        px = vx;
+        py = vy;
+        vx = wx;
+        vy = wy;
+        lp = lk;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Ear clipping (process, triangulate_functions.cu:108-217) on a 1/64-unit
 // polygon.  Writes triangle vertex indices into tri[3*(n-2)] and returns the
 // number of triangles written; *ok = 0 when the reference's error counter
@@ -391,7 +502,7 @@ __host__ __device__ inline int ear_clip(const int* x, const int* y, int n, uint8
 }
 
 // ear_clip on at most MAXN <= 16 vertices in counter-clockwise order, for
-// one lane of a wave: vertex k at P[stride * k], x | y << 16.  ear(A, B, C)
+// one lane of a wave: vertex k at P[stride * k], packed.  ear(A, B, C)
 // receives each triangle as it is cut; returns the number of vertices left (2
 // when the polygon is cut wholly).  The vertices stay where they are: a mask
 // holds those not cut off yet, and the three at hand move along it (after an
@@ -403,25 +514,58 @@ __host__ __device__ inline int ear_clip(const int* x, const int* y, int n, uint8
 // are; coordinates are 16 bits.
 __host__ __device__ inline int mad24(int a, int b, int c);
 
-// Shape of a polygon (vertex k at P[stride * k], x | y << 16): twice its
-// signed area, and whether it is convex once it stands counter-clockwise: no
-// corner turns right or back and the edges' directions go round once
-// (`convex`: straight corners allowed, `strict`: none).
+// Vertices packed x | y << 16 (16 bits each) or x | y << 8 (8 bits each).
+__host__ __device__ inline int vert_x(uint32_t w) { return (int)(int16_t)(w & 0xFFFFu); }
+__host__ __device__ inline int vert_y(uint32_t w) { return (int)w >> 16; }
+__host__ __device__ inline int vert_x(uint16_t w) { return (int)(int8_t)(w & 0xFFu); }
+__host__ __device__ inline int vert_y(uint16_t w) { return (int)(int8_t)(w >> 8); }
+
+// Does a polygon (vertex k at P[stride * k], packed as above) go round the
+// point (cx, cy) once, counter-clockwise, every edge seen from it turning
+// left?  Such a polygon does not meet itself, and ear clipping then cuts it
+// wholly: a polygon that does not meet itself has a triangulation by
+// diagonals that pass through no vertex, whose outer triangles are ears by
+// the reference's test, and cutting one leaves such a polygon again.
+template <class V>
+__host__ __device__ inline bool poly_star(const V* P, int stride, int n, int cx, int cy)
+{
+    const V L = P[stride * (n - 1)];
+    int px = vert_x(L) - cx, py = vert_y(L) - cy, rounds = 0, low = 1;
+    int half = py > 0 || (py == 0 && px > 0);
+    for (int k = 0; k < n; k++) {
+        const V w = P[stride * k];
+        const int x = vert_x(w) - cx, y = vert_y(w) - cy;
+        const int c = mad24(px, y, mad24(-py, x, 0));
+        low = c < low ? c : low;
+        const int h = y > 0 || (y == 0 && x > 0);
+        rounds += h & ~half;
+        half = h;
+        px = x;
+        py = y;
+    }
+    return low > 0 && rounds == 1;
+}
+
+// Shape of a polygon (packed as above): twice its signed area, and whether it
+// is convex once it stands counter-clockwise: no corner turns right or back
+// and the edges' directions go round once (`convex`: straight corners
+// allowed, `strict`: none).
 struct PolyShape {
     int area2;
     bool convex, strict;
 };
-__host__ __device__ inline PolyShape poly_shape(const uint32_t* P, int stride, int n)
+template <class V>
+__host__ __device__ inline PolyShape poly_shape(const V* P, int stride, int n)
 {
     PolyShape s;
     int a2 = 0, left = 0, right = 0, back = 0, straight = 0, rounds = 0;
-    const uint32_t L = P[stride * (n - 1)], K = P[stride * (n - 2)];
-    int px = (int)(int16_t)(L & 0xFFFFu), py = (int)L >> 16;
-    int ex = px - (int)(int16_t)(K & 0xFFFFu), ey = py - ((int)K >> 16);
+    const V L = P[stride * (n - 1)], K = P[stride * (n - 2)];
+    int px = vert_x(L), py = vert_y(L);
+    int ex = px - vert_x(K), ey = py - vert_y(K);
     int half = ey > 0 || (ey == 0 && ex > 0);
     for (int k = 0; k < n; k++) {  // edge from vertex k - 1 to k, and the corner before it
-        const uint32_t w = P[stride * k];
-        const int x = (int)(int16_t)(w & 0xFFFFu), y = (int)w >> 16, dx = x - px, dy = y - py;
+        const V w = P[stride * k];
+        const int x = vert_x(w), y = vert_y(w), dx = x - px, dy = y - py;
         a2 += mad24(px, y, mad24(-x, py, 0));
         const int c = mad24(ex, dy, mad24(-ey, dx, 0)), d = mad24(ex, dx, mad24(ey, dy, 0));
         left |= c > 0;
@@ -454,16 +598,16 @@ __host__ __device__ inline int mad24(int a, int b, int c)
 
 // With `test` false (the caller knows the polygon to be strictly convex) no
 // vertex can lie in another three's triangle, and none is looked at.
-template <int MAXN, class Ear>
-__host__ __device__ inline int ear_clip_ring(const uint32_t* P, int stride, int n, bool test, Ear ear)
+template <int MAXN, class V, class Ear>
+__host__ __device__ inline int ear_clip_ring(const V* P, int stride, int n, bool test, Ear ear)
 {
     static_assert(MAXN <= 16, "coordinates are 16 bits");
     int x[MAXN], y[MAXN];
 #pragma unroll
     for (int k = 0; k < MAXN; k++) {
-        const uint32_t w = k < n ? P[stride * k] : 0u;
-        x[k] = (int)(int16_t)(w & 0xFFFFu);
-        y[k] = (int)w >> 16;
+        const V w = k < n ? P[stride * k] : V(0);
+        x[k] = vert_x(w);
+        y[k] = vert_y(w);
     }
     uint32_t alive = (1u << n) - 1u;
     auto next = [&](int k) {
@@ -471,12 +615,10 @@ __host__ __device__ inline int ear_clip_ring(const uint32_t* P, int stride, int 
         return __builtin_ctz(m ? m : alive);
     };
     int nv = n, count = 2 * nv, u = n - 1, v = 0, w = 1;
-    uint32_t A = P[stride * u], B = P[stride * v], C = P[stride * w];
+    V A = P[stride * u], B = P[stride * v], C = P[stride * w];
     while (nv > 2) {
         if (0 >= (count--)) break;  // the reference gives up; the triangles cut so far stand
-        const int ax = (int)(int16_t)(A & 0xFFFFu), ay = (int)A >> 16;
-        const int bx = (int)(int16_t)(B & 0xFFFFu), by = (int)B >> 16;
-        const int cx = (int)(int16_t)(C & 0xFFFFu), cy = (int)C >> 16;
+        const int ax = vert_x(A), ay = vert_y(A), bx = vert_x(B), by = vert_y(B), cx = vert_x(C), cy = vert_y(C);
         // edges B -> C, A -> B, C -> A: cross = dx py - dy px + k
         const int dx1 = cx - bx, dy1 = cy - by, dx2 = bx - ax, dy2 = by - ay, dx3 = ax - cx, dy3 = ay - cy;
         bool cut = mad24(dx2, -dy3, mad24(dy2, dx3, 0)) > 0;
@@ -652,43 +794,64 @@ __host__ __device__ inline void tri_rows_or(int ax, int ay, int bx, int by, int 
 // (the masks' signed bit counts).  The union of the triangles (w >= 1) is
 // the parity exactly when every w is 0 or 1, i.e. when that sum equals the
 // number of set bits of cov: the caller's check.
-// P: vertex k at P[stride * k], x | y << 16 in 1/64 units of a cell;
-// coordinates are scaled by 2 S as for tri_rows_or.
-template <int MW>
-__host__ __device__ inline int poly_rows_xor(const uint32_t* P, int stride, int m, int S2, int kmin, uint32_t* cov)
+// P: vertex k at P[stride * k], packed, in 1/64 units of a cell; coordinates
+// are scaled by 2 S as for tri_rows_or.  Only the rows that an edge crosses
+// are visited (a smoothed cell's 8 to 16 edges cross one or two each, of 10
+// rows at 4x and 18 at 8x), the crossing's column from the exact numerator
+// by a reciprocal and one step: toggle(r, mask) receives each.
+template <int MW, class V, class Toggle>
+__host__ __device__ inline int poly_rows_cross(const V* P, int stride, int m, int S2, int kmin, Toggle toggle)
 {
-    const int sy0 = 128 * kmin + 64;
+    const int s0 = 128 * kmin + 64;  // the first sample row, and column
     int wsum = 0;
+    V A = P[stride * (m - 1)];
     for (int k = 0; k < m; k++) {
-        const uint32_t A = P[stride * k], B = P[stride * (k + 1 == m ? 0 : k + 1)];
-        const int px = (int)(int16_t)(A & 0xFFFFu) * S2, py = ((int)A >> 16) * S2;
-        const int qx = (int)(int16_t)(B & 0xFFFFu) * S2, qy = ((int)B >> 16) * S2;
-        const int dx = qx - px, dy = qy - py;
-        if (dy == 0) continue;
-        const int ylo = min(py, qy), yhi = max(py, qy);
-        const int D = 128 * (dy < 0 ? -dy : dy);
-        // column bound at row 0 (as tri_rows_or): N = dx (sy0 - py) + dy (px - sy0)
-        const int N0 = dx * (sy0 - py) + dy * (px - sy0) - (dy > 0 ? 1 : 0);
-        int q = floor_div(N0, D), rem = N0 - q * D;
-        const int qs = floor_div(128 * dx, D), rs = 128 * dx - qs * D;
-#pragma unroll
-        for (int r = 0; r < MW; r++) {
-            const int sy = sy0 + 128 * r;
-            const int b = dy > 0 ? q : -q - 1;  // last column left of the crossing
-            const uint32_t msk = b < 0 ? 0u : (b >= MW - 1 ? (MW == 32 ? ~0u : (1u << MW) - 1u) : (2u << b) - 1u);
-            if (sy >= ylo && sy < yhi) {
-                cov[r] ^= msk;
-                wsum += dy > 0 ? __builtin_popcount(msk) : -__builtin_popcount(msk);
+        const V B = P[stride * k];
+        int px = vert_x(A), py = vert_y(A), qx = vert_x(B), qy = vert_y(B);
+        A = B;
+        const int sign = py <= qy ? 1 : -1;  // the edge taken upward
+        if (sign < 0) {
+            swap2(&px, &qx);
+            swap2(&py, &qy);
+        }
+        px *= S2;
+        py *= S2;
+        const int dx = qx * S2 - px, dy = qy * S2 - py;
+        // rows sy with py <= sy < qy
+        int r = (py - s0 + 127) >> 7, end = (py + dy - s0 + 127) >> 7;
+        r = r < 0 ? 0 : r;
+        end = end > MW ? MW : end;
+        if (r >= end) continue;
+        const int D = 128 * dy;
+#ifdef __HIP_DEVICE_COMPILE__
+        const float inv = __builtin_amdgcn_rcpf((float)D);
+#else
+        const float inv = 1.0f / (float)D;
+#endif
+        // columns left of the crossing: 0 .. floor(N / D); an upward edge's
+        // covered side (N = e - 1 above 0) and a downward one's uncovered
+        // side end at the same column
+        int N = dx * (s0 + 128 * r - py) + dy * (px - s0) - 1;
+        for (; r < end; r++) {
+            int q = (int)floorf((float)N * inv);  // within 1 of the quotient
+            const int rem = N - q * D;
+            if (rem < 0) q--;
+            else if (rem >= D) q++;
+            const int cols = q < -1 ? 0 : q >= MW - 1 ? MW : q + 1;
+            if (cols > 0) {
+                toggle(r, cols >= 32 ? 0xFFFFFFFFu : (1u << cols) - 1u);
+                wsum += sign * cols;
             }
-            q += qs;
-            rem += rs;
-            if (rem >= D) {
-                rem -= D;
-                q++;
-            }
+            N += 128 * dx;
         }
     }
     return wsum;
+}
+
+template <int MW, class V>
+__host__ __device__ inline int poly_rows_xor(const V* P, int stride, int m, int S2, int kmin, uint32_t* cov)
+{
+    return poly_rows_cross<MW>(P, stride, m, S2, kmin, [&](int r, uint32_t mask) { cov[r] ^= mask; });
 }
 
 }  // namespace dpx

@@ -15,6 +15,7 @@
 #include "common.hpp"
 #include "geom.hpp"
 #include "graph.hpp"
+#include "hull_table.hpp"
 #include "pixel.hpp"
 
 namespace dpx {
@@ -85,22 +86,17 @@ __global__ void k_heuristic(uint8_t* __restrict__ graph, const uint8_t* __restri
     graph[idx] = (uint8_t)(c & ~heuristic_clear_mask(get, i, j, c, nb));
 }
 
-// The hulls of the 4096 cell keys (gen_hull_table.cpp): 32 KB, one word each.
-__device__ const uint64_t kHullTable[4096] = {
-#include "hull_table.inc"
-};
-
 // The kernels below write whole cells of 45 slots (360 bytes).  A thread
 // that writes its own cell's slots puts every lane of a store on a line of
 // its own, so the cells' values go to LDS first and a block then writes its
 // kRun cells as one contiguous range, adjacent lanes adjacent slots.
 constexpr int kRun = 64;
 
-__device__ inline dpx_point hull_point(uint64_t h, int t)
+__device__ inline dpx_point hull_point(HullBits h, int t)
 {
     dpx_point p;
-    p.x = 0.25f * (float)((int)((h >> (6 * t)) & 7u) - 1);
-    p.y = 0.25f * (float)((int)((h >> (6 * t + 3)) & 7u) - 1);
+    p.x = 0.25f * (float)hull_x(h, t);
+    p.y = 0.25f * (float)hull_y(h, t);
     return p;
 }
 
@@ -111,23 +107,23 @@ __device__ inline dpx_point hull_point(uint64_t h, int t)
 __global__ __launch_bounds__(256) void k_cells(const uint8_t* __restrict__ graph, size_t N,
                                                dpx_point* __restrict__ diagram, int32_t* __restrict__ edge_count)
 {
-    __shared__ uint64_t s_h[kRun];
+    __shared__ HullBits s_h[kRun];
     const size_t c0 = (size_t)blockIdx.x * kRun;
     const int t = threadIdx.x, cells = (int)(N - c0 < kRun ? N - c0 : kRun);
     if (t < cells) {
         const size_t idx = c0 + t;
         const uint32_t left = idx > 0 ? graph[idx - 1] : 0u;
         const uint32_t right = idx + 1 < N ? graph[idx + 1] : 0u;
-        const uint64_t h = kHullTable[cell_key(graph[idx], left, right)];
+        const HullBits h = kHullTable[cell_key(graph[idx], left, right)];
         s_h[t] = h;
-        edge_count[idx] = (int)(h >> 48);
+        edge_count[idx] = hull_count(h);
     }
     __syncthreads();
     dpx_point* d = diagram + c0 * kCellSize;
     for (int k = t; k < cells * kCellSize; k += 256) {
         const int c = k / kCellSize, q = k - c * kCellSize;
-        const uint64_t h = s_h[c];
-        const int n = (int)(h >> 48);
+        const HullBits h = s_h[c];
+        const int n = hull_count(h);
         dpx_point p = { 0.0f, 0.0f };
         if (q <= n) p = hull_point(h, q == n ? 0 : q);
         d[k] = p;
@@ -253,11 +249,11 @@ __global__ __launch_bounds__(256) void k_subdivide(ImgView im, const uint8_t* __
             if (any || s_n[own] == ANY) {
                 edge_count[idx] = subdivide_any(im, node, i, j, n, diagram, daux, eaux);
             } else {
-                struct HullX {
+                struct PointsX {
                     const uint32_t* p;
                     __device__ int operator[](int k) const { return point_x(p[k]); }
                 };
-                struct HullY {
+                struct PointsY {
                     const uint32_t* p;
                     __device__ int operator[](int k) const { return point_y(p[k]); }
                 };
@@ -266,11 +262,11 @@ __global__ __launch_bounds__(256) void k_subdivide(ImgView im, const uint8_t* __
                 auto nbr = [&](int e, auto f) {
                     const int c = own + edy(e) * CX + edx(e);
                     const uint32_t* q = s_hull + c * kSubPitch;
-                    return f(HullX{ q }, HullY{ q }, (int)s_n[c]);
+                    return f(PointsX{ q }, PointsY{ q }, (int)s_n[c]);
                 };
                 auto tj = [&](int x4, int y4) -> bool { return tj_kept(corners, x4, y4); };
                 int m = 0;
-                subdivide_cell_emit(HullX{ h }, HullY{ h }, n, node, nbr, tj, [&](int px, int py) {
+                subdivide_cell_emit(PointsX{ h }, PointsY{ h }, n, node, nbr, tj, [&](int px, int py) {
                     s_new[256 * m + t] = ((uint32_t)px & 0xFFFFu) | ((uint32_t)py << 16);
                     m++;
                 });
