@@ -559,18 +559,17 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     // resolved pixels of the first listed cells, so that every own
     // cell's rows are stored together (a line is then written by one store
     // instruction instead of being split between the direct and searched
-    // cells).  A pixel is kept as its colour; from S = 6 a tile whose listed
-    // cells would overflow that keeps the code of each pixel's winning
-    // candidate instead (1 byte: (1 - dy) * 3 + (1 - dx), 9 = clear colour),
-    // four times as many cells.  Measured: codes cost a decode per pixel, so
-    // tiles that fit keep colours; at S = 5 codes lose to the overflow stores.
-    constexpr bool CODES = S >= 6;
-    constexpr int PX_WORDS = 2048, PX_CELLS = PX_WORDS / (S * S), PX_CODE_CELLS = 4 * PX_WORDS / (S * S);
+    // cells).  A pixel is kept as its colour; from S = 5 a tile whose listed
+    // cells would overflow that keeps each row's winners instead (see
+    // Winners: one word a row up to 8x, where every cell of the tile fits,
+    // else two), and looks the colours up when it stores them.
+    constexpr bool CODES = S >= 5;
+    constexpr int ROW_WORDS = S <= 8 ? 1 : 2;  // of a row's packed winners
+    constexpr int PX_WORDS = 2048, PX_CELLS = PX_WORDS / (S * S), PX_CODE_CELLS = PX_WORDS / (S * ROW_WORDS);
     static_assert(PX_CELLS >= 1, "at least one buffered cell");
     __shared__ uint32_t s_px[PX_WORDS];
-    uint8_t* s_px8 = reinterpret_cast<uint8_t*>(s_px);
-    __shared__ uint16_t s_idx[RTX * RTY];    // list index of a listed own cell
-    __shared__ uint8_t s_simple[RTX * RTY];  // own cell shows its own colour only
+    __shared__ uint16_t s_idx[RTX * RTY];  // list index of a listed own cell, else kOwnColour
+    constexpr uint32_t kOwnColour = 0xFFFF;  // the cell shows its own colour only
     const uint8_t* s_g = reinterpret_cast<const uint8_t*>(s_g32);
 
     const int t = threadIdx.x;
@@ -695,21 +694,21 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     const bool mine = x0 + cx < it.W && y0 + cy < it.H;
     const bool simple = mine && simple_cell(s_info[kown], s_info[kown + RCX - 1], s_info[kown + RCX],
                                             s_info[kown + RCX + 1], s_info[kown + 1]);
-    if (mine && !simple) {
-        const int i = atomicAdd(&s_nlist, 1);
-        s_list[i] = (uint16_t)t;
+    {
+        uint32_t i = kOwnColour;
+        if (mine && !simple) {
+            i = (uint32_t)atomicAdd(&s_nlist, 1);
+            s_list[i] = (uint16_t)t;
+        }
         s_idx[t] = (uint16_t)i;
     }
-    s_simple[t] = simple ? 1 : 0;
     __syncthreads();
 
     // One unit = one output row (S pixels) of a listed cell, resolved
     // against the 3x3 candidates in draw order (highest cell index first).
     constexpr uint32_t FULL = (S >= 32) ? 0xFFFFFFFFu : ((1u << S) - 1u);
     const int nunits = s_nlist * S;
-    // uniform over the block; at 6x and 7x only tiles far beyond the colour
-    // buffer gain from codes (measured: sprites lose 5% at a threshold of 1x)
-    const bool codes = CODES && s_nlist > (S >= 8 ? 1 : 3) * PX_CELLS;
+    const bool codes = CODES && s_nlist > PX_CELLS;  // uniform over the block
     const int px_cells = codes ? PX_CODE_CELLS : PX_CELLS;
     auto fetch_rows = [&](int u, uint32_t* rows) {
         int own = s_list[u / S], ky = u % S;
@@ -738,65 +737,67 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
             }
         }
     };
+    // The winning candidate of every pixel of a row, as bit planes: pixel q's
+    // is the one at (1 - dx, 1 - dy) = (x0 + 2 x1, y0 + 2 y1) of bits q, or
+    // none (dx digit 3).  A candidate then costs three instructions for all
+    // of the row's pixels, and a pixel one product of four bits with their
+    // places in s_col, not a choice between nine colours: 170 -> 64
+    // instructions a row at 6x.
+    struct Winners {
+        uint32_t w[ROW_WORDS];
+    };
+    auto winners = [&](const uint32_t* rows) {
+        uint32_t seen = 0, won[9];
+#pragma unroll
+        for (int j = 0; j < 9; j++) {
+            const int sh = (j % 3 - 1) * S - KMIN;
+            const uint32_t bits = (sh >= 0 ? (rows[j] >> sh) : (rows[j] << -sh)) & FULL;
+            won[j] = bits & ~seen;
+            seen |= bits;
+        }
+        const uint32_t none = FULL & ~seen;
+        const uint32_t px0 = won[1] | won[4] | won[7] | none, px1 = won[2] | won[5] | won[8] | none;
+        const uint32_t py0 = won[3] | won[4] | won[5], py1 = won[6] | won[7] | won[8];
+        Winners r;
+        if constexpr (ROW_WORDS == 1) {
+            r.w[0] = px0 | px1 << 8 | py0 << 16 | py1 << 24;
+        } else {
+            r.w[0] = px0 | px1 << 16;
+            r.w[1] = py0 | py1 << 16;
+        }
+        return r;
+    };
+    // pixel q's colour; last: the cell's last candidate's place in s_col (dx = dy = 1)
+    auto winner_colour = [&](const Winners& r, int q, int last) -> uint32_t {
+        uint32_t off;
+        bool none;
+        if constexpr (ROW_WORDS == 1) {
+            const uint32_t bits = (r.w[0] >> q) & 0x01010101u;
+            off = __builtin_amdgcn_udot4(bits, 1u | 2u << 8 | (uint32_t)RCX << 16 | (uint32_t)(2 * RCX) << 24, 0u, false);
+            none = (bits & 0x0101u) == 0x0101u;
+        } else {
+            const uint32_t x = (r.w[0] >> q) & 0x00010001u, y = (r.w[1] >> q) & 0x00010001u;
+            off = (x & 3u) + (x >> 15) + (uint32_t)RCX * ((y & 3u) + (y >> 15));
+            none = x == 0x00010001u;
+        }
+        const uint32_t c = s_col[last - (int)off];
+        return none ? 0xFF000000u : c;
+    };
     auto resolve_unit = [&](int u, const uint32_t* rows) {
-        int own = s_list[u / S], ky = u % S;
-        int ux = own % RTX, uy = own / RTX;
-        uint32_t col[S];
+        const int own = s_list[u / S], ky = u % S;
+        const int ux = own % RTX, uy = own / RTX, last = (uy + 2) * RCX + ux + 2;
+        const Winners w = winners(rows);
         if constexpr (CODES) {
-            if (codes) {  // the same search, keeping candidate codes
-                uint8_t code[S];
+            if (codes && u / S < PX_CODE_CELLS) {
 #pragma unroll
-                for (int q = 0; q < S; q++) code[q] = 9;
-                uint32_t assigned = 0;
-#pragma unroll
-                for (int dy = 1; dy >= -1; dy--) {
-#pragma unroll
-                    for (int dx = 1; dx >= -1; dx--) {
-                        uint32_t row = rows[(1 - dy) * 3 + (1 - dx)];
-                        int sh = -dx * S - KMIN;
-                        uint32_t nb = (sh >= 0 ? (row >> sh) : (row << -sh)) & FULL & ~assigned;
-                        if (nb) {
-#pragma unroll
-                            for (int q = 0; q < S; q++)
-                                if ((nb >> q) & 1u) code[q] = (uint8_t)((1 - dy) * 3 + (1 - dx));
-                            assigned |= nb;
-                        }
-                    }
-                }
-                if (u / S < PX_CODE_CELLS) {
-#pragma unroll
-                    for (int q = 0; q < S; q++) s_px8[u * S + q] = code[q];
-                } else {
-#pragma unroll
-                    for (int q = 0; q < S; q++)
-                        col[q] = code[q] == 9 ? 0xFF000000u
-                                              : s_col[(uy + 2 - code[q] / 3) * RCX + (ux + 2 - code[q] % 3)];
-                    store_row(x0 + ux, (y0 + uy) * S + ky, col);  // beyond the buffer: written directly
-                }
+                for (int k = 0; k < ROW_WORDS; k++) s_px[u * ROW_WORDS + k] = w.w[k];
                 return;
             }
         }
+        uint32_t col[S];
 #pragma unroll
-        for (int q = 0; q < S; q++) col[q] = 0xFF000000u;
-        uint32_t assigned = 0;
-#pragma unroll
-        for (int dy = 1; dy >= -1; dy--) {
-#pragma unroll
-            for (int dx = 1; dx >= -1; dx--) {
-                uint32_t row = rows[(1 - dy) * 3 + (1 - dx)];
-                int sh = -dx * S - KMIN;
-                uint32_t bits = (sh >= 0 ? (row >> sh) : (row << -sh)) & FULL;
-                uint32_t nb = bits & ~assigned;
-                if (nb) {
-                    uint32_t c = s_col[(uy + 1 + dy) * RCX + (ux + 1 + dx)];
-#pragma unroll
-                    for (int q = 0; q < S; q++)
-                        if ((nb >> q) & 1u) col[q] = c;
-                    assigned |= nb;
-                }
-            }
-        }
-        if (u / S < PX_CELLS) {
+        for (int q = 0; q < S; q++) col[q] = winner_colour(w, q, last);
+        if (!codes && u / S < PX_CELLS) {
 #pragma unroll
             for (int q = 0; q < S; q++) s_px[u * S + q] = col[q];
         } else {
@@ -856,118 +857,113 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     // of a wave store adjacent cells, so each thread stores its own cell.  At
     // the other scales that would make every store instruction strided (S * 4
     // bytes between lanes, each line written in pieces by several
-    // instructions), so the tile's output is stored in chunks of CW pixels
-    // inside one cell, chunk c by thread c % 256: adjacent lanes store
-    // adjacent chunks of a row.  Searched cells beyond the pixel buffer were
-    // stored by the search itself; their chunks are skipped.  Measured: at 5x
-    // to 7x, with chunks of fewer than 4 pixels, the chunk loop's own work
-    // outweighs the coalescing once a tile's cells overflow the colour buffer
-    // (dense frames, sprites), so such tiles keep the per-cell stores; at 8x
-    // and from 9x up (rows of 36 bytes and more) chunks win on every tile.
+    // instructions), so the tile's rows are stored in chunks, adjacent lanes
+    // adjacent chunks: of 4 pixels (16 bytes) where the rows are so aligned,
+    // else of CW pixels inside one cell.  A thread goes from chunk to chunk
+    // by 256, which moves it dr rows and dj chunks on (one row more where
+    // that passes the row's end): the tile's cells in the frame, whatever
+    // their number, keep every lane busy, and a chunk's cell and pixel take
+    // two small products.  Searched cells beyond the pixel buffer were stored
+    // by the search itself; their chunks are skipped, or where a chunk may
+    // span two cells such tiles keep the per-cell stores (so do tiles at 5x
+    // to 7x whose rows allow only chunks of one or two pixels and whose cells
+    // overflow the buffer: there the chunks' own work outweighs the
+    // coalescing).  With the winners above, per batch: 16 640x480 frames at 8x
+    // 339 -> 259 us, 4096 sprites at 6x 164 -> 142, 64 console frames at 6x
+    // 207 -> 151, at 12x 726 -> 570; chunks read two and four at a time
+    // measured the same.
     constexpr int CW = (S % 4 == 0) ? 4 : ((S % 2 == 0) ? 2 : 1);
     // pixel (kx, ky) of listed cell i, own cell (lx, ly), from the buffer;
-    // use_codes (std::true_type: the tile keeps candidate codes) is fixed per
+    // use_codes (std::true_type: the tile keeps rows' winners) is fixed per
     // tile, outside the store loops
     auto buffered = [&](auto use_codes, int i, int kx, int ky, int lx, int ly) -> uint32_t {
         if constexpr (decltype(use_codes)::value) {
-            const int code = s_px8[(i * S + ky) * S + kx];
-            return code == 9 ? 0xFF000000u : s_col[(ly + 2 - code / 3) * RCX + (lx + 2 - code % 3)];
+            Winners r;
+#pragma unroll
+            for (int k = 0; k < ROW_WORDS; k++) r.w[k] = s_px[(i * S + ky) * ROW_WORDS + k];
+            return winner_colour(r, kx, (ly + 2) * RCX + lx + 2);
         } else {
             return s_px[(i * S + ky) * S + kx];
         }
     };
     bool chunked = false, wide = false;
     if constexpr (S != 1 && S != 2 && S != 4) {
-        const uintptr_t base = reinterpret_cast<uintptr_t>(out + it.out_off);
-        chunked = ((base | (uintptr_t)it.out_stride) & (4 * CW - 1)) == 0 &&
-                  (CW == 4 || S >= 9 || s_nlist <= PX_CELLS);
-        // odd scales: chunks of 4 pixels across cell boundaries when the rows
-        // are 16-byte aligned and every listed cell is buffered (no pixel of
-        // the tile was stored by the search)
-        if constexpr (CW == 1) wide = ((base | (uintptr_t)it.out_stride) & 15) == 0 && s_nlist <= px_cells;
+        const uintptr_t align = reinterpret_cast<uintptr_t>(out + it.out_off) | (uintptr_t)it.out_stride;
+        wide = (align & 15) == 0 && (S % 4 == 0 || s_nlist <= px_cells);
+        chunked = (align & (4 * CW - 1)) == 0 && (CW == 4 || S >= 9 || s_nlist <= px_cells);
     }
-    // Chunks of 4 pixels of a tile row (16-byte stores) that may span two
-    // cells (S >= 3): each pixel takes its colour from its own cell, simple
-    // or buffered.  Measured against one-pixel chunks: 3x 14% and 5x 24%
-    // faster (7x: 8% before the path for two simple cells); against the
-    // two-pixel chunks of 6x, 6-12% slower (the per-pixel lookups cost more
-    // than the wider stores save).
-    auto store_wide = [&](auto use_codes) {
-        constexpr int CPR = RTX * S / 4;   // chunks per output row of the tile
-        constexpr int NCH = RTY * S * CPR;
-        static_assert(RTX * S % 4 == 0, "whole chunks per tile row");
-        const int ncx = min(RTX, it.W - x0), rowpx = ncx * S;  // cells and pixels of a tile row in the frame
-        for (int c = t; c < NCH; c += 256) {
-            const int ry = c / CPR, px0 = 4 * (c % CPR);
-            const int ly = ry / S, ky = ry % S;
-            if (px0 >= rowpx || y0 + ly >= it.H) continue;
-            // the chunk's cells; past the frame's last column the pixels are
-            // not stored and take that column's cell
-            const int la = px0 / S, lb = min((px0 + 3) / S, ncx - 1);
-            const int oa = ly * RTX + la, ob = ly * RTX + lb;
-            const bool sa = s_simple[oa], sb = s_simple[ob];
-            const int ia = sa ? 0 : s_idx[oa], ib = sb ? 0 : s_idx[ob];  // simple: entry 0, ignored
-            const uint32_t va = s_col[(ly + 1) * RCX + la + 1], vb = s_col[(ly + 1) * RCX + lb + 1];
-            uint32_t col[4];
-            if (sa && sb) {  // both cells simple (most chunks): no buffer reads
+    // floor(v / S) for v < 2^12 (an exact reciprocal to 16 bits suffices)
+    auto over_s = [](int v) { return (int)(__umul24((unsigned)v, 65536u / S + 1u) >> 16); };
+    auto store_chunks = [&](auto use_codes, auto width) {
+        constexpr int N = decltype(width)::value;  // pixels of a chunk
+        const int ncx = min(RTX, it.W - x0), rows = min(RTY, it.H - y0) * S, rowpx = ncx * S;
+        const int cpr = (rowpx + N - 1) / N;  // chunks of a row
+        // (quotients below 2^9 from a reciprocal, half a unit clear of the next)
+        const float inv = __builtin_amdgcn_rcpf((float)cpr);
+        const int dr = (int)(256.5f * inv), dj = 256 - dr * cpr;
+        int row = (int)(((float)t + 0.5f) * inv), j = t - row * cpr;
+        const bool down = out_topdown(it.flags);
+        const ptrdiff_t pitch = down ? -(ptrdiff_t)it.out_stride : (ptrdiff_t)it.out_stride;
+        uint8_t* dst = out + it.out_off + (size_t)(down ? OH - 1 - y0 * S : y0 * S) * it.out_stride +
+                       (size_t)x0 * S * 4 + row * pitch + j * (4 * N);
+        const ptrdiff_t step = dr * pitch + dj * (4 * N), wrap = pitch - cpr * (4 * N);
+        while (row < rows) {
+            const int px0 = N * j, la = over_s(px0), kx = px0 - la * S, ly = over_s(row), ky = row - ly * S;
+            const uint32_t ia = s_idx[ly * RTX + la], va = s_col[(ly + 1) * RCX + la + 1];
+            uint32_t col[N];
+            bool stored = false;  // by the search
+            if constexpr (S % N == 0) {  // one cell
 #pragma unroll
-                for (int q = 0; q < 4; q++) col[q] = px0 + q >= (la + 1) * S ? vb : va;
+                for (int q = 0; q < N; q++) col[q] = va;
+                if (ia != kOwnColour) {
+                    stored = (int)ia >= px_cells;
+                    if (!stored) {
+#pragma unroll
+                        for (int q = 0; q < N; q++) col[q] = buffered(use_codes, (int)ia, kx + q, ky, la, ly);
+                    }
+                }
             } else {
+                // the chunk's second cell; past the frame's last column the
+                // pixels are not stored and take that column's cell
+                const int lb = min(la + 1, ncx - 1), split = S - kx;
+                const uint32_t ib = s_idx[ly * RTX + lb], vb = s_col[(ly + 1) * RCX + lb + 1];
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int p = px0 + q;
-                    const bool inb = p >= (la + 1) * S;  // pixel in the second cell
-                    const int lx = inb ? lb : la, i = inb ? ib : ia;
-                    const int kx = min(p - lx * S, S - 1);  // (past the frame: not stored)
-                    const uint32_t bv = buffered(use_codes, i, kx, ky, lx, ly);
-                    col[q] = (inb ? sb : sa) ? (inb ? vb : va) : bv;
+                for (int q = 0; q < N; q++) col[q] = q >= split ? vb : va;
+                if (ia != kOwnColour || ib != kOwnColour) {
+#pragma unroll
+                    for (int q = 0; q < N; q++) {
+                        const bool inb = q >= split;
+                        const uint32_t i = inb ? ib : ia;
+                        if (i != kOwnColour)
+                            col[q] = buffered(use_codes, (int)i, inb ? q - split : kx + q, ky, inb ? lb : la, ly);
+                    }
                 }
             }
-            const int Y = (y0 + ly) * S + ky;
-            const int row = out_topdown(it.flags) ? (OH - 1 - Y) : Y;
-            uint8_t* dst = out + it.out_off + (size_t)row * it.out_stride + ((size_t)x0 * S + px0) * 4;
-            if (px0 + 3 < rowpx) {
-                u32x4 v = { col[0], col[1], col[2], col[3] };
-                __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));
-            } else {
+            if (!stored) {
+                if constexpr (N == 4) {
+                    if (S % 4 == 0 || px0 + 3 < rowpx) {
+                        u32x4 v = { col[0], col[1], col[2], col[3] };
+                        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));
+                    } else {
 #pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (px0 + q < rowpx) __builtin_nontemporal_store(col[q], reinterpret_cast<uint32_t*>(dst + 4 * q));
+                        for (int q = 0; q < 4; q++)
+                            if (px0 + q < rowpx)
+                                __builtin_nontemporal_store(col[q], reinterpret_cast<uint32_t*>(dst + 4 * q));
+                    }
+                } else if constexpr (N == 2) {
+                    u32x2 v = { col[0], col[1] };
+                    __builtin_nontemporal_store(v, reinterpret_cast<u32x2*>(dst));
+                } else {
+                    __builtin_nontemporal_store(col[0], reinterpret_cast<uint32_t*>(dst));
+                }
             }
-        }
-    };
-    auto store_chunks = [&](auto use_codes) {
-        constexpr int CPC = S / CW;          // chunks per cell row
-        constexpr int CPR = RTX * CPC;       // chunks per output row of the tile
-        constexpr int NCH = RTY * S * CPR;   // chunks of the tile
-        for (int c = t; c < NCH; c += 256) {
-            const int ry = c / CPR, rc = c % CPR;
-            const int lx = rc / CPC, kx = (rc % CPC) * CW;
-            const int ly = ry / S, ky = ry % S;
-            if (x0 + lx >= it.W || y0 + ly >= it.H) continue;
-            const int own = ly * RTX + lx;
-            uint32_t col[CW];
-            if (s_simple[own]) {
-                const uint32_t v = s_col[(ly + 1) * RCX + lx + 1];
-#pragma unroll
-                for (int q = 0; q < CW; q++) col[q] = v;
-            } else {
-                const int i = s_idx[own];
-                if (i >= px_cells) continue;  // stored by the search
-#pragma unroll
-                for (int q = 0; q < CW; q++) col[q] = buffered(use_codes, i, kx + q, ky, lx, ly);
-            }
-            const int Y = (y0 + ly) * S + ky;
-            const int row = out_topdown(it.flags) ? (OH - 1 - Y) : Y;
-            uint8_t* dst = out + it.out_off + (size_t)row * it.out_stride + ((size_t)(x0 + lx) * S + kx) * 4;
-            if constexpr (CW == 4) {
-                u32x4 v = { col[0], col[1], col[2], col[3] };
-                __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));
-            } else if constexpr (CW == 2) {
-                u32x2 v = { col[0], col[1] };
-                __builtin_nontemporal_store(v, reinterpret_cast<u32x2*>(dst));
-            } else {
-                __builtin_nontemporal_store(col[0], reinterpret_cast<uint32_t*>(dst));
+            row += dr;
+            j += dj;
+            dst += step;
+            if (j >= cpr) {
+                j -= cpr;
+                row++;
+                dst += wrap;
             }
         }
     };
@@ -988,25 +984,21 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
             store_row(x0 + cx, (y0 + cy) * S + ky, col);
         }
     };
-    if (wide) {
-        if constexpr (CODES) {
-            if (codes) {
-                store_wide(std::true_type{});
-                return;
+    if constexpr (S != 1 && S != 2 && S != 4) {
+        using Wide = std::integral_constant<int, 4>;
+        using Narrow = std::integral_constant<int, CW>;
+        if (wide || chunked) {
+            if constexpr (CODES) {
+                if (codes) {
+                    if (wide) store_chunks(std::true_type{}, Wide{});
+                    else store_chunks(std::true_type{}, Narrow{});
+                    return;
+                }
             }
+            if (wide) store_chunks(std::false_type{}, Wide{});
+            else store_chunks(std::false_type{}, Narrow{});
+            return;
         }
-        store_wide(std::false_type{});
-        return;
-    }
-    if (chunked) {
-        if constexpr (CODES) {
-            if (codes) {
-                store_chunks(std::true_type{});
-                return;
-            }
-        }
-        store_chunks(std::false_type{});
-        return;
     }
     if (mine) {
         const int i = simple ? 0 : s_idx[t];  // a simple cell reads entry 0 and ignores it
