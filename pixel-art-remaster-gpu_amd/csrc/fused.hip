@@ -1,7 +1,7 @@
 // fused.hip -- the batched path: many frames or sprites of uneven size
 // through two fused kernels.
 //
-//   kf_graph   tile of 64x32 pixels (64x8 in small launches): lane words (YUV fields + class) once
+//   kf_graph   strip of 64 columns of a row block, one wave: lane words (YUV fields + class) once
 //              per pixel, similarity in four directions (the other four by
 //              symmetry) with block flags for the trivial crossing removal
 //              -> snapshot graph (1 B/px)
@@ -116,169 +116,358 @@ __global__ void kt_info(const uint32_t* __restrict__ mask, int S, uint16_t* __re
 
 
 // ---------------------------------------------------------------------------
-// ---------------------------------------------------------------------------
 // kf_graph: similarity graph + trivial crossing removal
 // ---------------------------------------------------------------------------
-// Three passes over LDS:
-//   1. lane words (pixel class + YUV fields, see lane_ref) of the tile and a
-//      halo: x0-1 .. x0+65, y0-2 .. y0+33;
-//   2. per position of x0-1 .. x0+64, y0-1 .. y0+32, the four edges it owns
-//      (up, up-right, right, down-right: bits 1, 2, 4, 7; similarity is
-//      symmetric, so each edge is tested once);
-//   3. per four pixels of a row at once (one byte each in a 32-bit word):
-//      the other four edges from the left, down, down-left and up-left
-//      neighbours' bytes, and the trivial removal: a 2x2 block is "full"
-//      (all four orthogonal edges, crossCheck_4's condition for removing
-//      both diagonals) iff its lower-left position has its up and right
-//      edges, the position above it its right edge and the position right
-//      of it its up edge; the flags of the four blocks around a pixel come
-//      from those bits of the neighbouring bytes.
-// Tiles are GTX x TY pixels: TY = GTY or kGraphTallTY, whichever converts
-// fewer rows (tiles x (TY + 4): 56 for 224-row frames, 4 tiles of 60 rows
-// against 7 of 36, 6% faster), or kGraphSmallTY for launches that would have
-// fewer than kGraphSmallTiles blocks of GTY rows (a launch of a few frames
-// then spreads over more CUs; the extra halo rows cost throughput only in
-// launches that fill the machine).
-constexpr int GTX = 64, GTY = 32, kGraphSmallTY = 8, kGraphTallTY = 56;
-constexpr uint64_t kGraphSmallTiles = 512;
-constexpr int GLX = GTX + 3;  // lane words per row
-constexpr int GHX = GTX + 2;  // positions of pass 2 per row
-constexpr int GHP = GTX + 8;  // byte pitch of pass 2's rows: column c is x = x0 - 4 + c
+// One wave marches down the rows of a strip of 64 columns, one column per
+// lane, with the lane word (pixel class + YUV fields, see lane_ref) of the
+// row above in a register and no LDS, barrier or second pass:
+//   * a similarity test is two subtractions, one three-input logic operation
+//     and a compare; the right neighbours' words come through the DPP shift
+//     of the subtraction itself.  Each pixel tests the four edges it owns
+//     (up, up-right, right, down-right: similarity is symmetric);
+//   * a compare leaves its 64 answers as one bit each in a scalar register
+//     pair, so the other four edges (the neighbours' own, one bit further
+//     left or one row down) and the trivial removal (a 2x2 block with all
+//     four orthogonal edges loses both diagonals, crossCheck_4) are scalar
+//     64-bit operations on whole rows, issued beside other waves' vector work;
+//   * the eight bits of a pixel's byte are shifted in by add-with-carry, a
+//     row mask as the carries.
+// The kernel is bound by vector issue (its bytes would take a quarter of its
+// time), so what counts is instructions a pixel: 46 against the 95 of 64-wide
+// tiles whose lane words and bytes went through LDS.  1024 frames of 256x224:
+// 169 -> 105 us, 82% of the vector issue rate; 16 of 640x480: 23 -> 15.6 us;
+// 4096 sprites of 8 to 64 pixels: 28 -> 17 us (their tiles were half empty).
+//
+// A strip's outer two lanes are its halo, so a strip yields 62 columns.  62
+// does not divide the widths of frames, so strips do not start over at a
+// frame's edge: an item's rows are cut into blocks of equal height, laid side
+// by side with one empty column before each, and the strips are cut from that
+// row of columns; a strip that holds the end of one block and the start of
+// the next works on both (lanes are independent but for the shift, and the
+// empty column belongs to the outside class).  256x224 in 4 blocks: 17
+// strips, 16.6 of them used.
+// Pixels are loaded kGraphRows rows at a time, one such group ahead (two
+// groups ahead: 109 -> 113 us, for the registers' copies).
+constexpr int kStripCols = 62;
+constexpr int kGraphRows = 4;
+// Rows of a launch's row blocks.  A wave alone takes 0.25 us a row, and each
+// block re-reads two halo rows, so blocks are as tall as leaves about
+// kGraphWaves strips, five waves a SIMD: measured at 2 / 6 / 14 / 30 / 56
+// rows, one 256x224 frame takes 3.7 / 4.7 / 6.0 / 9.2 / 15.1 us, 64 console
+// frames (4.2 Mpixel) 22 / 15.1 / 13.8 / 15.8 / 19.8, 128 of 320x224 59 / 31
+// / 22.6 / 21.1 / 22.9 and 1024 of 256x224 274 / 162 / 119 / 116 / 105.
+// Heights of 4 k + 2 make whole groups with the halo.
+constexpr uint64_t kGraphWaves = 4800;
+constexpr int kGraphMinRows = 2, kGraphMaxRows = 58;
 
-template <int TY>
-__global__ __launch_bounds__(256) void kf_graph(const DevItem* __restrict__ items, const uint2* __restrict__ tile_map,
-                                                int grid3d, const uint8_t* __restrict__ in,
-                                                uint8_t* __restrict__ gaux)
+inline int graph_rows(uint64_t pixels)
 {
-    constexpr int GLY = TY + 4, GHY = TY + 2;  // rows of lane words and of pass 2's positions
-    static_assert(GLY * (GLX - 64) <= 256 && GHY * (GHX - 64) <= 256, "the columns past 64 take one pass");
-    __shared__ uint32_t s_lane[GLX * GLY];
-    // pass 2's rows; first, for indexed items, the 256 palette lane words
-    __shared__ uint32_t s_h32[GHY * GHP / 4 > 256 ? GHY * GHP / 4 : 256];
-    uint8_t* s_h = reinterpret_cast<uint8_t*>(s_h32);
-    const int t = threadIdx.x;
-    // runs of 8 tiles per XCD: the lines that neighbouring tiles' rows share
-    // (a 64-pixel row of 3-byte pixels and its halo span 2-3 lines of 128
-    // bytes) are fetched once into one L2 (HBM reads 365 -> 183 MB for 1024
-    // frames of 256x224, 1.04x the input; the kernel's time is its VALU work)
-    const TileAt at = locate_tile<8>(tile_map, grid3d);
-    const DevItem it = items[at.item];
-    const int x0 = at.tx * GTX, y0 = at.ty * TY;
+    const int rows = (int)std::min<uint64_t>(pixels / (kStripCols * kGraphWaves), kGraphMaxRows);
+    return std::max((rows + 2) / kGraphRows * kGraphRows - 2, kGraphMinRows);
+}
 
-    // pass 1.  Byte offsets within an item fit 31 bits (checked on the host).
-    const uint8_t* base = in + it.in_off;
-    const bool rgb = it.flags & DPX_RGB, topdown = it.flags & DPX_TOPDOWN;
-    const bool indexed = it.flags & DPX_INDEXED;
-    const bool alpha = (it.flags & DPX_ALPHA) && it.ch == 4;
-    const uint32_t o0 = rgb ? 2 : 0, o2 = 2 - o0;
-    if (indexed) {
-        // the lane words of the 256 palette entries, in pass 2's rows until
-        // pass 2 writes them
-        const uint32_t e = reinterpret_cast<const uint32_t*>(in + it.pal_off)[t];
-        const int c0 = (e >> (8 * o0)) & 0xFF, c1 = (e >> 8) & 0xFF, c2 = (e >> (8 * o2)) & 0xFF;
-        uint32_t lw = yuv_lanes(yuv_pack(c0, c1, c2)) | kLaneOpaque;
-        if ((it.flags & DPX_ALPHA) && (e >> 24) == 0) lw = kLaneTransparent;
-        s_h32[t] = lw;
-        __syncthreads();
-    }
-    // Lane word of pixel (x, y) at byte offset `off` of the item's buffer:
-    // one 4-byte load (any alignment) where the 4 bytes lie inside the
-    // item's rows, else byte loads (the last pixel of the last row in
-    // memory of a 3-channel frame without row padding).
-    const uint32_t in_end = (uint32_t)(it.H - 1) * (uint32_t)it.stride + (uint32_t)(it.W * it.ch);
-    auto lane_word = [&](uint32_t off) -> uint32_t {
-        if (indexed) return s_h32[base[off]];
-        uint32_t w;
-        if (off + 4u <= in_end)
-            __builtin_memcpy(&w, base + off, 4);
-        else
-            w = base[off] | (uint32_t)base[off + 1] << 8 | (uint32_t)base[off + 2] << 16 |
-                (it.ch == 4 ? (uint32_t)base[off + 3] << 24 : 0u);
-        const int c0 = (w >> (8 * o0)) & 0xFF, c1 = (w >> 8) & 0xFF, c2 = (w >> (8 * o2)) & 0xFF;
-        if (alpha && (w >> 24) == 0) return kLaneTransparent;
-        return yuv_lanes(yuv_pack(c0, c1, c2)) | kLaneOpaque;
-    };
-    // Window column c (x = x0 - 1 + c), row r (y = y0 - 2 + r).  Columns
-    // 0..63: one per thread (t % 64), every fourth row from t / 64, the byte
-    // offset stepping by four rows; columns 64..GLX-1: one word per thread.
-    // (Reading aligned rows as groups of four pixels, dwordx3 per thread and
-    // four conversions each, measured slower: 0.153 -> 0.160-0.173 ms.)
-    {
-        const int c = t & 63, x = x0 - 1 + c;
-        const bool xin = (unsigned)x < (unsigned)it.W;
-        int y = y0 - 2 + (t >> 6);
-        // modulo 2^32 (rows outside the frame may lie outside int); used only inside the frame
-        uint32_t off = (uint32_t)(topdown ? it.H - 1 - y : y) * (uint32_t)it.stride + (uint32_t)(x * it.ch);
-        const uint32_t step = (uint32_t)((topdown ? -4 : 4) * it.stride);
-        for (int r = t >> 6; r < GLY; r += 4, y += 4, off += step) {
-            uint32_t lw = 0;
-            if (xin && (unsigned)y < (unsigned)it.H) lw = lane_word(off);
-            s_lane[r * GLX + c] = lw;
+struct GraphSplit {
+    uint32_t blocks, rows, strips;
+};
+
+__host__ __device__ inline GraphSplit graph_split(int W, int H, int max_rows)
+{
+    GraphSplit s;
+    s.blocks = ((uint32_t)H + (uint32_t)max_rows - 1) / (uint32_t)max_rows;
+    s.rows = ((uint32_t)H + s.blocks - 1) / s.blocks;
+    s.blocks = ((uint32_t)H + s.rows - 1) / s.rows;  // (blocks of s.rows rows that hold a row)
+    // columns 1 .. blocks * (W + 1) - 1 of the row of blocks carry pixels
+    s.strips = (s.blocks * ((uint32_t)W + 1) - 1 + kStripCols - 1) / kStripCols;
+    return s;
+}
+
+// One more bit of each lane's byte: v + v + (the lane's bit of m).  m is the
+// result of a scalar operation: a vector compare's result would have to be
+// two wait states old, and the compiler does not look into the block for it.
+__device__ inline void shift_in(uint32_t& v, uint64_t m)
+{
+    uint64_t c;
+    asm("v_addc_co_u32_e64 %0, %1, %0, %0, %2" : "+v"(v), "=s"(c) : "s"(m));
+}
+
+// Two lane words a, b are similar iff bit 8 of each 10-bit lane of a - b + t
+// + 256 and of b - a + t + 256 is set (a lane holds 6 .. 518, so none borrows
+// or carries; with d the fields' difference, bit 8 of the first is set iff -t
+// <= d <= 255 - t) and the classes are equal, which leaves 3 in the class bits
+// of both.
+constexpr uint32_t kSimilarBias = 3u << 30 | (256u + 5) << 20 | (256u + 7) << 10 | (256u + 6);
+constexpr uint32_t kSimilarTest = 3u << 30 | 1u << 28 | 1u << 18 | 1u << 8;
+
+// A row of lane words as the tests take it: l, l + bias and bias - l.
+struct LaneRow {
+    uint32_t l, plus, minus;
+};
+
+// The edges between row a and row b above it: a's up and up-right edges, b's
+// right and down-right ones (the lane's pixel as their left end).  One block,
+// so that the neighbour's word comes by the DPP shift of the subtraction
+// itself (left to the compiler, a shifted word with two uses is moved first)
+// and no shifted operand was written less than two instructions before.  The
+// shifted operand is an addend or the minuend: a reversed subtraction
+// (v_subrev) with a shift shifts its minuend.
+struct RowEdges {
+    uint64_t up, up_right, right, down_right;
+};
+
+__device__ inline RowEdges row_edges(const LaneRow& a, LaneRow& b)
+{
+    RowEdges e;
+    uint32_t u, v, r0, r1, x, y, d0, d1;
+#define DPX_RIGHT " wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+    asm("v_add_u32_e32 %[bp], %[bias], %[b]\n\t"
+        "v_sub_u32_e32 %[bm], %[bias], %[b]\n\t"
+        "v_sub_u32_e32 %[u], %[ap], %[b]\n\t"
+        "v_sub_u32_e32 %[v], %[bp], %[a]\n\t"
+        "v_add_u32_dpp %[d0], %[am], %[b]" DPX_RIGHT
+        "v_sub_u32_dpp %[d1], %[ap], %[b]" DPX_RIGHT
+        "v_add_u32_dpp %[r0], %[bm], %[b]" DPX_RIGHT
+        "v_sub_u32_dpp %[r1], %[bp], %[b]" DPX_RIGHT
+        "v_add_u32_dpp %[x], %[bm], %[a]" DPX_RIGHT
+        "v_sub_u32_dpp %[y], %[bp], %[a]" DPX_RIGHT
+        "v_bitop3_b32 %[u], %[u], %[test], %[v] bitop3:0x80\n\t"
+        "v_bitop3_b32 %[d0], %[d0], %[test], %[d1] bitop3:0x80\n\t"
+        "v_bitop3_b32 %[r0], %[r0], %[test], %[r1] bitop3:0x80\n\t"
+        "v_bitop3_b32 %[x], %[x], %[test], %[y] bitop3:0x80\n\t"
+        "v_cmp_eq_u32_e64 %[eu], %[test], %[u]\n\t"
+        "v_cmp_eq_u32_e64 %[ed], %[test], %[d0]\n\t"
+        "v_cmp_eq_u32_e64 %[er], %[test], %[r0]\n\t"
+        "v_cmp_eq_u32_e64 %[ex], %[test], %[x]"
+        : [bp] "=&v"(b.plus), [bm] "=&v"(b.minus), [u] "=&v"(u), [v] "=&v"(v), [d0] "=&v"(d0), [d1] "=&v"(d1),
+          [r0] "=&v"(r0), [r1] "=&v"(r1), [x] "=&v"(x), [y] "=&v"(y), [eu] "=&s"(e.up), [ed] "=&s"(e.down_right),
+          [er] "=&s"(e.right), [ex] "=&s"(e.up_right)
+        : [a] "v"(a.l), [ap] "v"(a.plus), [am] "v"(a.minus), [b] "v"(b.l), [bias] "s"(kSimilarBias),
+          [test] "s"(kSimilarTest));
+#undef DPX_RIGHT
+    return e;
+}
+
+__device__ inline bool lane_of(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
+// How pixels become lane words.
+enum GraphPixels {
+    kPixelsPlain,    // 3 or 4 bytes, blue first, no alpha test
+    kPixelsGeneral,  // either order, alpha test
+    kPixelsIndexed,  // one byte, the palette's lane words in LDS
+};
+
+template <int PIXELS>
+__device__ __forceinline__ void graph_strip(const DevItem& it, const GraphSplit sp, uint32_t strip,
+                                            const uint8_t* __restrict__ in, const uint32_t* s_pal,
+                                            uint8_t* __restrict__ gaux)
+{
+    constexpr int G = kGraphRows;
+    const uint32_t lane = threadIdx.x;
+    const bool topdown = it.flags & DPX_TOPDOWN;
+    const int W = it.W, H = it.H;
+    // the lane's column: block and x (-1: the empty column before a block);
+    // lanes past the last block stand on its last column and are not stored
+    const uint32_t p = strip * kStripCols + lane;
+    const uint32_t blk = p / ((uint32_t)W + 1);
+    const bool col = blk < sp.blocks && p % ((uint32_t)W + 1) != 0;
+    const uint32_t b = min(blk, sp.blocks - 1);
+    const int x = col ? (int)(p % ((uint32_t)W + 1)) - 1 : (blk < sp.blocks ? 0 : W - 1);
+    const int y0 = (int)(b * sp.rows);
+    const uint64_t cols = __builtin_amdgcn_ballot_w64(col);
+    const uint64_t mine = cols & 0x7FFFFFFFFFFFFFFEull;  // the columns stored by this strip
+    const int y0_first = __builtin_amdgcn_readlane(y0, 0), y0_last = __builtin_amdgcn_readlane(y0, 63);
+    const int R = (int)sp.rows + 2;  // row r is y = y0 - 1 + r
+
+    // Pixels are read through a buffer descriptor of the item's rows, which
+    // answers 0 past its end (rows above or below the frame).  Row r of a lane
+    // lies at voff + (r - 1) * step modulo 2^32; byte offsets within an item
+    // fit 31 bits (checked on the host).  Rows r_lo .. r_hi - 1 lie in the
+    // frame for every lane.  The last pixel of a frame of 3-byte pixels is
+    // read by bytes (`tail`: the strip holds it): its 4-byte word would end
+    // past the frame.
+    const uint32_t step = (uint32_t)(topdown ? -it.stride : it.stride);
+    const uint32_t voff = (uint32_t)(topdown ? H - 1 - y0 : y0) * (uint32_t)it.stride + (uint32_t)(x * it.ch);
+    const uint32_t in_end = (uint32_t)(H - 1) * (uint32_t)it.stride + (uint32_t)(W * it.ch);
+    const auto src = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(in + it.in_off), 0, in_end, 0x00020000);
+    const int r_lo = 1 - y0_first, r_hi = H + 1 - y0_last;
+    const bool tail = PIXELS != kPixelsIndexed && it.ch < 4 &&
+                      __builtin_amdgcn_ballot_w64(x == W - 1 && (topdown ? y0 <= 1 : y0 + (int)sp.rows >= H - 1)) != 0;
+
+    uint32_t px[G];
+    auto fetch = [&](int r0) {
+        uint32_t o = voff + (uint32_t)(r0 - 1) * step;
+#pragma unroll
+        for (int q = 0; q < G; q++) {
+            if constexpr (PIXELS == kPixelsIndexed)
+                px[q] = __builtin_amdgcn_raw_buffer_load_b8(src, (int)o, 0, 0);
+            else
+                px[q] = __builtin_amdgcn_raw_buffer_load_b32(src, (int)o, 0, 0);
+            o += step;
         }
-    }
-    if (t < (GLX - 64) * GLY) {
-        const int c = 64 + t % (GLX - 64), r = t / (GLX - 64);
-        const int x = x0 - 1 + c, y = y0 - 2 + r;
-        uint32_t lw = 0;
-        if ((unsigned)x < (unsigned)it.W && (unsigned)y < (unsigned)it.H)
-            lw = lane_word((uint32_t)((topdown ? it.H - 1 - y : y) * it.stride + x * it.ch));
-        s_lane[r * GLX + c] = lw;
-    }
-    __syncthreads();
-    // pass 2: position (x0 - 1 + cx, y0 - 1 + cy), same column split
-    auto edges = [&](int cx, int cy) {
-        const int c = (cy + 1) * GLX + cx;  // its lane word
-        uint32_t up = s_lane[c + GLX], ur = s_lane[c + GLX + 1], rt = s_lane[c + 1], dr = s_lane[c - GLX + 1];
-        LaneRef a = lane_ref(s_lane[c]);
-        uint32_t h = lane_similar(a, up) << 1 | lane_similar(a, ur) << 2 | lane_similar(a, rt) << 4 |
-                     lane_similar(a, dr) << 7;
-        s_h[cy * GHP + cx + 3] = (uint8_t)h;
     };
-    for (int cy = t >> 6; cy < GHY; cy += 4) edges(t & 63, cy);
-    if (t < (GHX - 64) * GHY) edges(64 + t % (GHX - 64), t / (GHX - 64));
-    __syncthreads();
-    // pass 3
-    uint8_t* g = gaux + it.g_off;
-    for (int k = t; k < GTX / 4 * TY; k += 256) {
-        int q = k % (GTX / 4), ly = k / (GTX / 4);
-        int x = x0 + 4 * q, y = y0 + ly;
-        if (x >= it.W || y >= it.H) continue;
-        const uint32_t* dn = s_h32 + ly * (GHP / 4) + q;  // row y-1; word q+1 holds x .. x+3
-        const uint32_t* md = dn + GHP / 4;
-        const uint32_t* up = md + GHP / 4;
-        uint32_t own = md[1], left = __builtin_amdgcn_alignbyte(md[1], md[0], 3);
-        uint32_t down = dn[1], dl = __builtin_amdgcn_alignbyte(dn[1], dn[0], 3);
-        uint32_t ul = __builtin_amdgcn_alignbyte(up[1], up[0], 3);
-        uint32_t edges = (own & 0x96969696u) | ((left & 0x10101010u) >> 1) | ((down & 0x02020202u) << 5) |
-                         ((dl & 0x04040404u) << 3) | ((ul & 0x80808080u) >> 7);
-        // full flags (bit 0 of each byte) of the blocks whose lower-left
-        // positions are the bytes of h: its up (bit 1) and right (bit 4)
-        // edges, the right edge of the byte above (in hu) and the up edge of
-        // the byte to the right (in hr, h shifted by one position)
-        auto full = [](uint32_t h, uint32_t hr, uint32_t hu) {
-            return (h >> 1) & (h >> 4) & (hu >> 4) & (hr >> 1) & 0x01010101u;
-        };
-        const uint32_t fm1 = full(md[1], __builtin_amdgcn_alignbyte(md[2], md[1], 1), up[1]);  // x .. x+3, row y
-        const uint32_t fm0 = full(md[0], __builtin_amdgcn_alignbyte(md[1], md[0], 1), up[0]);  // byte 3: x-1
-        const uint32_t fd1 = full(dn[1], __builtin_amdgcn_alignbyte(dn[2], dn[1], 1), md[1]);  // row y-1
-        const uint32_t fd0 = full(dn[0], __builtin_amdgcn_alignbyte(dn[1], dn[0], 1), md[0]);
-        uint32_t clear = (fm1 << 2) | __builtin_amdgcn_alignbyte(fm1, fm0, 3) |
-                         (__builtin_amdgcn_alignbyte(fd1, fd0, 3) << 5) | (fd1 << 7);
-        uint32_t v = edges & ~clear;
-        uint8_t* dst = g + (uint32_t)(y * it.W + x);
-        if (it.graph_w4) {
-            *reinterpret_cast<uint32_t*>(dst) = v;
+    // the pixels of a group once more, by bytes
+    auto fetch_bytes = [&](int r0) {
+        const uint32_t o = voff + (uint32_t)(r0 - 1) * step;
+#pragma unroll
+        for (int q = 0; q < G; q++) {
+            px[q] = 0;
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                px[q] |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(src, (int)(o + (uint32_t)q * step) + k, 0, 0)
+                         << (8 * k);
+        }
+    };
+
+    // Lane words.  Colours of three bytes c0, c1, c2: n = 299 c0 + 587 c1 +
+    // 114 c2 as two byte dot products, luma's quotient as in luma() (the high
+    // half of a 24-bit product, whose low half is 704 n / 1000 for a multiple
+    // of 1000 and at least 4294968 otherwise: the multiples but 0, black, take
+    // luma()'s double expression); the packed word is put together in the lane
+    // word's 10-bit lanes at once, where negative U and V borrow from the
+    // lane above as they do in yuv_pack's bytes (a lane below zero there is
+    // below zero here, since |U|, |V| < 256).
+    const uint32_t cls = col ? kLaneOpaque : 0u, cls_clear = col ? kLaneTransparent : 0u;
+    const uint32_t order = (it.flags & DPX_RGB) ? 0x03000102u : 0x03020100u;
+    const uint32_t clear_below = ((it.flags & DPX_ALPHA) && it.ch == 4) ? 1u << 24 : 0u;
+    const uint32_t col_mask = col ? ~0u : 0u;
+    auto lane_words = [&](uint32_t* v) {
+        if constexpr (PIXELS == kPixelsIndexed) {
+#pragma unroll
+            for (int q = 0; q < G; q++) v[q] = s_pal[v[q]] & col_mask;
         } else {
-            int n = min(4, it.W - x);
-            for (int b = 0; b < n; b++) dst[b] = (uint8_t)(v >> (8 * b));
+            uint32_t y[G];
+            uint64_t whole[G];
+#pragma unroll
+            for (int q = 0; q < G; q++) {
+                if constexpr (PIXELS == kPixelsGeneral) v[q] = __builtin_amdgcn_perm(0u, v[q], order);
+                const uint32_t n = __builtin_amdgcn_udot4(
+                    v[q], 0x00724B2Bu, __builtin_amdgcn_udot4(v[q], 0x00000201u, 0u, false) << 8, false);
+                y[q] = (uint32_t)(((uint64_t)(n & 0xFFFFFFu) * 4294968u) >> 32);
+                whole[q] = __builtin_amdgcn_ballot_w64((n & 0xFFFFFFu) * 4294968u - 1u < 4294967u);
+            }
+            uint64_t any = 0;
+#pragma unroll
+            for (int q = 0; q < G; q++) any |= whole[q];
+            if (any) {
+#pragma unroll
+                for (int q = 0; q < G; q++)
+                    if (whole[q])
+                        y[q] = (uint32_t)luma((int)(v[q] & 0xFFu), (int)((v[q] >> 8) & 0xFFu),
+                                              (int)((v[q] >> 16) & 0xFFu));
+            }
+#pragma unroll
+            for (int q = 0; q < G; q++) {
+                const int u = (int)((float)((int)((v[q] >> 16) & 0xFFu) - (int)y[q]) * 0.492f);
+                const int vv = (int)((float)((int)(v[q] & 0xFFu) - (int)y[q]) * 0.877f);
+                uint32_t f = (y[q] << 10) + (uint32_t)u;
+                asm("" : "+v"(f));  // (keeps the sum two shift-and-adds)
+                f = (((f << 10) + (uint32_t)vv) & 0x0FF3FCFFu) | cls;
+                if constexpr (PIXELS == kPixelsGeneral) f = v[q] < clear_below ? cls_clear : f;
+                v[q] = f;
+            }
         }
+    };
+
+    // The bytes are stored through a buffer descriptor of the item's graph:
+    // lanes whose pixel is not this strip's to write get an offset past its
+    // end, which the hardware drops, so that a group of rows has no branch
+    // and its rows overlap.
+    const uint32_t goff = (uint32_t)y0 * (uint32_t)W + (uint32_t)x;
+    const auto out = __builtin_amdgcn_make_buffer_rsrc(gaux + it.g_off, 0, W * H, 0x00020000);
+    uint64_t every = ~0ull;
+    asm("" : "+s"(every));  // (kept an operand, see shift_in)
+
+    LaneRow a = {};                           // row r - 1
+    uint64_t ra = 0, dra = 0, ua = 0, ura = 0;  // row r - 1's R and kept DR; row r - 2's U and kept UR
+    const uint32_t gput = lane_of(mine) ? goff : ~0u;
+
+    fetch(0);
+    // Loads and stores return in one order, so that waiting for a group's
+    // pixels need not wait for the stores issued after them, if their number
+    // is always the same: every pass below issues G stores, and so does the
+    // way into the loop (dropped).
+#pragma unroll
+    for (int q = 0; q < G; q++) __builtin_amdgcn_raw_buffer_store_b8((uint8_t)0, out, -1, 0, 0);
+    for (int r0 = 0; r0 < R; r0 += G) {
+        if (tail && (topdown ? r0 < 2 : r0 + G >= r_hi)) fetch_bytes(r0);
+        uint32_t w[G];
+#pragma unroll
+        for (int q = 0; q < G; q++) w[q] = px[q];
+        if (r0 + G < R) fetch(r0 + G);
+        lane_words(w);
+        if (r0 < r_lo || r0 + G > r_hi) {
+#pragma unroll
+            for (int q = 0; q < G; q++) w[q] = (unsigned)(y0 - 1 + r0 + q) < (unsigned)H ? w[q] : 0u;
+        }
+        RowEdges ed[G];
+#pragma unroll
+        for (int q = 0; q < G; q++) {
+            LaneRow b;
+            b.l = w[q];
+            ed[q] = row_edges(a, b);
+            a = b;
+        }
+        uint32_t byte[G];
+#pragma unroll
+        for (int q = 0; q < G; q++) {
+            const uint64_t u = ed[q].up & every, rt = ed[q].right & every;
+            const uint64_t full = u & ra & rt & (u >> 1);  // blocks with lower-left pixels in row r - 1
+            const uint64_t urk = ed[q].up_right & ~full, drk = ed[q].down_right & ~full;
+            byte[q] = lane_of(dra) ? 1u : 0u;
+            shift_in(byte[q], ua);
+            shift_in(byte[q], ura << 1);
+            shift_in(byte[q], ra);
+            shift_in(byte[q], ra << 1);
+            shift_in(byte[q], urk);
+            shift_in(byte[q], u);
+            shift_in(byte[q], drk << 1);
+            ra = rt;
+            dra = drk;
+            ua = u;
+            ura = urk;
+        }
+        // byte[q] is row r0 + q - 1's; rows 1 .. R - 2 in the frame are stored
+        uint32_t to[G];
+#pragma unroll
+        for (int q = 0; q < G; q++) to[q] = gput;
+        if (r0 < r_lo + 1 || r0 < 2 || r0 + G > min(r_hi + 1, R)) {
+#pragma unroll
+            for (int q = 0; q < G; q++)
+                to[q] = r0 + q >= 2 && r0 + q < R && (unsigned)(y0 - 2 + r0 + q) < (unsigned)H ? gput : ~0u;
+        }
+#pragma unroll
+        for (int q = 0; q < G; q++)
+            __builtin_amdgcn_raw_buffer_store_b8((uint8_t)byte[q], out, (int)to[q], (int)((uint32_t)max(r0 + q - 2, 0) * (uint32_t)W), 0);
     }
 }
 
-using GraphFn = void (*)(const DevItem*, const uint2*, int, const uint8_t*, uint8_t*);
-inline GraphFn graph_kernel(int ty)
+__global__ __launch_bounds__(64) void kf_graph(const DevItem* __restrict__ items, const uint2* __restrict__ tile_map,
+                                               int grid3d, int max_rows, const uint8_t* __restrict__ in,
+                                               uint8_t* __restrict__ gaux)
 {
-    return ty == kGraphSmallTY ? kf_graph<kGraphSmallTY> : ty == kGraphTallTY ? kf_graph<kGraphTallTY> : kf_graph<GTY>;
+    __shared__ uint32_t s_pal[256];
+    // runs of 8 strips per XCD: the lines that neighbouring strips' rows share
+    // are fetched once into one L2
+    const TileAt at = locate_tile<8>(tile_map, grid3d);
+    const DevItem it = items[at.item];
+    const uint32_t strip = (uint32_t)at.ty << 16 | (uint32_t)at.tx;
+    const GraphSplit sp = graph_split(it.W, it.H, max_rows);
+    if (it.flags & DPX_INDEXED) {
+        // the lane words of the 256 palette entries
+        const uint32_t order = (it.flags & DPX_RGB) ? 0x03000102u : 0x03020100u;
+        for (int k = threadIdx.x; k < 256; k += 64) {
+            const uint32_t e = __builtin_amdgcn_perm(0u, reinterpret_cast<const uint32_t*>(in + it.pal_off)[k], order);
+            uint32_t lw = yuv_lanes(yuv_pack((int)(e & 0xFFu), (int)((e >> 8) & 0xFFu), (int)((e >> 16) & 0xFFu))) |
+                          kLaneOpaque;
+            if ((it.flags & DPX_ALPHA) && (e >> 24) == 0) lw = kLaneTransparent;
+            s_pal[k] = lw;
+        }
+        __syncthreads();
+        graph_strip<kPixelsIndexed>(it, sp, strip, in, s_pal, gaux);
+    } else if (it.flags & (DPX_RGB | DPX_ALPHA)) {
+        graph_strip<kPixelsGeneral>(it, sp, strip, in, s_pal, gaux);
+    } else {
+        graph_strip<kPixelsPlain>(it, sp, strip, in, s_pal, gaux);
+    }
 }
 
 }  // namespace dpx
@@ -306,7 +495,7 @@ struct BatchPlan {
     uintptr_t out_mod = 0;  // d_out % 16
     dim3 ggrid;
     int g3d = 0;
-    int gty = dpx::GTY;  // graph tile rows (kf_graph<gty>)
+    int grows = dpx::kGraphMinRows;  // rows of kf_graph's blocks
     size_t off_items = 0, off_gmap = 0;
     std::vector<PlanGroup> groups;
 };
@@ -518,7 +707,6 @@ size_t desc_bytes(size_t n)
     return 2 * n * sizeof(DevItem) + 64 * (2 * 2 * (kMaxScale + 1) + 4);
 }
 
-// Tiles per item when all items of a prefix have the same count, else 0.
 // Launch grid of a kernel with TX x TY tiles over `dev`: (tile columns, tile
 // rows, items) when all items have the same tile grid, else 1-D over all
 // tiles with a map from block to (item, tile row << 16 | tile column).
@@ -538,6 +726,22 @@ dim3 tile_grid(const std::vector<DevItem>& dev, int TX, int TY, int* grid3d, std
         for (unsigned y = 0; y < ty; y++)
             for (unsigned x = 0; x < tx; x++) map->push_back(make_uint2((unsigned)k, y << 16 | x));
     }
+    return dim3((unsigned)map->size(), 1, 1);
+}
+
+// The same for kf_graph's strips: (strips, 1, items), or 1-D with a map to
+// (item, strip).
+dim3 strip_grid(const std::vector<DevItem>& dev, int max_rows, int* grid3d, std::vector<uint2>* map)
+{
+    const uint32_t n0 = graph_split(dev[0].W, dev[0].H, max_rows).strips;
+    bool same = dev.size() <= 65535;
+    for (const DevItem& d : dev) same = same && graph_split(d.W, d.H, max_rows).strips == n0;
+    map->clear();
+    *grid3d = same ? 1 : 0;
+    if (same) return dim3(n0, 1, (unsigned)dev.size());
+    for (size_t k = 0; k < dev.size(); k++)
+        for (uint32_t q = 0, n = graph_split(dev[k].W, dev[k].H, max_rows).strips; q < n; q++)
+            map->push_back(make_uint2((unsigned)k, q));
     return dim3((unsigned)map->size(), 1, 1);
 }
 
@@ -741,15 +945,10 @@ static int build_plan(dpx_context* ctx, const uint8_t* d_out, const dpx_item* it
     // launch grids
     int g3d = 0;
     std::vector<uint2> gmap;
-    uint64_t gtiles = 0, gtall = 0;
-    for (const DevItem& d : dev) {
-        gtiles += (uint64_t)((d.W + GTX - 1) / GTX) * ((d.H + GTY - 1) / GTY);
-        gtall += (uint64_t)((d.W + GTX - 1) / GTX) * ((d.H + kGraphTallTY - 1) / kGraphTallTY);
-    }
-    plan.gty = gtiles < kGraphSmallTiles                                ? kGraphSmallTY
-               : gtall * (kGraphTallTY + 4) < gtiles * (GTY + 4) ? kGraphTallTY
-                                                                 : GTY;
-    const dim3 ggrid = tile_grid(dev, GTX, plan.gty, &g3d, &gmap);
+    uint64_t pixels = 0;
+    for (const DevItem& d : dev) pixels += (uint64_t)d.W * d.H;
+    plan.grows = graph_rows(pixels);
+    const dim3 ggrid = strip_grid(dev, plan.grows, &g3d, &gmap);
     for (auto& kv : groups)
         kv.second.grid = tile_grid(kv.second.dev, kv.second.tx, 256 / kv.second.tx, &kv.second.grid3d, &kv.second.map);
 
@@ -825,8 +1024,7 @@ static int launch_plan(dpx_context* ctx, const BatchPlan& plan, const LaunchArgs
 {
     const DevItem* d_items = reinterpret_cast<const DevItem*>(la.desc + plan.off_items);
     const uint2* d_gmap = reinterpret_cast<const uint2*>(la.desc + plan.off_gmap);
-    hipLaunchKernelGGL(graph_kernel(plan.gty), plan.ggrid, dim3(256), 0, stream, d_items, d_gmap, plan.g3d, d_in,
-                       la.gaux);
+    hipLaunchKernelGGL(kf_graph, plan.ggrid, dim3(64), 0, stream, d_items, d_gmap, plan.g3d, plan.grows, d_in, la.gaux);
     if (ev_mid) DPX_HIP(hipEventRecord(ev_mid, stream));
     for (const PlanGroup& pg : plan.groups) {
         RasterFn fn = pick_raster(pg.scale, pg.sub, pg.tx, pg.walk);
@@ -923,6 +1121,7 @@ struct NodeArgs {
     const DevItem* items;
     const uint2* map;
     int g3d;
+    int grows;
     const uint8_t* in;
     const uint8_t* gaux_c;
     uint8_t* gaux;
@@ -948,10 +1147,12 @@ hipKernelNodeParams node_params(dpx_plan* p, int kind, int group, const uint8_t*
         a.items = reinterpret_cast<const DevItem*>(p->d_desc + p->plan.off_items);
         a.map = reinterpret_cast<const uint2*>(p->d_desc + p->plan.off_gmap);
         a.g3d = p->plan.g3d;
-        void* v[5] = { &a.items, &a.map, &a.g3d, &a.in, &a.gaux };
+        a.grows = p->plan.grows;
+        void* v[6] = { &a.items, &a.map, &a.g3d, &a.grows, &a.in, &a.gaux };
         memcpy(a.ptrs, v, sizeof(v));
-        np.func = reinterpret_cast<void*>(graph_kernel(p->plan.gty));
+        np.func = reinterpret_cast<void*>(kf_graph);
         np.gridDim = p->plan.ggrid;
+        np.blockDim = dim3(64);
     } else {
         const PlanGroup& pg = p->plan.groups[group];
         a.items = reinterpret_cast<const DevItem*>(p->d_desc + pg.off_items);
@@ -1157,11 +1358,17 @@ constexpr size_t na_info_off(int S) { return na_mask_off(S) + na_mask_bytes(S); 
 constexpr int kNaMaxItems = 4096;
 constexpr int kNaTX = kDefaultTileX, kNaTY = 256 / kDefaultTileX;  // raster tiles (the default shape)
 constexpr size_t kNaGraphTiles = 65536, kNaRasterTiles = 524288;
+// Limits are counted in graph tiles of 64x32 pixels.  The map holds two strips
+// a tile: blocks of 32 rows never take more ((blocks * (W + 1) + 60) / 62
+// strips against blocks * ceil(W / 64) tiles), and lower blocks are used only
+// where their strips fit too.
+constexpr int kNaGX = 64, kNaGY = 32;
+constexpr size_t kNaGraphStrips = 2 * kNaGraphTiles;
 constexpr size_t kNaGraphBytes = 48u << 20;
 constexpr size_t kNaOffItems = na_mask_off(kMaxScale + 1);
 constexpr size_t kNaOffGroupItems = kNaOffItems + na_align(kNaMaxItems * sizeof(DevItem));
 constexpr size_t kNaOffGmap = kNaOffGroupItems + na_align(kNaMaxItems * sizeof(DevItem));
-constexpr size_t kNaOffRmap = kNaOffGmap + na_align(kNaGraphTiles * sizeof(uint2));
+constexpr size_t kNaOffRmap = kNaOffGmap + na_align(kNaGraphStrips * sizeof(uint2));
 constexpr size_t kNaOffGraph = kNaOffRmap + na_align(kNaRasterTiles * sizeof(uint2));
 constexpr size_t kNaScratchBytes = kNaOffGraph + kNaGraphBytes;
 static_assert(kNaScratchBytes < (64u << 20), "scratch stays under 64 MiB");
@@ -1169,17 +1376,18 @@ static_assert(kNaScratchBytes < (64u << 20), "scratch stays under 64 MiB");
 static __device__ __align__(256) uint8_t scratch[kNaScratchBytes];
 
 // One item of a k_na_put launch: its descriptor, its slots in the item
-// arrays and the first entries of its tiles in the two tile maps.
+// arrays and the first entries of its strips and tiles in the two maps.
 struct NaPut {
     DevItem d;
     uint32_t index;  // in the item array (the graph launch's items)
     uint32_t gslot;  // in the grouped item array
     uint32_t gpos;   // gslot - the group's first slot (the raster launch's items)
-    uint32_t gtile, rtile;
+    uint32_t gstrip, rtile;
 };
 constexpr int kNaPutChunk = 32;
 struct NaPutArgs {
     uint32_t n;
+    int grows;  // rows of the graph launch's blocks
     NaPut it[kNaPutChunk];
 };
 static_assert(sizeof(NaPutArgs) <= 4000, "kernel arguments stay under 4 KB");
@@ -1194,9 +1402,8 @@ __global__ __launch_bounds__(256) void k_na_put(NaPutArgs a, DevItem* __restrict
             items[p.index] = p.d;
             group_items[p.gslot] = p.d;
         }
-        const uint32_t gx = (uint32_t)(p.d.W + GTX - 1) / GTX, gy = (uint32_t)(p.d.H + GTY - 1) / GTY;
-        for (uint32_t t = threadIdx.x; t < gx * gy; t += blockDim.x)
-            gmap[p.gtile + t] = make_uint2(p.index, (t / gx) << 16 | (t % gx));
+        const uint32_t gs = graph_split(p.d.W, p.d.H, a.grows).strips;
+        for (uint32_t t = threadIdx.x; t < gs; t += blockDim.x) gmap[p.gstrip + t] = make_uint2(p.index, t);
         const uint32_t rx = (uint32_t)(p.d.W + kNaTX - 1) / kNaTX, ry = (uint32_t)(p.d.H + kNaTY - 1) / kNaTY;
         for (uint32_t t = threadIdx.x; t < rx * ry; t += blockDim.x)
             rmap[p.rtile + t] = make_uint2(p.gpos, (t / rx) << 16 | (t % rx));
@@ -1251,13 +1458,15 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
     // its item and tile counts
     uint32_t gcount[2 * (kMaxScale + 1)] = {}, gtiles[2 * (kMaxScale + 1)] = {};
     size_t gbytes = 0, graph_tiles = 0, raster_tiles = 0;
+    uint64_t pixels = 0;
     for (int k = 0; k < n_items; k++) {
         DevItem d;
         if (int rc = make_dev_item(items[k], k, d_out, 0, d)) return rc;
         DPX_CHECK(!d.subdivide, DPX_EINVAL,
                   "item %d: subdivision needs per-cell row buffers; dpx_batch_run_noalloc takes items without it", k);
         gbytes += align_up((size_t)d.W * d.H, 256);
-        graph_tiles += (size_t)((d.W + GTX - 1) / GTX) * ((d.H + GTY - 1) / GTY);
+        graph_tiles += (size_t)((d.W + kNaGX - 1) / kNaGX) * ((d.H + kNaGY - 1) / kNaGY);
+        pixels += (uint64_t)d.W * d.H;
         const size_t rt = (size_t)((d.W + kNaTX - 1) / kNaTX) * ((d.H + kNaTY - 1) / kNaTY);
         raster_tiles += rt;
         const int g = 2 * d.scale + d.subdivide;
@@ -1270,6 +1479,14 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
     DPX_CHECK(graph_tiles <= kNaGraphTiles && raster_tiles <= kNaRasterTiles, DPX_EINVAL,
               "batch has %zu graph and %zu raster tiles: dpx_batch_run_noalloc holds at most %zu and %zu", graph_tiles,
               raster_tiles, kNaGraphTiles, kNaRasterTiles);
+    auto count_strips = [&](int rows) {
+        size_t n = 0;
+        for (int k = 0; k < n_items; k++) n += graph_split(items[k].width, items[k].height, rows).strips;
+        return n;
+    };
+    int grows = graph_rows(pixels);
+    size_t graph_strips = count_strips(grows);
+    if (graph_strips > kNaGraphStrips) graph_strips = count_strips(grows = kNaGY);
     uint8_t* base = nullptr;
     if (int rc = na_setup(dev, stream, &base)) return rc;
     DevItem* d_items = reinterpret_cast<DevItem*>(base + kNaOffItems);
@@ -1290,6 +1507,7 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
     uint32_t gnext[2 * (kMaxScale + 1)] = {}, gtnext[2 * (kMaxScale + 1)] = {};
     NaPutArgs args;
     memset(&args, 0, sizeof(args));
+    args.grows = grows;
     uint64_t goff = 0;
     uint32_t gt = 0;
     for (int k = 0; k < n_items; k++) {
@@ -1299,9 +1517,9 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
         p.index = (uint32_t)k;
         p.gpos = gnext[g]++;
         p.gslot = gslot0[g] + p.gpos;
-        p.gtile = gt;
+        p.gstrip = gt;
         p.rtile = gtile0[g] + gtnext[g];
-        gt += (uint32_t)(((p.d.W + GTX - 1) / GTX) * ((p.d.H + GTY - 1) / GTY));
+        gt += graph_split(p.d.W, p.d.H, grows).strips;
         gtnext[g] += (uint32_t)(((p.d.W + kNaTX - 1) / kNaTX) * ((p.d.H + kNaTY - 1) / kNaTY));
         goff += align_up((size_t)p.d.W * p.d.H, 256);
         if (args.n == kNaPutChunk || k == n_items - 1) {
@@ -1309,8 +1527,8 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
             args.n = 0;
         }
     }
-    hipLaunchKernelGGL(kf_graph<GTY>, dim3((unsigned)graph_tiles), dim3(256), 0, stream, d_items, d_gmap, 0, d_in,
-                       d_graph);
+    hipLaunchKernelGGL(kf_graph, dim3((unsigned)graph_strips), dim3(64), 0, stream, d_items, d_gmap, 0,
+                       grows, d_in, d_graph);
     for (int g = 0; g < 2 * (kMaxScale + 1); g++) {
         if (!gcount[g]) continue;
         const int S = g / 2;
