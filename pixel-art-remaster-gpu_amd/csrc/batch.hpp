@@ -58,8 +58,8 @@ __host__ __device__ inline uint32_t coverage_info(const uint32_t* rows, int S)
     return info | (full ? 1u : 0u);
 }
 
-// Cell masks at 1x and 2x follow the row table (kt_cell).
-constexpr int kMaxCellScale = 2;
+// Cell masks at 1x to 4x follow the row table (kt_cell).
+constexpr int kMaxCellScale = 4;
 
 // A cell whose own square it covers fully, and into which none of the four
 // cells drawn after it (up-left, up, up-right, right) reaches, shows its own
@@ -568,6 +568,8 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     constexpr int PX_WORDS = 2048, PX_CELLS = PX_WORDS / (S * S), PX_CODE_CELLS = PX_WORDS / (S * ROW_WORDS);
     static_assert(PX_CELLS >= 1, "at least one buffered cell");
     __shared__ uint32_t s_px[PX_WORDS];
+    // 3x and 4x: the winners of listed cells' pixels (two words a cell)
+    __shared__ uint32_t s_plane[!SUB && (S == 3 || S == 4) ? 2 * RTX * RTY : 1];
     __shared__ uint16_t s_idx[RTX * RTY];  // list index of a listed own cell, else kOwnColour
     constexpr uint32_t kOwnColour = 0xFFFF;  // the cell shows its own colour only
     const uint8_t* s_g = reinterpret_cast<const uint8_t*>(s_g32);
@@ -805,7 +807,54 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
         }
     };
 
-    if constexpr (!SUB && S <= kMaxCellScale) {
+    if constexpr (!SUB && (S == 3 || S == 4)) {
+        // 3x and 4x: one thread per listed cell picks the winners of all its
+        // pixels (nine independent loads from the cell-mask table, planes of
+        // S * S bits), then one thread per row of a listed cell looks its
+        // colours up.  Rows that each fetch and resolve their own nine table
+        // rows do the first part S times over: per batch at 4x, 1024 frames
+        // of 256x224 884 -> 850 us, 64 console frames 83 -> 77, 128 indexed
+        // frames 141 -> 133; 64 console frames at 3x 88 -> 82.
+        const uint16_t* cell_table = reinterpret_cast<const uint16_t*>(mask_table + kKeys * MW);
+        const int nlist = s_nlist;
+        for (int i = t; i < nlist; i += 256) {
+            const int own = s_list[i];
+            const int ux = own % RTX, uy = own / RTX;
+            uint32_t m[9];
+#pragma unroll
+            for (int j = 0; j < 9; j++) {
+                const uint32_t key = s_key[(uy + 2 - j / 3) * RCX + (ux + 2 - j % 3)];
+                m[j] = key != kNoCell ? cell_table[key * 9 + j] : 0u;
+            }
+            uint32_t seen = 0;
+#pragma unroll
+            for (int j = 0; j < 9; j++) {
+                const uint32_t nb = m[j] & ~seen;
+                seen |= m[j];
+                m[j] = nb;
+            }
+            const uint32_t none = ~seen & ((1u << (S * S)) - 1u);
+            s_plane[i] = (m[1] | m[4] | m[7] | none) | (m[2] | m[5] | m[8] | none) << 16;
+            s_plane[RTX * RTY + i] = (m[3] | m[4] | m[5]) | (m[6] | m[7] | m[8]) << 16;
+        }
+        __syncthreads();
+        for (int u = t; u < nunits; u += 256) {
+            const int i = u / S, ky = u % S, own = s_list[i];
+            const int ux = own % RTX, uy = own / RTX, last = (uy + 2) * RCX + ux + 2;
+            Winners r;
+            r.w[0] = __builtin_amdgcn_perm(s_plane[RTX * RTY + i] >> (ky * S), s_plane[i] >> (ky * S), 0x06040200u);
+            uint32_t col[S];
+#pragma unroll
+            for (int q = 0; q < S; q++) col[q] = winner_colour(r, q, last);
+            if (i < PX_CELLS) {
+#pragma unroll
+                for (int q = 0; q < S; q++) s_px[u * S + q] = col[q];
+            } else {
+                store_row(x0 + ux, (y0 + uy) * S + ky, col);  // beyond the buffer: written directly
+            }
+        }
+        __syncthreads();
+    } else if constexpr (!SUB && S <= 2) {
         // 1x and 2x: one thread per listed cell, the candidates' samples of
         // it from the cell-mask table (nine independent loads), resolved in
         // the same draw order as the rows of the other scales.  Measured: 2x

@@ -10,7 +10,7 @@
 //              (and, with subdivision, hulls, smoothed polygons and their
 //              coverage) in LDS; cells whose S*S pixels are all their own
 //              colour are simple, the rest are listed and resolved row by
-//              row (1x, 2x: cell by cell) against the 3x3 candidate cells
+//              row (1x to 4x: cell by cell) against the 3x3 candidate cells
 //              in draw order into an LDS pixel buffer; then every row of
 //              the tile's output is stored once, simple and resolved pixels
 //              by the same store instructions.
@@ -20,7 +20,7 @@
 // bitmasks (kt_mask): bit b of row r of key k says whether sample
 // (kmin+b, kmin+r) of the cell's local sample grid is covered, kmin =
 // -(S/2)-1, MW = 2S+2 rows and columns (local [-0.5, 1.5] of the cell); into
-// a 16-bit summary per key (kt_info, coverage_info); and at 1x and 2x into
+// a 16-bit summary per key (kt_info, coverage_info); and at 1x to 4x into
 // each key's sample mask of each neighbour cell (kt_cell).
 //
 // With subdivision, kf_smooth runs between the two: it resolves the
