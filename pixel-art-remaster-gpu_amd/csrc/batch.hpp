@@ -58,8 +58,40 @@ __host__ __device__ inline uint32_t coverage_info(const uint32_t* rows, int S)
     return info | (full ? 1u : 0u);
 }
 
-// Cell masks at 1x to 4x follow the row table (kt_cell).
-constexpr int kMaxCellScale = 4;
+// Cell masks: what a cell shows of the 3x3 cells around it, per cell the
+// samples of all its rows at once (up to 7x).  Mask j = (1 - dy) * 3 + (1 - dx) is what
+// the cell contributes as candidate (dx, dy) of the cell at (-dx, -dy) from
+// it: up to 4x bit ky * S + q of 16, from 5x bit q of byte ky of 64 (sample q
+// of row ky).  The masks of the table's keys follow its rows (kt_cell).
+constexpr int kMaxCellScale = 7, kMaxCellScale16 = 4;
+__host__ __device__ constexpr size_t cell_table_bytes(int S)
+{
+    return S > kMaxCellScale ? 0 : (size_t)kKeys * 9 * (S <= kMaxCellScale16 ? 2 : 8);
+}
+template <int S>
+using CellMask = std::conditional_t<S <= kMaxCellScale16, uint32_t, uint64_t>;
+
+// The nine masks of a cell with coverage rows `row(r)`, each handed to
+// put(j, mask).
+template <int S, class R, class F>
+__host__ __device__ inline void cell_masks(R row, F put)
+{
+    const int kmin = mask_kmin(S), mw = mask_w(S);
+    constexpr int STEP = S <= kMaxCellScale16 ? S : 8;
+#pragma unroll
+    for (int j = 0; j < 9; j++) {
+        const int dy = 1 - j / 3, dx = 1 - j % 3, sh = -dx * S - kmin;
+        CellMask<S> m = 0;
+#pragma unroll
+        for (int ky = 0; ky < S; ky++) {
+            const int r = ky - dy * S - kmin;
+            if (r < 0 || r >= mw) continue;
+            const uint32_t bits = (sh >= 0 ? (row(r) >> sh) : (row(r) << -sh)) & ((1u << S) - 1u);
+            m |= (CellMask<S>)bits << (ky * STEP);
+        }
+        put(j, m);
+    }
+}
 
 // A cell whose own square it covers fully, and into which none of the four
 // cells drawn after it (up-left, up, up-right, right) reaches, shows its own
@@ -568,8 +600,10 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     constexpr int PX_WORDS = 2048, PX_CELLS = PX_WORDS / (S * S), PX_CODE_CELLS = PX_WORDS / (S * ROW_WORDS);
     static_assert(PX_CELLS >= 1, "at least one buffered cell");
     __shared__ uint32_t s_px[PX_WORDS];
-    // 3x and 4x: the winners of listed cells' pixels (two words a cell)
-    __shared__ uint32_t s_plane[!SUB && (S == 3 || S == 4) ? 2 * RTX * RTY : 1];
+    // 3x to 7x: the winners of listed cells' pixels, as two words a cell up to
+    // 4x, a word a row from 5x (tiles that do not keep them in s_px)
+    constexpr bool MASKS = !SUB && S >= 3 && S <= kMaxCellScale;
+    __shared__ uint32_t s_plane[!MASKS ? 1 : S <= kMaxCellScale16 ? 2 * RTX * RTY : PX_CELLS * S];
     __shared__ uint16_t s_idx[RTX * RTY];  // list index of a listed own cell, else kOwnColour
     constexpr uint32_t kOwnColour = 0xFFFF;  // the cell shows its own colour only
     const uint8_t* s_g = reinterpret_cast<const uint8_t*>(s_g32);
@@ -807,53 +841,78 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
         }
     };
 
-    if constexpr (!SUB && (S == 3 || S == 4)) {
-        // 3x and 4x: one thread per listed cell picks the winners of all its
-        // pixels (nine independent loads from the cell-mask table, planes of
-        // S * S bits), then one thread per row of a listed cell looks its
-        // colours up.  Rows that each fetch and resolve their own nine table
-        // rows do the first part S times over: per batch at 4x, 1024 frames
-        // of 256x224 884 -> 850 us, 64 console frames 83 -> 77, 128 indexed
-        // frames 141 -> 133; 64 console frames at 3x 88 -> 82.
-        const uint16_t* cell_table = reinterpret_cast<const uint16_t*>(mask_table + kKeys * MW);
-        const int nlist = s_nlist;
-        for (int i = t; i < nlist; i += 256) {
-            const int own = s_list[i];
+    if constexpr (MASKS) {
+        // 3x to 7x: a listed cell's winners are picked for all its pixels at
+        // once, from nine independent loads of the cell-mask table: one thread
+        // a cell up to 4x, two (four rows each) from 5x.  A tile that keeps
+        // winners is then resolved, else one thread per row of a listed cell
+        // looks its colours up.  Rows that each fetch and resolve their own
+        // nine table rows do the first part S times over: per batch at 4x,
+        // 1024 frames of 256x224 884 -> 850 us, 64 console frames 83 -> 77,
+        // 128 indexed frames 141 -> 133; at 6x, 4096 sprites 129 -> 120, 8
+        // frames of 640x480 97 -> 83.  At 8x the stores bound the batch
+        // either way, and the rows, spread over more threads, keep them
+        // flowing (16 frames of 640x480: 256 us against 264).
+        constexpr int TB = S <= kMaxCellScale16 ? 2 : 4;  // bytes of a thread's masks
+        constexpr int PARTS = S <= kMaxCellScale16 ? 1 : 2;
+        const uint8_t* cell_table = reinterpret_cast<const uint8_t*>(mask_table + kKeys * MW);
+        const int nparts = s_nlist * PARTS;
+        for (int p = t; p < nparts; p += 256) {
+            const int i = p / PARTS, h = p % PARTS, own = s_list[i];
             const int ux = own % RTX, uy = own / RTX;
             uint32_t m[9];
 #pragma unroll
             for (int j = 0; j < 9; j++) {
                 const uint32_t key = s_key[(uy + 2 - j / 3) * RCX + (ux + 2 - j % 3)];
-                m[j] = key != kNoCell ? cell_table[key * 9 + j] : 0u;
+                m[j] = 0;
+                if (key != kNoCell) __builtin_memcpy(&m[j], cell_table + ((key * 9 + j) * PARTS + h) * TB, TB);
             }
             uint32_t seen = 0;
 #pragma unroll
             for (int j = 0; j < 9; j++) {
-                const uint32_t nb = m[j] & ~seen;
+                const uint32_t won = m[j] & ~seen;
                 seen |= m[j];
-                m[j] = nb;
+                m[j] = won;
             }
-            const uint32_t none = ~seen & ((1u << (S * S)) - 1u);
-            s_plane[i] = (m[1] | m[4] | m[7] | none) | (m[2] | m[5] | m[8] | none) << 16;
-            s_plane[RTX * RTY + i] = (m[3] | m[4] | m[5]) | (m[6] | m[7] | m[8]) << 16;
-        }
-        __syncthreads();
-        for (int u = t; u < nunits; u += 256) {
-            const int i = u / S, ky = u % S, own = s_list[i];
-            const int ux = own % RTX, uy = own / RTX, last = (uy + 2) * RCX + ux + 2;
-            Winners r;
-            r.w[0] = __builtin_amdgcn_perm(s_plane[RTX * RTY + i] >> (ky * S), s_plane[i] >> (ky * S), 0x06040200u);
-            uint32_t col[S];
-#pragma unroll
-            for (int q = 0; q < S; q++) col[q] = winner_colour(r, q, last);
-            if (i < PX_CELLS) {
-#pragma unroll
-                for (int q = 0; q < S; q++) s_px[u * S + q] = col[q];
+            const uint32_t px0 = m[1] | m[4] | m[7] | ~seen, px1 = m[2] | m[5] | m[8] | ~seen;
+            const uint32_t py0 = m[3] | m[4] | m[5], py1 = m[6] | m[7] | m[8];
+            if constexpr (PARTS == 1) {
+                s_plane[2 * i] = __builtin_amdgcn_perm(px1, px0, 0x05040100u);
+                s_plane[2 * i + 1] = py0 | py1 << 16;
             } else {
-                store_row(x0 + ux, (y0 + uy) * S + ky, col);  // beyond the buffer: written directly
+                uint32_t* words = (codes ? s_px : s_plane) + i * S + 4 * h;  // (every cell fits the former)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    // byte r of the four planes: row 4 h + r
+                    const uint32_t two = (uint32_t)(4 + r) << 8 | (uint32_t)r;
+                    const uint32_t w = __builtin_amdgcn_perm(px1, px0, 0x0C0C0000u | two) |
+                                       __builtin_amdgcn_perm(py1, py0, two << 16 | 0x0C0Cu);
+                    if (r < S - 4 || h == 0) words[r] = w;
+                }
             }
         }
         __syncthreads();
+        if (!codes) {
+            for (int u = t; u < nunits; u += 256) {
+                const int i = u / S, ky = u % S, own = s_list[i];
+                const int ux = own % RTX, uy = own / RTX, last = (uy + 2) * RCX + ux + 2;
+                Winners r;
+                if constexpr (S <= kMaxCellScale16)
+                    r.w[0] = __builtin_amdgcn_perm(s_plane[2 * i + 1] >> (ky * S), s_plane[2 * i] >> (ky * S), 0x06040200u);
+                else
+                    r.w[0] = s_plane[u];
+                uint32_t col[S];
+#pragma unroll
+                for (int q = 0; q < S; q++) col[q] = winner_colour(r, q, last);
+                if (i < PX_CELLS) {
+#pragma unroll
+                    for (int q = 0; q < S; q++) s_px[u * S + q] = col[q];
+                } else {
+                    store_row(x0 + ux, (y0 + uy) * S + ky, col);  // beyond the buffer: written directly
+                }
+            }
+            __syncthreads();
+        }
     } else if constexpr (!SUB && S <= 2) {
         // 1x and 2x: one thread per listed cell, the candidates' samples of
         // it from the cell-mask table (nine independent loads), resolved in

@@ -10,7 +10,7 @@
 //              (and, with subdivision, hulls, smoothed polygons and their
 //              coverage) in LDS; cells whose S*S pixels are all their own
 //              colour are simple, the rest are listed and resolved row by
-//              row (1x to 4x: cell by cell) against the 3x3 candidate cells
+//              row (1x to 7x: cell by cell) against the 3x3 candidate cells
 //              in draw order into an LDS pixel buffer; then every row of
 //              the tile's output is stored once, simple and resolved pixels
 //              by the same store instructions.
@@ -20,7 +20,7 @@
 // bitmasks (kt_mask): bit b of row r of key k says whether sample
 // (kmin+b, kmin+r) of the cell's local sample grid is covered, kmin =
 // -(S/2)-1, MW = 2S+2 rows and columns (local [-0.5, 1.5] of the cell); into
-// a 16-bit summary per key (kt_info, coverage_info); and at 1x to 4x into
+// a 16-bit summary per key (kt_info, coverage_info); and at 1x to 7x into
 // each key's sample mask of each neighbour cell (kt_cell).
 //
 // With subdivision, kf_smooth runs between the two: it resolves the
@@ -84,27 +84,25 @@ __global__ void kt_mask(int S, uint32_t* __restrict__ mask)
 }
 
 
-// Cell masks (scales up to kMaxCellScale): entry j = (1 - dy) * 3 + (1 - dx)
-// of key k holds, as bit ky * S + q, whether a cell of key k covers sample q
-// of row ky of the cell at (-dx, -dy) from it, i.e. what k contributes when
-// it is the candidate at (dx, dy) of that cell.  They follow the row table
-// in the same allocation.
-__global__ void kt_cell(const uint32_t* __restrict__ mask, int S, uint16_t* __restrict__ cell)
+// The keys' cell masks (cell_masks), after the row table in the same
+// allocation: entry key * 9 + j.
+template <int S>
+__global__ void kt_cell(const uint32_t* __restrict__ mask, uint8_t* __restrict__ cell)
 {
-    int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= kKeys * 9) return;
-    const int key = gid / 9, j = gid % 9, dy = 1 - j / 3, dx = 1 - j % 3;
-    const int kmin = mask_kmin(S), mw = mask_w(S);
-    const uint32_t full = (1u << S) - 1u;
-    const int sh = -dx * S - kmin;
-    uint32_t m = 0;
-    for (int ky = 0; ky < S; ky++) {
-        const int r = ky - dy * S - kmin;
-        if (r < 0 || r >= mw) continue;
-        const uint32_t row = mask[(size_t)key * mw + r];
-        m |= ((sh >= 0 ? (row >> sh) : (row << -sh)) & full) << (ky * S);
-    }
-    cell[gid] = (uint16_t)m;
+    constexpr int TB = S <= kMaxCellScale16 ? 2 : 8;
+    const int key = blockIdx.x * blockDim.x + threadIdx.x;
+    if (key >= kKeys) return;
+    const uint32_t* rows = mask + (size_t)key * mask_w(S);
+    cell_masks<S>([&](int r) { return rows[r]; },
+                  [&](int j, CellMask<S> m) { __builtin_memcpy(cell + (size_t)(key * 9 + j) * TB, &m, TB); });
+}
+
+using CellFn = void (*)(const uint32_t*, uint8_t*);
+inline CellFn pick_cell_table(int S)
+{
+    static constexpr CellFn fns[kMaxCellScale + 1] = { nullptr,    kt_cell<1>, kt_cell<2>, kt_cell<3>, kt_cell<4>,
+                                                       kt_cell<5>, kt_cell<6>, kt_cell<7> };
+    return S <= kMaxCellScale ? fns[S] : nullptr;
 }
 
 __global__ void kt_info(const uint32_t* __restrict__ mask, int S, uint16_t* __restrict__ info)
@@ -619,13 +617,13 @@ int ensure_mask(dpx_context* ctx, int S)
 {
     if (ctx->d_mask[S] && ctx->d_info[S]) return DPX_OK;
     size_t n = (size_t)kKeys * mask_w(S);
-    const size_t cell_bytes = S <= kMaxCellScale ? (size_t)kKeys * 9 * sizeof(uint16_t) : 0;
+    const size_t cell_bytes = cell_table_bytes(S);
     if (!ctx->d_mask[S]) DPX_HIP(hipMalloc(&ctx->d_mask[S], n * sizeof(uint32_t) + cell_bytes));
     if (!ctx->d_info[S]) DPX_HIP(hipMalloc(&ctx->d_info[S], kKeys * sizeof(uint16_t)));
     hipLaunchKernelGGL(kt_mask, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, S, ctx->d_mask[S]);
     if (cell_bytes)
-        hipLaunchKernelGGL(kt_cell, dim3((unsigned)((kKeys * 9 + 255) / 256)), dim3(256), 0, 0, ctx->d_mask[S], S,
-                           reinterpret_cast<uint16_t*>(ctx->d_mask[S] + n));
+        hipLaunchKernelGGL(pick_cell_table(S), dim3(kKeys / 256), dim3(256), 0, 0, ctx->d_mask[S],
+                           reinterpret_cast<uint8_t*>(ctx->d_mask[S] + n));
     hipLaunchKernelGGL(kt_info, dim3(kKeys / 256), dim3(256), 0, 0, ctx->d_mask[S], S, ctx->d_info[S]);
     DPX_HIP(hipGetLastError());
     DPX_HIP(hipDeviceSynchronize());
@@ -1328,8 +1326,8 @@ extern "C" int dpx_batch_timing_read(dpx_context* ctx, dpx_batch_times* out)
 // dpx_batch_run_noalloc: the batched path with every buffer beyond the
 // caller's input and output in one static device array, `scratch`, so that a
 // call allocates nothing.  Layout (all offsets 256-byte aligned):
-//   tables     per scale 1..15 the coverage rows (with the cell masks at 1x
-//              and 2x) and the coverage summaries, built on the first call
+//   tables     per scale 1..15 the coverage rows (with the cell masks at 1x to
+//              7x) and the coverage summaries, built on the first call
 //              on each device;
 //   items      the batch's device items, in item order and grouped by
 //              (scale, subdivision);
@@ -1344,7 +1342,7 @@ namespace {
 constexpr size_t na_align(size_t v) { return (v + 255) / 256 * 256; }
 constexpr size_t na_mask_bytes(int S)
 {
-    return na_align((size_t)kKeys * mask_w(S) * 4 + (S <= kMaxCellScale ? (size_t)kKeys * 9 * 2 : 0));
+    return na_align((size_t)kKeys * mask_w(S) * 4 + cell_table_bytes(S));
 }
 constexpr size_t na_info_bytes() { return na_align((size_t)kKeys * 2); }
 constexpr size_t na_mask_off(int S)
@@ -1429,8 +1427,8 @@ int na_setup(int dev, hipStream_t stream, uint8_t** out)
             const size_t n = (size_t)kKeys * mask_w(S);
             hipLaunchKernelGGL(kt_mask, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, S, mask);
             if (S <= kMaxCellScale)
-                hipLaunchKernelGGL(kt_cell, dim3((unsigned)((kKeys * 9 + 255) / 256)), dim3(256), 0, stream, mask, S,
-                                   reinterpret_cast<uint16_t*>(mask + n));
+                hipLaunchKernelGGL(pick_cell_table(S), dim3(kKeys / 256), dim3(256), 0, stream, mask,
+                                   reinterpret_cast<uint8_t*>(mask + n));
             hipLaunchKernelGGL(kt_info, dim3(kKeys / 256), dim3(256), 0, stream, mask, S,
                                reinterpret_cast<uint16_t*>(ptr + na_info_off(S)));
         }
