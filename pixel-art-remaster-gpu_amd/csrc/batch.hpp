@@ -59,37 +59,33 @@ __host__ __device__ inline uint32_t coverage_info(const uint32_t* rows, int S)
 }
 
 // Cell masks: what a cell shows of the 3x3 cells around it, per cell the
-// samples of all its rows at once (up to 7x).  Mask j = (1 - dy) * 3 + (1 - dx) is what
+// samples of all its rows at once.  Mask j = (1 - dy) * 3 + (1 - dx) is what
 // the cell contributes as candidate (dx, dy) of the cell at (-dx, -dy) from
-// it: up to 4x bit ky * S + q of 16, from 5x bit q of byte ky of 64 (sample q
-// of row ky).  The masks of the table's keys follow its rows (kt_cell).
-constexpr int kMaxCellScale = 7, kMaxCellScale16 = 4;
+// it: up to 4x bit ky * S + q of 16, from 5x bit q of byte ky (sample q of row
+// ky).  The masks of the table's keys follow its rows (kt_cell: 2 or 8 bytes
+// a mask); a smoothed cell's are written by kf_smooth (2 or S bytes a mask,
+// then the summary's low byte) in place of its rows.
+constexpr int kMaxCellScale = 8, kMaxCellScale16 = 4;
 __host__ __device__ constexpr size_t cell_table_bytes(int S)
 {
     return S > kMaxCellScale ? 0 : (size_t)kKeys * 9 * (S <= kMaxCellScale16 ? 2 : 8);
 }
-template <int S>
-using CellMask = std::conditional_t<S <= kMaxCellScale16, uint32_t, uint64_t>;
 
-// The nine masks of a cell with coverage rows `row(r)`, each handed to
-// put(j, mask).
+// The rows of the nine masks of a cell with coverage rows `row(r)`: put(j,
+// ky, bits), those without any left out.
 template <int S, class R, class F>
-__host__ __device__ inline void cell_masks(R row, F put)
+__host__ __device__ inline void cell_mask_rows(R row, F put)
 {
-    const int kmin = mask_kmin(S), mw = mask_w(S);
-    constexpr int STEP = S <= kMaxCellScale16 ? S : 8;
+    constexpr int kmin = mask_kmin(S), mw = mask_w(S);
 #pragma unroll
     for (int j = 0; j < 9; j++) {
         const int dy = 1 - j / 3, dx = 1 - j % 3, sh = -dx * S - kmin;
-        CellMask<S> m = 0;
 #pragma unroll
         for (int ky = 0; ky < S; ky++) {
             const int r = ky - dy * S - kmin;
             if (r < 0 || r >= mw) continue;
-            const uint32_t bits = (sh >= 0 ? (row(r) >> sh) : (row(r) << -sh)) & ((1u << S) - 1u);
-            m |= (CellMask<S>)bits << (ky * STEP);
+            put(j, ky, (sh >= 0 ? (row(r) >> sh) : (row(r) << -sh)) & ((1u << S) - 1u));
         }
-        put(j, m);
     }
 }
 
@@ -178,10 +174,11 @@ constexpr uint16_t kNoCell = 0xFFFF;
     constexpr int GY = TS::GY, AY = TS::AY, RDW = TS::DW, RDB = TS::DB;                                    \
     (void)RTX; (void)RTY; (void)RCX; (void)RCY; (void)RWW; (void)RWB; (void)GY; (void)AY; (void)RDW; (void)RDB
 
-// Per-cell coverage rows of smoothed cells (kf_smooth -> kf_raster<S, true>):
-// MW words of sample rows and one word of coverage summary per cell, cell
-// (x, y) of an item at word (y * W + x) * (MW + 1) of its range.
-__host__ __device__ constexpr int rows_words(int S) { return mask_w(S) + 1; }
+// Per-cell coverage of smoothed cells (kf_smooth -> kf_raster<S, true>): up to
+// 8x the nine cell masks and the coverage summary, from 9x MW words of sample
+// rows and one of summary; cell (x, y) of an item at word (y * W + x) *
+// rows_words(S) of its range.
+__host__ __device__ constexpr int rows_words(int S) { return (int)cell_row_words(S); }
 
 // The snapshot rows ay0 .. ay0 + AY - 1 of a tile's window into LDS.  With
 // W % 4 == 0 the graph rows are word aligned and a word is either wholly
@@ -389,8 +386,9 @@ __device__ inline void tile_resolved_load(const DevItem& it, const uint8_t* __re
 // tile of cells (subdivision_Kernel kernel.cu:216-261 on the cells_Kernel
 // hulls, then triangulate_Kernel's ear clipping, kernel.cu:264-282), each
 // own cell once.  Writes the tile's resolved graph bytes to gfin and, for
-// every smoothed (non-internal) cell, the coverage rows of its triangles at
-// scale S with their summary to `rows` (rows_words(S) words per cell).
+// every smoothed (non-internal) cell, the coverage of its triangles at scale S
+// with its summary to `rows` (rows_words(S) words per cell: its cell masks up
+// to 8x, its rows from 9x).
 // Internal cells (node 90) keep their hull (kernel.cu:231): the raster takes
 // their rows from the table.
 //
@@ -429,8 +427,8 @@ __global__ __launch_bounds__(256, 3) void kf_smooth(const DevItem* __restrict__ 
     // vertex k of column t at [k * 256 + t]; a hull has at most 8 vertices,
     // its smoothed polygon at most 16, within the cells around (-64 .. 127)
     __shared__ uint16_t s_poly[16 * 256];
-    // sample row r of column t at [r * PITCH + t], then the summary; first the walk window
-    constexpr int COV = RW * PITCH, WALK_WORDS = WALK ? WalkWindow<TX>::BYTES / 4 : 0;
+    // sample row r of column t at [r * PITCH + t], then its masks and summary; first the walk window
+    constexpr int COV = (MW + 1) * PITCH, WALK_WORDS = WALK ? WalkWindow<TX>::BYTES / 4 : 0;
     __shared__ uint32_t s_cov[COV > WALK_WORDS ? COV : WALK_WORDS];
     const uint8_t* s_g = reinterpret_cast<const uint8_t*>(s_g32);
 
@@ -551,10 +549,24 @@ __global__ __launch_bounds__(256, 3) void kf_smooth(const DevItem* __restrict__ 
         uint32_t cov[MW];
 #pragma unroll
         for (int r = 0; r < MW; r++) cov[r] = C[PITCH * r];
-        C[PITCH * MW] = coverage_info(cov, S);
+        const uint32_t info = coverage_info(cov, S);
+        if constexpr (S <= kMaxCellScale) {
+            uint32_t word[RW] = {};
+            cell_mask_rows<S>([&](int r) { return cov[r]; },
+                              [&](int j, int ky, uint32_t bits) {
+                                  const int at = S <= kMaxCellScale16 ? 16 * j + ky * S : 8 * (j * S + ky);
+                                  word[at / 32] |= bits << (at % 32);
+                              });
+            constexpr int at = S <= kMaxCellScale16 ? 16 * 9 : 8 * 9 * S;
+            word[at / 32] |= (info & 0xFFu) << (at % 32);
+#pragma unroll
+            for (int r = 0; r < RW; r++) C[PITCH * r] = word[r];
+        } else {
+            C[PITCH * MW] = info;
+        }
     }
     __syncthreads();
-    // the rows of a cell by adjacent lanes
+    // the words of a cell by adjacent lanes
     uint32_t* dst = rows + it.rows_off / 4;
     for (int k = t; k < nlist * RW; k += 256) {
         const int c = k / RW, r = k - c * RW, own = s_list[c];
@@ -600,9 +612,9 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     constexpr int PX_WORDS = 2048, PX_CELLS = PX_WORDS / (S * S), PX_CODE_CELLS = PX_WORDS / (S * ROW_WORDS);
     static_assert(PX_CELLS >= 1, "at least one buffered cell");
     __shared__ uint32_t s_px[PX_WORDS];
-    // 3x to 7x: the winners of listed cells' pixels, as two words a cell up to
+    // the winners of listed cells' pixels, as two words a cell up to
     // 4x, a word a row from 5x (tiles that do not keep them in s_px)
-    constexpr bool MASKS = !SUB && S >= 3 && S <= kMaxCellScale;
+    constexpr bool MASKS = SUB ? S <= kMaxCellScale : S >= 3 && S <= 7;
     __shared__ uint32_t s_plane[!MASKS ? 1 : S <= kMaxCellScale16 ? 2 * RTX * RTY : PX_CELLS * S];
     __shared__ uint16_t s_idx[RTX * RTY];  // list index of a listed own cell, else kOwnColour
     constexpr uint32_t kOwnColour = 0xFFFF;  // the cell shows its own colour only
@@ -677,7 +689,8 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
                 uint32_t src = 0xFFFFFFFFu;
                 if ((key & 0xFFu) != 90) {
                     src = (uint32_t)(it.rows_off / 4) + ((uint32_t)y * (uint32_t)it.W + (uint32_t)x) * RW;
-                    info = (uint8_t)(cell_rows[src + MW] & 0x1Fu);
+                    constexpr int at = S > kMaxCellScale ? 32 * MW : S <= kMaxCellScale16 ? 16 * 9 : 8 * 9 * S;
+                    info = (uint8_t)((cell_rows[src + at / 32] >> (at % 32)) & 0x1Fu);
                 } else {
                     info = (uint8_t)(info_table[key] & 0x1Fu);
                 }
@@ -842,7 +855,7 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     };
 
     if constexpr (MASKS) {
-        // 3x to 7x: a listed cell's winners are picked for all its pixels at
+        // 3x to 7x, with subdivision 1x to 8x: a listed cell's winners are picked for all its pixels at
         // once, from nine independent loads of the cell-mask table: one thread
         // a cell up to 4x, two (four rows each) from 5x.  A tile that keeps
         // winners is then resolved, else one thread per row of a listed cell
@@ -852,7 +865,9 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
         // 128 indexed frames 141 -> 133; at 6x, 4096 sprites 129 -> 120, 8
         // frames of 640x480 97 -> 83.  At 8x the stores bound the batch
         // either way, and the rows, spread over more threads, keep them
-        // flowing (16 frames of 640x480: 256 us against 264).
+        // flowing (16 frames of 640x480: 256 us against 264).  With
+        // subdivision kf_smooth writes masks too, and 16 frames of 640x480
+        // take 644 -> 617 us at 8x, 501 -> 476 at 6x and 336 -> 292 at 4x.
         constexpr int TB = S <= kMaxCellScale16 ? 2 : 4;  // bytes of a thread's masks
         constexpr int PARTS = S <= kMaxCellScale16 ? 1 : 2;
         const uint8_t* cell_table = reinterpret_cast<const uint8_t*>(mask_table + kKeys * MW);
@@ -863,9 +878,17 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
             uint32_t m[9];
 #pragma unroll
             for (int j = 0; j < 9; j++) {
-                const uint32_t key = s_key[(uy + 2 - j / 3) * RCX + (ux + 2 - j % 3)];
+                const int k = (uy + 2 - j / 3) * RCX + (ux + 2 - j % 3);
+                const uint32_t key = s_key[k];
                 m[j] = 0;
-                if (key != kNoCell) __builtin_memcpy(&m[j], cell_table + ((key * 9 + j) * PARTS + h) * TB, TB);
+                if (key != kNoCell) {
+                    const uint8_t* src = cell_table + ((key * 9 + j) * PARTS + h) * TB;
+                    if constexpr (SUB) {
+                        if (s_src[k] != 0xFFFFFFFFu)
+                            src = reinterpret_cast<const uint8_t*>(cell_rows + s_src[k]) + j * (PARTS == 1 ? 2 : S) + 4 * h;
+                    }
+                    __builtin_memcpy(&m[j], src, TB);
+                }
             }
             uint32_t seen = 0;
 #pragma unroll

@@ -23,11 +23,15 @@ constexpr size_t kPaletteBytes = 1024;
 // Returns DPX_ENODEV when the process sees no GPU.
 int require_device();
 
-// Sizes a context's cell-row buffer (subdivided items) to at least `bytes`.
+// Sizes a context's cell coverage buffer (subdivided items) to at least `bytes`.
 int context_reserve_rows(dpx_context* ctx, size_t bytes);
 
-// Cell-row words per cell at scale S: 2S + 2 sample rows and a summary.
-constexpr size_t cell_row_words(int S) { return 2 * (size_t)S + 3; }
+// Coverage words per cell at scale S: nine cell masks of 2 bytes (up to 4x) or
+// S bytes (up to 8x), or 2S + 2 sample rows, and a summary.
+constexpr size_t cell_row_words(int S)
+{
+    return S <= 4 ? 5 : S <= 8 ? (9 * (size_t)S + 1 + 3) / 4 : 2 * (size_t)S + 3;
+}
 
 }  // namespace dpx
 

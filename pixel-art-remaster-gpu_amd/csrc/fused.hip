@@ -10,7 +10,7 @@
 //              (and, with subdivision, hulls, smoothed polygons and their
 //              coverage) in LDS; cells whose S*S pixels are all their own
 //              colour are simple, the rest are listed and resolved row by
-//              row (1x to 7x: cell by cell) against the 3x3 candidate cells
+//              row (up to 7x: cell by cell) against the 3x3 candidate cells
 //              in draw order into an LDS pixel buffer; then every row of
 //              the tile's output is stored once, simple and resolved pixels
 //              by the same store instructions.
@@ -20,7 +20,7 @@
 // bitmasks (kt_mask): bit b of row r of key k says whether sample
 // (kmin+b, kmin+r) of the cell's local sample grid is covered, kmin =
 // -(S/2)-1, MW = 2S+2 rows and columns (local [-0.5, 1.5] of the cell); into
-// a 16-bit summary per key (kt_info, coverage_info); and at 1x to 7x into
+// a 16-bit summary per key (kt_info, coverage_info); and at 1x to 8x into
 // each key's sample mask of each neighbour cell (kt_cell).
 //
 // With subdivision, kf_smooth runs between the two: it resolves the
@@ -84,7 +84,7 @@ __global__ void kt_mask(int S, uint32_t* __restrict__ mask)
 }
 
 
-// The keys' cell masks (cell_masks), after the row table in the same
+// The keys' cell masks (cell_mask_rows), after the row table in the same
 // allocation: entry key * 9 + j.
 template <int S>
 __global__ void kt_cell(const uint32_t* __restrict__ mask, uint8_t* __restrict__ cell)
@@ -93,15 +93,17 @@ __global__ void kt_cell(const uint32_t* __restrict__ mask, uint8_t* __restrict__
     const int key = blockIdx.x * blockDim.x + threadIdx.x;
     if (key >= kKeys) return;
     const uint32_t* rows = mask + (size_t)key * mask_w(S);
-    cell_masks<S>([&](int r) { return rows[r]; },
-                  [&](int j, CellMask<S> m) { __builtin_memcpy(cell + (size_t)(key * 9 + j) * TB, &m, TB); });
+    uint64_t m[9] = {};
+    cell_mask_rows<S>([&](int r) { return rows[r]; },
+                      [&](int j, int ky, uint32_t bits) { m[j] |= (uint64_t)bits << (ky * (TB == 2 ? S : 8)); });
+    for (int j = 0; j < 9; j++) __builtin_memcpy(cell + (size_t)(key * 9 + j) * TB, &m[j], TB);
 }
 
 using CellFn = void (*)(const uint32_t*, uint8_t*);
 inline CellFn pick_cell_table(int S)
 {
     static constexpr CellFn fns[kMaxCellScale + 1] = { nullptr,    kt_cell<1>, kt_cell<2>, kt_cell<3>, kt_cell<4>,
-                                                       kt_cell<5>, kt_cell<6>, kt_cell<7> };
+                                                       kt_cell<5>, kt_cell<6>, kt_cell<7>, kt_cell<8> };
     return S <= kMaxCellScale ? fns[S] : nullptr;
 }
 
@@ -885,7 +887,7 @@ static int make_dev_item(const dpx_item& a, int k, const uint8_t* d_out, uint64_
               kMaxScale);
     DPX_CHECK(a.out_stride >= 4 * a.width * a.scale && a.out_stride % 4 == 0 && a.out_offset % 4 == 0, DPX_EINVAL,
               "item %d: output layout (stride %d, offset %llu)", k, a.out_stride, (unsigned long long)a.out_offset);
-    DPX_CHECK(!a.subdivide || (uint64_t)a.width * a.height * rows_words(a.scale) < ((uint64_t)1 << 32), DPX_EINVAL,
+    DPX_CHECK(!a.subdivide || (uint64_t)a.width * a.height * (2 * a.scale + 3) < ((uint64_t)1 << 32), DPX_EINVAL,
               "item %d: %dx%d at scale %d with subdivision exceeds 2^32 cell-row words", k, a.width, a.height, a.scale);
     memset(&d, 0, sizeof(d));
     d.in_off = a.in_offset;
@@ -1327,7 +1329,7 @@ extern "C" int dpx_batch_timing_read(dpx_context* ctx, dpx_batch_times* out)
 // caller's input and output in one static device array, `scratch`, so that a
 // call allocates nothing.  Layout (all offsets 256-byte aligned):
 //   tables     per scale 1..15 the coverage rows (with the cell masks at 1x to
-//              7x) and the coverage summaries, built on the first call
+//              8x) and the coverage summaries, built on the first call
 //              on each device;
 //   items      the batch's device items, in item order and grouped by
 //              (scale, subdivision);

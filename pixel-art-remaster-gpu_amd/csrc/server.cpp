@@ -461,7 +461,7 @@ extern "C" int dpx_server_open_stream(dpx_server* srv, int width, int height, in
         if (int rc = dpx_context_reserve(lane.ctx, items, std::max(pixels, srv->reserved_pixels.load()),
                                          params->scale))
             return rc;
-        // subdivided frames also need cell rows (a word per sample row and one more per cell)
+        // subdivided frames also need the cells' coverage
         if (params->subdivide)
             if (int rc = context_reserve_rows(lane.ctx, (size_t)items * align256((size_t)pixels * 4 *
                                                                                  cell_row_words(params->scale))))
