@@ -23,6 +23,10 @@ constexpr size_t kPaletteBytes = 1024;
 // Returns DPX_ENODEV when the process sees no GPU.
 int require_device();
 
+// hipMemcpy from the device to host memory that need not be pinned, for
+// results of megabytes.
+hipError_t download(void* dst, const void* src, size_t n);
+
 // Sizes a context's cell coverage buffer (subdivided items) to at least `bytes`.
 int context_reserve_rows(dpx_context* ctx, size_t bytes);
 

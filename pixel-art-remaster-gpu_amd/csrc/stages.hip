@@ -1151,21 +1151,14 @@ extern "C" int dpx_stage_components(const uint8_t* d_graph, int W, int H, int32_
 // -------------------------------------------------------------------------
 namespace {
 
+// A frame's device buffers, in one allocation: each hipMalloc and hipFree
+// takes the driver's time, seven of them longer than the kernels.
 struct FrameBuffers {
     uint8_t *img = nullptr, *graph = nullptr, *graph_aux = nullptr, *out = nullptr;
-    dpx_point *diagram = nullptr, *diagram_aux = nullptr, *pos = nullptr;
+    dpx_point *diagram = nullptr, *diagram_aux = nullptr;
     int32_t *ec = nullptr, *ec_aux = nullptr;
-    ~FrameBuffers()
-    {
-        (void)hipFree(img);
-        (void)hipFree(graph);
-        (void)hipFree(graph_aux);
-        (void)hipFree(out);
-        (void)hipFree(diagram);
-        (void)hipFree(diagram_aux);
-        (void)hipFree(ec);
-        (void)hipFree(ec_aux);
-    }
+    uint8_t* all = nullptr;
+    ~FrameBuffers() { (void)hipFree(all); }
 };
 
 // Runs the stages up to triangulation on a frame already in fb.img.
@@ -1187,18 +1180,28 @@ int run_stages(FrameBuffers& fb, int W, int H, int stride, int ch, uint32_t flag
     return DPX_OK;
 }
 
-int alloc_frame(FrameBuffers& fb, int W, int H, int stride, bool subdivide)
+int alloc_frame(FrameBuffers& fb, int W, int H, int stride, bool subdivide, size_t out_bytes)
 {
-    size_t N = (size_t)W * H;
-    DPX_HIP(hipMalloc(&fb.img, (size_t)stride * H));
-    DPX_HIP(hipMalloc(&fb.graph, N));
-    DPX_HIP(hipMalloc(&fb.graph_aux, N));
-    DPX_HIP(hipMalloc(&fb.diagram, N * dpx::kCellSize * sizeof(dpx_point)));
-    DPX_HIP(hipMalloc(&fb.ec, N * sizeof(int32_t)));
-    if (subdivide) {
-        DPX_HIP(hipMalloc(&fb.diagram_aux, N * dpx::kCellSize * sizeof(dpx_point)));
-        DPX_HIP(hipMalloc(&fb.ec_aux, N * sizeof(int32_t)));
-    }
+    const size_t N = (size_t)W * H;
+    size_t bytes = 0;
+    auto place = [&](size_t n) {
+        const size_t at = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return at;
+    };
+    const size_t img = place((size_t)stride * H), graph = place(N), graph_aux = place(N);
+    const size_t diagram = place(N * dpx::kCellSize * sizeof(dpx_point)), ec = place(N * sizeof(int32_t));
+    const size_t diagram_aux = place(subdivide ? N * dpx::kCellSize * sizeof(dpx_point) : 0);
+    const size_t ec_aux = place(subdivide ? N * sizeof(int32_t) : 0), out = place(out_bytes);
+    DPX_HIP(hipMalloc(&fb.all, bytes));
+    fb.img = fb.all + img;
+    fb.graph = fb.all + graph;
+    fb.graph_aux = fb.all + graph_aux;
+    fb.diagram = reinterpret_cast<dpx_point*>(fb.all + diagram);
+    fb.ec = reinterpret_cast<int32_t*>(fb.all + ec);
+    fb.diagram_aux = reinterpret_cast<dpx_point*>(fb.all + diagram_aux);
+    fb.ec_aux = reinterpret_cast<int32_t*>(fb.all + ec_aux);
+    fb.out = fb.all + out;
     return DPX_OK;
 }
 
@@ -1221,21 +1224,19 @@ extern "C" int dpx_frame(const uint8_t* img, int W, int H, int stride, int ch, c
     }
     size_t N = (size_t)W * H;
     FrameBuffers fb;
-    if (int rc = alloc_frame(fb, W, H, stride, sub)) return rc;
+    if (int rc = alloc_frame(fb, W, H, stride, sub, out_rgba ? (size_t)out_stride * H * scale : 0)) return rc;
     DPX_HIP(hipMemcpy(fb.img, img, (size_t)stride * H, hipMemcpyHostToDevice));
     if (int rc = run_stages(fb, W, H, stride, ch, params->flags, sub)) return rc;
     if (out_rgba) {
-        DPX_HIP(hipMalloc(&fb.out, (size_t)out_stride * H * scale));
         if (int rc = dpx_stage_rasterize(fb.img, W, H, stride, ch, params->flags, fb.diagram, fb.ec, scale, fb.out,
                                          out_stride, nullptr))
             return rc;
     }
     DPX_HIP(hipDeviceSynchronize());
-    if (out_rgba) DPX_HIP(hipMemcpy(out_rgba, fb.out, (size_t)out_stride * H * scale, hipMemcpyDeviceToHost));
+    if (out_rgba) DPX_HIP(download(out_rgba, fb.out, (size_t)out_stride * H * scale));
     if (graph_out) DPX_HIP(hipMemcpy(graph_out, fb.graph, N, hipMemcpyDeviceToHost));
     if (edge_count_out) DPX_HIP(hipMemcpy(edge_count_out, fb.ec, N * sizeof(int32_t), hipMemcpyDeviceToHost));
-    if (diagram_out)
-        DPX_HIP(hipMemcpy(diagram_out, fb.diagram, N * kCellSize * sizeof(dpx_point), hipMemcpyDeviceToHost));
+    if (diagram_out) DPX_HIP(download(diagram_out, fb.diagram, N * kCellSize * sizeof(dpx_point)));
     return DPX_OK;
 }
 
@@ -1249,7 +1250,7 @@ extern "C" dpx_point* launch_kernel(dpx_point* pos, dpx_uchar4* colorPos, float 
     if (check_img(img_data, W, H, img_widthstep, 3, 0) || require_device()) return nullptr;
     size_t N = (size_t)W * H;
     FrameBuffers fb;
-    if (alloc_frame(fb, W, H, img_widthstep, subdivide)) return nullptr;
+    if (alloc_frame(fb, W, H, img_widthstep, subdivide, 0)) return nullptr;
     if (hipMemcpy(fb.img, img_data, (size_t)img_widthstep * H, hipMemcpyHostToDevice) != hipSuccess) {
         fail(DPX_EHIP, "image upload failed");
         return nullptr;
@@ -1271,7 +1272,7 @@ extern "C" dpx_point* launch_kernel(dpx_point* pos, dpx_uchar4* colorPos, float 
     bool ok = true;
     if (edge_count_h)
         ok = ok && hipMemcpy(edge_count_h, fb.ec, N * sizeof(int32_t), hipMemcpyDeviceToHost) == hipSuccess;
-    ok = ok && hipMemcpy(diagram_h, fb.diagram, N * kCellSize * sizeof(dpx_point), hipMemcpyDeviceToHost) == hipSuccess;
+    ok = ok && download(diagram_h, fb.diagram, N * kCellSize * sizeof(dpx_point)) == hipSuccess;
     if (graph_h) ok = ok && hipMemcpy(graph_h, fb.graph, N, hipMemcpyDeviceToHost) == hipSuccess;
     if (!ok) {
         free(diagram_h);

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import weakref
 from ctypes import POINTER, c_bool, c_char_p, c_double, c_float, c_int, c_uint32, c_uint64, c_void_p
 
 import numpy as np
@@ -243,10 +244,12 @@ def launch_kernel(img: np.ndarray, width: int, height: int, subdivide: bool = Fa
                             bool(subdivide))
     if not ptr:
         raise DepixelError(-1, last_error())
+    # the array stands on the library's malloc'd memory (a copy of 360 bytes a
+    # pixel took as long as the frame) and frees it with its last view
     n = width * height * CELL_SIZE * 2
-    diag = np.ctypeslib.as_array(ctypes.cast(ptr, POINTER(c_float)), shape=(n,)).copy().reshape(-1, 2)
-    libc.free(ptr)
-    return diag, ec, graph
+    mem = (c_float * n).from_address(ptr)
+    weakref.finalize(mem, libc.free, ptr).atexit = False
+    return np.frombuffer(mem, dtype=np.float32).reshape(-1, 2), ec, graph
 
 
 # --------------------------------------------------------------------------
