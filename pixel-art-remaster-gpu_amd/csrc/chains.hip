@@ -43,8 +43,8 @@
 // the ranking's launches in front of them; bytes and arithmetic are small
 // (640x480: 272 k links of 12 B).  Measured, against one wave that took the
 // walks in scan order (a microsecond a walk): dithered 640x480 frames 6.3 ->
-// 0.61 ms, those with a face of thousands of abandoned walks 9-13 -> 3.3-3.9
-// ms; 256x224 game frames 0.61-1.64 -> 0.31-0.82 ms; 64x48 0.29 -> 0.17 ms.
+// 0.55 ms, those with a face of thousands of abandoned walks 9-13 -> 3.3-3.9
+// ms; 256x224 game frames 0.61-1.64 -> 0.30-0.81 ms; 64x48 0.29 -> 0.16 ms.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -779,15 +779,22 @@ __device__ inline bool short_waits(const Bc& b, int p)
 // of the others, whose first rounds change what it sees, so it waits for
 // some of them: rounds 0, 1, 4 and 7, then whenever no short path waits
 // (640x480: 2-3 evaluations in place of 7-9).
-constexpr int kChunk = 8;
+// A wave evaluates the paths of its chunk one after another, 4 us each and
+// more: with chunks of 8 a round of a 640x480 frame took 38 us, of 2 it takes
+// 11 to 31 (of 1: no better, twice the waves).  Rounds without long paths need
+// no LDS and fill the machine.
+constexpr int kChunk = 2;
 constexpr bool long_round(int r) { return r <= 1 || r % 3 == 1; }
+template <bool LONG>
 __global__ __launch_bounds__(kSimBlock) void k_bc_sim(Bc b, int r, int slot)
 {
-    __shared__ LongLds s;
     if (b.ctr[kStatus] != 0) return;
-    const int n_long = slot < 0 ? 0 : slot == 0 ? b.ctr[kLongs] : b.ctr[kWaitingLong + slot];
-    for (int k = blockIdx.x; k < n_long; k += gridDim.x)
-        sim_path_long<kSimBlock>(b, slot == 0 ? b.longs[k] : b.dlong[k], s, NoteFlag{});
+    if constexpr (LONG) {
+        __shared__ LongLds s;
+        const int n_long = slot == 0 ? b.ctr[kLongs] : b.ctr[kWaitingLong + slot];
+        for (int k = blockIdx.x; k < n_long; k += gridDim.x)
+            sim_path_long<kSimBlock>(b, slot == 0 ? b.longs[k] : b.dlong[k], s, NoteFlag{});
+    }
     if (r > 0 && b.ctr[kWaiting + r] == 0) return;
     constexpr int WAVES = kSimBlock / 64;
     const int n = b.ctr[kPaths], lane = threadIdx.x & 63;
@@ -1094,7 +1101,8 @@ extern "C" int dpx_stage_border_chains(const uint8_t* d_graph, int W, int H, uin
     hipLaunchKernelGGL(k_bc_sort, dim3((unsigned)std::min<size_t>(E / kShort + 1, 256)), dim3(kSortBlock), 0, s, b);
     int slot = 0;  // of the long paths that wait
     for (int r = 0; r < kGridRounds; r++) {
-        hipLaunchKernelGGL(k_bc_sim, sims, dim3(kSimBlock), 0, s, b, r, long_round(r) ? slot++ : -1);
+        if (long_round(r)) hipLaunchKernelGGL(k_bc_sim<true>, sims, dim3(kSimBlock), 0, s, b, r, slot++);
+        else hipLaunchKernelGGL(k_bc_sim<false>, sims, dim3(kSimBlock), 0, s, b, r, -1);
         hipLaunchKernelGGL(k_bc_spread, per_node, dim3(256), 0, s, b, r, slot);
     }
     hipLaunchKernelGGL(k_bc_finish, dim3(1), dim3(kFinishBlock), 0, s, b, slot);
