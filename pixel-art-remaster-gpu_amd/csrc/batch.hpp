@@ -400,12 +400,19 @@ __device__ inline void tile_resolved_load(const DevItem& it, const uint8_t* __re
 // triangles cut so far are the cell), runs for the few polygons for which
 // that is not plain, gathered into the first lanes.  The cells are listed by
 // the size of their hull, so that the lanes of a wave end together.  16 frames
-// of 640x480 at 8x: 335 us (606 with every row of every edge visited, every
+// of 640x480 at 8x: 290 us (606 with every row of every edge visited, every
 // cell clipped, and hulls and colours read per vertex); 64 of 251x223 at 4x:
-// 145 (334).
+// 128 (334).
 // ---------------------------------------------------------------------------
+// Blocks a CU, for which the registers are allotted: as many as their LDS
+// leaves room for (a wave waits for two thirds of its time, most of it at
+// barriers).  One block more than before takes 16 frames of 640x480 at 8x from
+// 616 to 566 us a batch, at 6x 477 to 449 and at 4x 291 to 275, 64 of 251x223
+// at 4x 235 to 220; 8 blocks at 4x spill: 233.
+constexpr int smooth_blocks(int S, bool walk) { return walk ? 3 : S <= 4 ? 7 : S <= 6 ? 6 : S <= 8 ? 5 : 3; }
+
 template <int S, int TX, bool WALK>
-__global__ __launch_bounds__(256, 3) void kf_smooth(const DevItem* __restrict__ items, const uint2* __restrict__ tile_map,
+__global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const DevItem* __restrict__ items, const uint2* __restrict__ tile_map,
                                                  int grid3d, const uint8_t* __restrict__ in,
                                                  const uint8_t* __restrict__ gaux, uint8_t* __restrict__ gfin,
                                                  uint32_t* __restrict__ rows)
@@ -413,12 +420,8 @@ __global__ __launch_bounds__(256, 3) void kf_smooth(const DevItem* __restrict__ 
     DPX_TILE_NAMES(TX);
     constexpr int MW = mask_w(S), KMIN = mask_kmin(S), RW = rows_words(S);
     constexpr int PITCH = 257;  // of the rows: adjacent rows of a cell in adjacent banks
-    __shared__ uint32_t s_aux32[AY * RWW];
-    __shared__ uint32_t s_p32[(GY + 1) * RWW];
-    __shared__ uint16_t s_blk[(GY + 1) * RDB];
     __shared__ int s_nblk;
     __shared__ uint32_t s_g32[GY * RWW];
-    __shared__ HullBits s_hull[RCX * RCY];
     __shared__ uint16_t s_list[RTX * RTY];
     __shared__ int s_bin[16];  // own cells to smooth per hull size
     __shared__ int s_nlist, s_nclip;
@@ -429,7 +432,18 @@ __global__ __launch_bounds__(256, 3) void kf_smooth(const DevItem* __restrict__ 
     __shared__ uint16_t s_poly[16 * 256];
     // sample row r of column t at [r * PITCH + t], then its masks and summary; first the walk window
     constexpr int COV = (MW + 1) * PITCH, WALK_WORDS = WALK ? WalkWindow<TX>::BYTES / 4 : 0;
-    __shared__ uint32_t s_cov[COV > WALK_WORDS ? COV : WALK_WORDS];
+    // What is needed until the polygons are made lies where the rows come
+    // after them (the walk window is read meanwhile and keeps it apart): a
+    // block more fits each CU.
+    constexpr int HULL_WORDS = RCX * RCY * (int)(sizeof(HullBits) / 4), AUX_WORDS = AY * RWW, P_WORDS = (GY + 1) * RWW;
+    constexpr int EARLY = HULL_WORDS + AUX_WORDS + P_WORDS + ((GY + 1) * RDB + 1) / 2;
+    constexpr int LATE = COV > WALK_WORDS ? COV : WALK_WORDS;
+    __shared__ __align__(8) uint32_t s_cov[WALK ? LATE + EARLY + 1 : LATE > EARLY ? LATE : EARLY];
+    uint32_t* s_early = s_cov + (WALK ? (LATE + 1) / 2 * 2 : 0);
+    HullBits* s_hull = reinterpret_cast<HullBits*>(s_early);
+    uint32_t* s_aux32 = s_early + HULL_WORDS;
+    uint32_t* s_p32 = s_aux32 + AUX_WORDS;
+    uint16_t* s_blk = reinterpret_cast<uint16_t*>(s_p32 + P_WORDS);
     const uint8_t* s_g = reinterpret_cast<const uint8_t*>(s_g32);
 
     const int t = threadIdx.x;
@@ -504,6 +518,9 @@ __global__ __launch_bounds__(256, 3) void kf_smooth(const DevItem* __restrict__ 
             P[256 * m] = (uint16_t)(((uint32_t)px & 0xFFu) | ((uint32_t)py << 8));
             m++;
         });
+    }
+    __syncthreads();
+    if (t < nlist) {
 #pragma unroll
         for (int r = 0; r < MW; r++) C[PITCH * r] = 0;
         // seen from its pixel's centre almost every cell goes round once
