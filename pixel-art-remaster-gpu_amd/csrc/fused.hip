@@ -20,7 +20,7 @@
 // bitmasks (kt_mask): bit b of row r of key k says whether sample
 // (kmin+b, kmin+r) of the cell's local sample grid is covered, kmin =
 // -(S/2)-1, MW = 2S+2 rows and columns (local [-0.5, 1.5] of the cell); into
-// a 16-bit summary per key (kt_info, coverage_info); and at 1x to 8x into
+// a summary byte per key (kt_info, coverage_info's low bits); and at 1x to 8x into
 // each key's sample mask of each neighbour cell (kt_cell).
 //
 // With subdivision, kf_smooth runs between the two: it resolves the
@@ -107,11 +107,11 @@ inline CellFn pick_cell_table(int S)
     return S <= kMaxCellScale ? fns[S] : nullptr;
 }
 
-__global__ void kt_info(const uint32_t* __restrict__ mask, int S, uint16_t* __restrict__ info)
+__global__ void kt_info(const uint32_t* __restrict__ mask, int S, uint8_t* __restrict__ info)
 {
     int key = blockIdx.x * blockDim.x + threadIdx.x;
     if (key >= kKeys) return;
-    info[key] = (uint16_t)coverage_info(mask + (size_t)key * mask_w(S), S);
+    info[key] = (uint8_t)coverage_info(mask + (size_t)key * mask_w(S), S);
 }
 
 
@@ -504,7 +504,7 @@ struct dpx_context {
     BatchPlan plan;
     int device = 0;
     uint32_t* d_mask[dpx::kMaxScale + 1] = {};
-    uint16_t* d_info[dpx::kMaxScale + 1] = {};
+    uint8_t* d_info[dpx::kMaxScale + 1] = {};
     uint8_t *d_gaux = nullptr, *d_gfin = nullptr;
     size_t g_cap = 0;
     uint32_t* d_rows = nullptr;  // cell rows of smoothed cells (kf_smooth)
@@ -621,7 +621,7 @@ int ensure_mask(dpx_context* ctx, int S)
     size_t n = (size_t)kKeys * mask_w(S);
     const size_t cell_bytes = cell_table_bytes(S);
     if (!ctx->d_mask[S]) DPX_HIP(hipMalloc(&ctx->d_mask[S], n * sizeof(uint32_t) + cell_bytes));
-    if (!ctx->d_info[S]) DPX_HIP(hipMalloc(&ctx->d_info[S], kKeys * sizeof(uint16_t)));
+    if (!ctx->d_info[S]) DPX_HIP(hipMalloc(&ctx->d_info[S], kKeys));
     hipLaunchKernelGGL(kt_mask, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, S, ctx->d_mask[S]);
     if (cell_bytes)
         hipLaunchKernelGGL(pick_cell_table(S), dim3(kKeys / 256), dim3(256), 0, 0, ctx->d_mask[S],
@@ -1129,7 +1129,7 @@ struct NodeArgs {
     const uint32_t* rows_c;
     uint32_t* rows;
     const uint32_t* mask;
-    const uint16_t* info;
+    const uint8_t* info;
     uint8_t* out;
     void* ptrs[10];
 };
@@ -1346,7 +1346,7 @@ constexpr size_t na_mask_bytes(int S)
 {
     return na_align((size_t)kKeys * mask_w(S) * 4 + cell_table_bytes(S));
 }
-constexpr size_t na_info_bytes() { return na_align((size_t)kKeys * 2); }
+constexpr size_t na_info_bytes() { return na_align((size_t)kKeys); }
 constexpr size_t na_mask_off(int S)
 {
     size_t o = 0;
@@ -1432,7 +1432,7 @@ int na_setup(int dev, hipStream_t stream, uint8_t** out)
                 hipLaunchKernelGGL(pick_cell_table(S), dim3(kKeys / 256), dim3(256), 0, stream, mask,
                                    reinterpret_cast<uint8_t*>(mask + n));
             hipLaunchKernelGGL(kt_info, dim3(kKeys / 256), dim3(256), 0, stream, mask, S,
-                               reinterpret_cast<uint16_t*>(ptr + na_info_off(S)));
+                               ptr + na_info_off(S));
         }
         DPX_HIP(hipGetLastError());
         DPX_HIP(hipStreamSynchronize(stream));
@@ -1537,7 +1537,7 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
         hipLaunchKernelGGL(fn, dim3(gtiles[g]), dim3(256), 0, stream, d_gitems + gslot0[g], d_rmap + gtile0[g], 0,
                            d_in, d_graph, nullptr, nullptr,
                            reinterpret_cast<const uint32_t*>(base + na_mask_off(S)),
-                           reinterpret_cast<const uint16_t*>(base + na_info_off(S)), d_out);
+                           base + na_info_off(S), d_out);
     }
     DPX_HIP(hipGetLastError());
     return DPX_OK;
