@@ -180,31 +180,35 @@ constexpr uint16_t kNoCell = 0xFFFF;
 // rows_words(S) of its range.
 __host__ __device__ constexpr int rows_words(int S) { return (int)cell_row_words(S); }
 
-// The snapshot rows ay0 .. ay0 + AY - 1 of a tile's window into LDS.  With
-// W % 4 == 0 the graph rows are word aligned and a word is either wholly
-// inside the frame or wholly outside.
+// The bytes of pixels (x .. x + 3, y) of a graph of the item, 0 where they
+// lie outside the frame (x is a multiple of 4).  One load at any alignment
+// also where the rows are not whole words (byte by byte, 64 smoothed frames of
+// 251x223 took 168 us a batch at 2x, not 161, and 444 at 8x, not 437); it
+// stays inside the item's slot, whose size is rounded up to 256 bytes.
+__device__ inline uint32_t graph_word(const DevItem& it, const uint8_t* __restrict__ g, int x, int y)
+{
+    if ((unsigned)x >= (unsigned)it.W || (unsigned)y >= (unsigned)it.H) return 0u;
+    const uint32_t off = (uint32_t)(y * it.W + x);
+    if (it.graph_w4) return *reinterpret_cast<const uint32_t*>(g + off);
+    const uint32_t at = min(off, (((uint32_t)(it.W * it.H) + 255u) & ~255u) - 4u);
+    uint32_t v;
+    __builtin_memcpy(&v, g + at, 4);
+    v >>= 8u * (off - at);
+    const int n = it.W - x;
+    return n < 4 ? v & ((1u << (8 * n)) - 1u) : v;
+}
+
+
+// The snapshot rows ay0 .. ay0 + AY - 1 of a tile's window into LDS.
 template <int TX>
 __device__ inline void tile_snapshot_load(const DevItem& it, const uint8_t* __restrict__ aux, int x0, int ay0,
                                           uint32_t* s_aux32, int t)
 {
     DPX_TILE_NAMES(TX);
-    if (it.graph_w4) {
-        if (t < AY * RWW) {
-            int r = t / RWW, w = t % RWW;
-            int x = x0 - 8 + 4 * w, y = ay0 + r;
-            uint32_t v = 0;
-            if (w >= 1 && w <= RDW && (unsigned)x < (unsigned)it.W && (unsigned)y < (unsigned)it.H)
-                v = *reinterpret_cast<const uint32_t*>(aux + (uint32_t)(y * it.W + x));
-            s_aux32[t] = v;
-        }
-    } else {
-        uint8_t* s8 = reinterpret_cast<uint8_t*>(s_aux32);
-        for (int k = t; k < AY * RWB; k += 256) {
-            int r = k / RWB, c = k % RWB;
-            int x = x0 - 8 + c, y = ay0 + r;
-            bool ok = c >= 4 && c < 4 + RDB && (unsigned)x < (unsigned)it.W && (unsigned)y < (unsigned)it.H;
-            s8[k] = ok ? aux[(uint32_t)(y * it.W + x)] : 0;
-        }
+    static_assert(AY * RWW <= 256, "a word a thread");
+    if (t < AY * RWW) {
+        const int r = t / RWW, w = t % RWW;
+        s_aux32[t] = w >= 1 && w <= RDW ? graph_word(it, aux, x0 - 8 + 4 * w, ay0 + r) : 0u;
     }
 }
 
@@ -343,12 +347,10 @@ __device__ inline void tile_resolve(const DevItem& it, const uint8_t* __restrict
         // the resolved graph of the tile's own cells, when the caller keeps it
         if (gfin && y >= y0 && y < y0 + RTY && w >= 2 && w <= RDW - 1 && y < it.H && x < it.W) {
             uint8_t* dst = gfin + it.g_off + (uint32_t)(y * it.W + x);
-            if (it.graph_w4) {
-                *reinterpret_cast<uint32_t*>(dst) = res;
-            } else {
-                int n = min(4, it.W - x);
+            const int n = it.W - x;
+            if (n >= 4) __builtin_memcpy(dst, &res, 4);  // (one store at any alignment)
+            else
                 for (int q = 0; q < n; q++) dst[q] = (uint8_t)(res >> (8 * q));
-            }
         }
     }
 }
@@ -360,24 +362,10 @@ __device__ inline void tile_resolved_load(const DevItem& it, const uint8_t* __re
                                           uint32_t* s_g32, int t)
 {
     DPX_TILE_NAMES(TX);
-    const uint8_t* g = gfin + it.g_off;
-    if (it.graph_w4) {
-        if (t < GY * RWW) {
-            int r = t / RWW, w = t % RWW;
-            int x = x0 - 8 + 4 * w, y = y0 - 1 + r;
-            uint32_t v = 0;
-            if (w >= 1 && w <= RDW && (unsigned)x < (unsigned)it.W && (unsigned)y < (unsigned)it.H)
-                v = *reinterpret_cast<const uint32_t*>(g + (uint32_t)(y * it.W + x));
-            s_g32[t] = v;
-        }
-    } else {
-        uint8_t* s8 = reinterpret_cast<uint8_t*>(s_g32);
-        for (int k = t; k < GY * RWB; k += 256) {
-            int r = k / RWB, c = k % RWB;
-            int x = x0 - 8 + c, y = y0 - 1 + r;
-            bool ok = c >= 4 && c < 4 + RDB && (unsigned)x < (unsigned)it.W && (unsigned)y < (unsigned)it.H;
-            s8[k] = ok ? g[(uint32_t)(y * it.W + x)] : 0;
-        }
+    static_assert(GY * RWW <= 256, "a word a thread");
+    if (t < GY * RWW) {
+        const int r = t / RWW, w = t % RWW;
+        s_g32[t] = w >= 1 && w <= RDW ? graph_word(it, gfin + it.g_off, x0 - 8 + 4 * w, y0 - 1 + r) : 0u;
     }
 }
 
