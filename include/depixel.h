@@ -276,7 +276,7 @@ int dpx_batch_timing_read(dpx_context* ctx, dpx_batch_times* out);
  * it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops).  Every buffer beyond d_in and d_out (tables,
  * descriptors, tile maps, the graph snapshot) lives in one static device
- * array of the library, 58 MiB on each GPU it runs on, held until the
+ * array of the library, 60 MiB on each GPU it runs on, held until the
  * process ends.  Limits: at most 4096 items, at most 48 MiB of graph bytes
  * (one per pixel, each item rounded up to 256: e.g. 836 frames of 256x224),
  * at most 65,536 graph tiles (64x32 pixels) and 524,288 raster tiles (32x8);
