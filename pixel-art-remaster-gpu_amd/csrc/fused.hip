@@ -1019,6 +1019,14 @@ struct LaunchArgs {
     uint32_t* rows;  // cell rows of smoothed cells
 };
 
+// Dynamic LDS of a raster launch, which the kernel does not use: at 8x it
+// leaves five blocks a CU in place of eight (as the walk window does by
+// itself).  There the stores bound the batch, and fewer blocks storing at once
+// get more of them through: 4096 sprites 204 -> 189 us a batch, 64 console
+// frames 206 -> 195, 32 of 256x224 at 8x 346 -> 337.  Below 8x fewer blocks
+// are slower (4x by 10%), above it neither way holds for all content.
+constexpr unsigned raster_pad(int S, bool sub, bool walk) { return S == 8 && !sub && !walk ? 10 * 1024 : 0; }
+
 static int launch_plan(dpx_context* ctx, const BatchPlan& plan, const LaunchArgs& la, const uint8_t* d_in,
                        uint8_t* d_out, hipStream_t stream, hipEvent_t ev_mid)
 {
@@ -1037,7 +1045,8 @@ static int launch_plan(dpx_context* ctx, const BatchPlan& plan, const LaunchArgs
             hipLaunchKernelGGL(sf, pg.grid, dim3(256), 0, stream, d_gitems, d_rmap, pg.grid3d, d_in, la.gaux, la.gfin,
                                la.rows);
         }
-        hipLaunchKernelGGL(fn, pg.grid, dim3(256), 0, stream, d_gitems, d_rmap, pg.grid3d, d_in, la.gaux,
+        hipLaunchKernelGGL(fn, pg.grid, dim3(256), raster_pad(pg.scale, pg.sub, pg.walk), stream, d_gitems, d_rmap,
+                           pg.grid3d, d_in, la.gaux,
                            (pg.sub || la.keep) ? la.gfin : nullptr, la.rows, ctx->d_mask[pg.scale],
                            ctx->d_info[pg.scale], d_out);
     }
@@ -1171,6 +1180,7 @@ hipKernelNodeParams node_params(dpx_plan* p, int kind, int group, const uint8_t*
             void* v[10] = { &a.items, &a.map, &a.g3d, &a.in, &a.gaux_c, &a.gfin, &a.rows_c, &a.mask, &a.info, &a.out };
             memcpy(a.ptrs, v, sizeof(v));
             np.func = reinterpret_cast<void*>(pick_raster(pg.scale, pg.sub, pg.tx, pg.walk));
+            np.sharedMemBytes = raster_pad(pg.scale, pg.sub, pg.walk);
         }
         np.gridDim = pg.grid;
     }
@@ -1534,7 +1544,7 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
         const int S = g / 2;
         RasterFn fn = pick_raster(S, g % 2, kNaTX);
         DPX_CHECK(fn, DPX_EINVAL, "no raster kernel for scale %d", S);
-        hipLaunchKernelGGL(fn, dim3(gtiles[g]), dim3(256), 0, stream, d_gitems + gslot0[g], d_rmap + gtile0[g], 0,
+        hipLaunchKernelGGL(fn, dim3(gtiles[g]), dim3(256), raster_pad(S, g % 2, false), stream, d_gitems + gslot0[g], d_rmap + gtile0[g], 0,
                            d_in, d_graph, nullptr, nullptr,
                            reinterpret_cast<const uint32_t*>(base + na_mask_off(S)),
                            base + na_info_off(S), d_out);
