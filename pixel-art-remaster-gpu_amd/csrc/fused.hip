@@ -1544,8 +1544,8 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
         const int S = g / 2;
         RasterFn fn = pick_raster(S, g % 2, kNaTX);
         DPX_CHECK(fn, DPX_EINVAL, "no raster kernel for scale %d", S);
-        hipLaunchKernelGGL(fn, dim3(gtiles[g]), dim3(256), raster_pad(S, g % 2, false), stream, d_gitems + gslot0[g], d_rmap + gtile0[g], 0,
-                           d_in, d_graph, nullptr, nullptr,
+        hipLaunchKernelGGL(fn, dim3(gtiles[g]), dim3(256), raster_pad(S, g % 2, false), stream,
+                           d_gitems + gslot0[g], d_rmap + gtile0[g], 0, d_in, d_graph, nullptr, nullptr,
                            reinterpret_cast<const uint32_t*>(base + na_mask_off(S)),
                            base + na_info_off(S), d_out);
     }
