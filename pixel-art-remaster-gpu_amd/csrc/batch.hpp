@@ -12,6 +12,7 @@
 #include "graph.hpp"
 #include "hull_table.hpp"
 #include "pixel.hpp"
+#include "strips.hpp"
 
 namespace dpx {
 
@@ -652,8 +653,9 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     {
         // a colour is one 4-byte load at any alignment, through a descriptor
         // of the item's rows that answers 0 past their end (the cells outside
-        // the frame, whose colours nothing reads); only the last pixel of a
-        // frame of 3-byte pixels is read by bytes.  Three or four byte loads
+        // the frame, whose colours nothing reads); the last pixel of a frame
+        // of 3-byte pixels, whose word would end past the item, is read by
+        // bytes instead (see word_crosses).  Three or four byte loads
         // a colour, each tested for the frame: 1024 frames of 256x224 at 4x
         // 836 us a batch against 799, 64 console frames 75.9 against 71.6.
         const uint32_t in_end = (uint32_t)(it.H - 1) * (uint32_t)it.stride + (uint32_t)(it.W * it.ch);
@@ -672,12 +674,13 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
             const bool inside = k < RCX * RCY && (unsigned)x < (unsigned)it.W && (unsigned)y < (unsigned)it.H;
             const int row = topdown ? it.H - 1 - y : y;
             // row * stride < 2^31 (checked on the host); the stride itself may exceed 2^24
-            const uint32_t off = inside ? (uint32_t)row * (uint32_t)it.stride + __umul24(x, it.ch) : ~0u;
+            const uint32_t off = (uint32_t)row * (uint32_t)it.stride + __umul24(x, it.ch);
             if (indexed) {
-                c[q] = __builtin_amdgcn_raw_buffer_load_b8(src, (int)off, 0, 0);
+                c[q] = __builtin_amdgcn_raw_buffer_load_b8(src, (int)(inside ? off : ~0u), 0, 0);
             } else {
-                c[q] = __builtin_amdgcn_raw_buffer_load_b32(src, (int)off, 0, 0);
-                if (inside && off + 4 > in_end)
+                const bool last = word_crosses(off, in_end, it.ch);
+                c[q] = __builtin_amdgcn_raw_buffer_load_b32(src, (int)(inside && !last ? off : ~0u), 0, 0);
+                if (inside && last)
                     c[q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(src, (int)off, 0, 0) |
                            (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(src, (int)off + 1, 0, 0) << 8 |
                            (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(src, (int)off + 2, 0, 0) << 16;

@@ -40,6 +40,7 @@
 #include <vector>
 
 #include "batch.hpp"
+#include "strips.hpp"
 
 namespace dpx {
 
@@ -138,49 +139,8 @@ __global__ void kt_info(const uint32_t* __restrict__ mask, int S, uint8_t* __res
 // 169 -> 105 us, 82% of the vector issue rate; 16 of 640x480: 23 -> 15.6 us;
 // 4096 sprites of 8 to 64 pixels: 28 -> 17 us (their tiles were half empty).
 //
-// A strip's outer two lanes are its halo, so a strip yields 62 columns.  62
-// does not divide the widths of frames, so strips do not start over at a
-// frame's edge: an item's rows are cut into blocks of equal height, laid side
-// by side with one empty column before each, and the strips are cut from that
-// row of columns; a strip that holds the end of one block and the start of
-// the next works on both (lanes are independent but for the shift, and the
-// empty column belongs to the outside class).  256x224 in 4 blocks: 17
-// strips, 16.6 of them used.
-// Pixels are loaded kGraphRows rows at a time, one such group ahead (two
-// groups ahead: 109 -> 113 us, for the registers' copies).
-constexpr int kStripCols = 62;
-constexpr int kGraphRows = 4;
-// Rows of a launch's row blocks.  A wave alone takes 0.25 us a row, and each
-// block re-reads two halo rows, so blocks are as tall as leaves about
-// kGraphWaves strips, five waves a SIMD: measured at 2 / 6 / 14 / 30 / 56
-// rows, one 256x224 frame takes 3.7 / 4.7 / 6.0 / 9.2 / 15.1 us, 64 console
-// frames (4.2 Mpixel) 22 / 15.1 / 13.8 / 15.8 / 19.8, 128 of 320x224 59 / 31
-// / 22.6 / 21.1 / 22.9 and 1024 of 256x224 274 / 162 / 119 / 116 / 105.
-// Heights of 4 k + 2 make whole groups with the halo.
-constexpr uint64_t kGraphWaves = 4800;
-constexpr int kGraphMinRows = 2, kGraphMaxRows = 58;
-
-inline int graph_rows(uint64_t pixels)
-{
-    const int rows = (int)std::min<uint64_t>(pixels / (kStripCols * kGraphWaves), kGraphMaxRows);
-    return std::max((rows + 2) / kGraphRows * kGraphRows - 2, kGraphMinRows);
-}
-
-struct GraphSplit {
-    uint32_t blocks, rows, strips;
-};
-
-__host__ __device__ inline GraphSplit graph_split(int W, int H, int max_rows)
-{
-    GraphSplit s;
-    s.blocks = ((uint32_t)H + (uint32_t)max_rows - 1) / (uint32_t)max_rows;
-    s.rows = ((uint32_t)H + s.blocks - 1) / s.blocks;
-    s.blocks = ((uint32_t)H + s.rows - 1) / s.rows;  // (blocks of s.rows rows that hold a row)
-    // columns 1 .. blocks * (W + 1) - 1 of the row of blocks carry pixels
-    s.strips = (s.blocks * ((uint32_t)W + 1) - 1 + kStripCols - 1) / kStripCols;
-    return s;
-}
-
+// The strips are cut as strips.hpp says: 62 columns each (the outer two lanes
+// are halo), several row blocks of an item side by side.
 // One more bit of each lane's byte: v + v + (the lane's bit of m).  m is the
 // result of a scalar operation: a vector compare's result would have to be
 // two wait states old, and the compiler does not look into the block for it.
@@ -264,37 +224,37 @@ __device__ __forceinline__ void graph_strip(const DevItem& it, const GraphSplit 
     const uint32_t lane = threadIdx.x;
     const bool topdown = it.flags & DPX_TOPDOWN;
     const int W = it.W, H = it.H;
-    // the lane's column: block and x (-1: the empty column before a block);
-    // lanes past the last block stand on its last column and are not stored
-    const uint32_t p = strip * kStripCols + lane;
-    const uint32_t blk = p / ((uint32_t)W + 1);
-    const bool col = blk < sp.blocks && p % ((uint32_t)W + 1) != 0;
-    const uint32_t b = min(blk, sp.blocks - 1);
-    const int x = col ? (int)(p % ((uint32_t)W + 1)) - 1 : (blk < sp.blocks ? 0 : W - 1);
-    const int y0 = (int)(b * sp.rows);
+    const StripLane sl = strip_lane(W, sp, strip, lane);
+    const bool col = sl.col;
+    const int x = sl.x, y0 = sl.y0;
     const uint64_t cols = __builtin_amdgcn_ballot_w64(col);
     const uint64_t mine = cols & 0x7FFFFFFFFFFFFFFEull;  // the columns stored by this strip
     const int y0_first = __builtin_amdgcn_readlane(y0, 0), y0_last = __builtin_amdgcn_readlane(y0, 63);
     const int R = (int)sp.rows + 2;  // row r is y = y0 - 1 + r
 
-    // Pixels are read through a buffer descriptor of the item's rows, which
-    // answers 0 past its end (rows above or below the frame).  Row r of a lane
-    // lies at voff + (r - 1) * step modulo 2^32; byte offsets within an item
-    // fit 31 bits (checked on the host).  Rows r_lo .. r_hi - 1 lie in the
-    // frame for every lane.  The last pixel of a frame of 3-byte pixels is
-    // read by bytes (`tail`: the strip holds it): its 4-byte word would end
-    // past the frame.
-    const uint32_t step = (uint32_t)(topdown ? -it.stride : it.stride);
-    const uint32_t voff = (uint32_t)(topdown ? H - 1 - y0 : y0) * (uint32_t)it.stride + (uint32_t)(x * it.ch);
+    // Pixels are read through a buffer descriptor of the item's rows.  Rows
+    // r_lo .. r_hi - 1 lie in the frame for every lane.  Groups that may hold
+    // the last pixel of a frame of 3-byte pixels (`tail`: a lane of the strip
+    // loads it) leave it out of their word loads and read it by bytes.
+    const uint32_t step = strip_step(it.stride, topdown);
+    const uint32_t voff = strip_offset(sl, H, it.stride, it.ch, topdown);
     const uint32_t in_end = (uint32_t)(H - 1) * (uint32_t)it.stride + (uint32_t)(W * it.ch);
     const auto src = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(in + it.in_off), 0, in_end, 0x00020000);
     const int r_lo = 1 - y0_first, r_hi = H + 1 - y0_last;
     const bool tail = PIXELS != kPixelsIndexed && it.ch < 4 &&
-                      __builtin_amdgcn_ballot_w64(x == W - 1 && (topdown ? y0 <= 1 : y0 + (int)sp.rows >= H - 1)) != 0;
+                      __builtin_amdgcn_ballot_w64(strip_loads_last(sl, W, H, topdown, strip_loaded_rows(sp))) != 0;
 
     uint32_t px[G];
     auto fetch = [&](int r0) {
         uint32_t o = voff + (uint32_t)(r0 - 1) * step;
+        if (tail && group_loads_last(r0, topdown, r_hi)) {  // (as many loads as below)
+#pragma unroll
+            for (int q = 0; q < G; q++) {
+                px[q] = __builtin_amdgcn_raw_buffer_load_b32(src, (int)(word_crosses(o, in_end, 3) ? ~0u : o), 0, 0);
+                o += step;
+            }
+            return;
+        }
 #pragma unroll
         for (int q = 0; q < G; q++) {
             if constexpr (PIXELS == kPixelsIndexed)
@@ -388,7 +348,7 @@ __device__ __forceinline__ void graph_strip(const DevItem& it, const GraphSplit 
 #pragma unroll
     for (int q = 0; q < G; q++) __builtin_amdgcn_raw_buffer_store_b8((uint8_t)0, out, -1, 0, 0);
     for (int r0 = 0; r0 < R; r0 += G) {
-        if (tail && (topdown ? r0 < 2 : r0 + G >= r_hi)) fetch_bytes(r0);
+        if (tail && group_loads_last(r0, topdown, r_hi)) fetch_bytes(r0);
         uint32_t w[G];
 #pragma unroll
         for (int q = 0; q < G; q++) w[q] = px[q];
