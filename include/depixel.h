@@ -216,7 +216,9 @@ int dpx_context_create(int device, dpx_context** out);
 void dpx_context_destroy(dpx_context* ctx);
 /* Size the context's device buffers for batches of up to max_items items of
  * up to max_item_pixels pixels each, and build the tables of `scale` (0: none),
- * so that dpx_batch_run never has to grow them (growing waits for the device). */
+ * so that dpx_batch_run never has to grow them (growing waits for the device)
+ * for items without subdivision whose raster tiles form the same grid, scale
+ * by scale (other batches also need a map of their tiles, or coverage). */
 int dpx_context_reserve(dpx_context* ctx, int max_items, int64_t max_item_pixels, int scale);
 /* Enqueue the batch on `stream`; returns once enqueued.  The context's
  * scratch (graph buffers, descriptors) is reused across calls: calls on one

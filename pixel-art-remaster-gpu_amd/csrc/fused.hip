@@ -658,13 +658,14 @@ int grow_desc(dpx_context* ctx, size_t need)
     return DPX_OK;
 }
 
-// Descriptor bytes of a batch of n items whose items share a tile grid: the
+// Descriptor bytes of a batch of up to n items of up to `pixels` pixels: the
 // items twice (all, and per group), each array 64-byte aligned, with room for
-// one group per (scale, subdivision) pair.  (Batches of mixed sizes add tile
-// maps and may grow the buffer.)
-size_t desc_bytes(size_t n)
+// one group per (scale, subdivision) pair, and kf_graph's map of strips, which
+// items of the same tile grid need as well when their strips differ.  (Groups
+// of mixed sizes add raster tile maps and may grow the buffer.)
+size_t desc_bytes(size_t n, size_t pixels)
 {
-    return 2 * n * sizeof(DevItem) + 64 * (2 * 2 * (kMaxScale + 1) + 4);
+    return 2 * n * sizeof(DevItem) + graph_strips_bound(n, pixels) * sizeof(uint2) + 64 * (2 * 2 * (kMaxScale + 1) + 4);
 }
 
 // Launch grid of a kernel with TX x TY tiles over `dev`: (tile columns, tile
@@ -750,7 +751,7 @@ extern "C" int dpx_context_reserve(dpx_context* ctx, int max_items, int64_t max_
     std::lock_guard<std::mutex> lock(ctx->mu);
     DPX_HIP(hipSetDevice(ctx->device));
     if (int rc = grow_graph(ctx, (size_t)max_items * align_up((size_t)max_item_pixels, 256))) return rc;
-    if (int rc = grow_desc(ctx, desc_bytes((size_t)max_items))) return rc;
+    if (int rc = grow_desc(ctx, desc_bytes((size_t)max_items, (size_t)max_item_pixels))) return rc;
     if (scale > 0)
         if (int rc = ensure_mask(ctx, scale)) return rc;
     return DPX_OK;

@@ -53,6 +53,18 @@ __host__ __device__ inline GraphSplit graph_split(int W, int H, int max_rows)
     return s;
 }
 
+// No batch of up to n items of up to `pixels` pixels has more strips.  With
+// row blocks of r = graph_rows(T) rows, T the batch's pixels, an item of W x H
+// has at most (W + 61) / 62 strips where H <= r, and else, as ceil(H / r) < 2 H
+// / r and H <= W H, fewer than (4 W H / r + 61) / 62; and T / r is at most 3 *
+// kStripCols * kGraphWaves below the height's cap, T / kGraphMaxRows on it.
+inline size_t graph_strips_bound(size_t n, size_t pixels)
+{
+    const size_t total = n * pixels, per_rows = std::min<size_t>(total / kGraphMinRows, 3 * kStripCols * kGraphWaves);
+    return (n * (std::min<size_t>(pixels, 32768) + 61) + 4 * std::max<size_t>(per_rows, total / kGraphMaxRows)) /
+               kStripCols + 1;
+}
+
 // The column of a lane of a strip: whether it carries pixels, its x and its
 // block's first row.  The empty column before a block stands on the block's
 // first column, lanes past the last block on its last; neither is stored.
