@@ -38,7 +38,10 @@ int require_device()
 // them meanwhile: a 256x224 frame's diagram, 20.6 MB, in 530 us instead of
 // 1155.  The slots are kept (a pinned allocation takes longer than the copy)
 // and freed when the library is unloaded; a call that finds them in use, or
-// cannot have them or a thread, copies as before.
+// cannot have them or a thread, copies as before.  So does one whose
+// destination the runtime knows: memory that is pinned already takes the
+// link's rate directly (a 640x480 frame at 8x, 78.6 MB: 2.2 ms a call, through
+// the slots 2.6 to 7.8, by the cores the threads get).
 namespace {
 
 constexpr size_t kChunk = 4 << 20, kSlots = 2, kDownloadMin = 4 << 20;
@@ -59,13 +62,23 @@ Staging& staging()
     return s;
 }
 
+// Is p the runtime's own memory (pinned, managed, a device's)?
+bool known(const void* p)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return false;
+}
+
 }  // namespace
 
 hipError_t download(void* dst, const void* src, size_t n)
 {
+    if (n < kDownloadMin || known(dst)) return hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
     Staging& st = staging();
     std::unique_lock<std::mutex> lock(st.mu, std::try_to_lock);
-    if (n < kDownloadMin || !lock.owns_lock()) return hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+    if (!lock.owns_lock()) return hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
     if (!st.pin && hipHostMalloc((void**)&st.pin, kChunk * kSlots, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
         st.pin = nullptr;
