@@ -605,7 +605,7 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     __shared__ uint16_t s_key[RCX * RCY];
     __shared__ uint8_t s_info[RCX * RCY];  // coverage summary bits 0..4 (simple_cell)
     __shared__ uint32_t s_col[RCX * RCY];
-    __shared__ uint32_t s_src[SUB ? RCX * RCY : 1];  // smoothed candidates: word offset of their rows
+    __shared__ uint32_t s_src[SUB ? RCX * RCY : 1];  // smoothed candidates: word offset of their rows in the item's
     __shared__ uint16_t s_list[RTX * RTY];  // own cells that need the candidate search
     __shared__ int s_nlist;
     // resolved pixels of the first listed cells, so that every own
@@ -633,6 +633,8 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     const DevItem it = items[at.item];
     const int x0 = at.tx * RTX, y0 = at.ty * RTY;
     const uint8_t* aux = gaux + it.g_off;
+    // (an item's coverage is less than 2^32 words, checked on the host; a batch's may be more)
+    const uint32_t* item_rows = SUB ? cell_rows + it.rows_off / 4 : nullptr;
     const int ay0 = y0 - 2;  // first snapshot row
 
     if (t == 0) {
@@ -717,9 +719,9 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
                 // an internal one (node 90) keeps its hull: the table's
                 uint32_t src = 0xFFFFFFFFu;
                 if ((key & 0xFFu) != 90) {
-                    src = (uint32_t)(it.rows_off / 4) + ((uint32_t)y * (uint32_t)it.W + (uint32_t)x) * RW;
+                    src = ((uint32_t)y * (uint32_t)it.W + (uint32_t)x) * RW;
                     constexpr int at = S > kMaxCellScale ? 32 * MW : S <= kMaxCellScale16 ? 16 * 9 : 8 * 9 * S;
-                    info = (uint8_t)((cell_rows[src + at / 32] >> (at % 32)) & 0x1Fu);
+                    info = (uint8_t)((item_rows[src + at / 32] >> (at % 32)) & 0x1Fu);
                 } else {
                     info = info_table[key] & 0x1Fu;
                 }
@@ -806,7 +808,7 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
                 if (!(own_full && before_own) && r >= 0 && r < MW && s_key[k] != kNoCell) {
                     if constexpr (SUB) {
                         const uint32_t src = s_src[k];
-                        row = src != 0xFFFFFFFFu ? cell_rows[src + r] : mask_table[(uint32_t)s_key[k] * MW + r];
+                        row = src != 0xFFFFFFFFu ? item_rows[src + r] : mask_table[(uint32_t)s_key[k] * MW + r];
                     } else {
                         row = mask_table[(uint32_t)s_key[k] * MW + r];
                     }
@@ -914,7 +916,7 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
                     const uint8_t* src = cell_table + ((key * 9 + j) * PARTS + h) * TB;
                     if constexpr (SUB) {
                         if (s_src[k] != 0xFFFFFFFFu)
-                            src = reinterpret_cast<const uint8_t*>(cell_rows + s_src[k]) + j * (PARTS == 1 ? 2 : S) + 4 * h;
+                            src = reinterpret_cast<const uint8_t*>(item_rows + s_src[k]) + j * (PARTS == 1 ? 2 : S) + 4 * h;
                     }
                     __builtin_memcpy(&m[j], src, TB);
                 }
