@@ -585,10 +585,14 @@ __device__ inline void sim_short(const Bc& b, int p, uint32_t off, uint32_t len,
 // smallest of each 64, so that a walk of any length is three LDS reads: the
 // 64 positions around its start, the minima, the 64 positions that hold the
 // first marked one (cycles of 6,000 positions with 3,000 walks of 250 steps
-// are met in 640x480 frames).  Beyond, the times lie in T and a walk reads
-// the positions ahead of it in chunks.
+// are met in 640x480 frames).  Beyond, the times lie in T and the LDS holds
+// the smallest of each 64 << shift of them, and of each 64 of those: a walk is
+// two reads of T around LDS reads.  (Game frames of 1280x960 and up have faces
+// of 30,000 positions and thousands of walks of that length: reading T ahead
+// of each walk, through device-scope atomics, 1280x960 took 50 to 108 ms and
+// 1920x1080 7 to 141.)
 struct LongLds {
-    uint32_t tm[kLong];
+    uint32_t tm[kLong];  // times, or beyond kLong positions the smallest of each 64 << shift
     uint16_t ring[kLong];
     uint32_t bm[kLong / 64];
     int ct;
@@ -601,7 +605,7 @@ __device__ inline void wave_settle()  // this wave's LDS writes are seen by its 
 }
 
 // The place of the first position after P, n of them (wrapping), whose time
-// is below st; -1: none.  For paths in LDS.
+// is below st; -1: none.  On the entries of tm.
 __device__ inline int first_marked(const LongLds& s, int P, bool cyc, uint32_t st)
 {
     const int lane = threadIdx.x & 63, B = P >> 6, pl = P & 63;
@@ -635,15 +639,26 @@ __device__ inline void sim_long(const Bc& b, int p, uint32_t off, uint32_t len, 
     const bool cyc = len & kCycle;
     __syncthreads();  // (the block's path before: its LDS, its tau)
     const int32_t tau = __hip_atomic_load(&b.tau[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), old_ct = b.ct[p];
+    // (T is this block's alone until the kernel ends, and written anew by every evaluation)
     uint32_t* tg = b.T + off;
     auto get = [&](int q) -> uint32_t {
         if constexpr (LDS) return s.tm[q];
-        else return __hip_atomic_load(&tg[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else return __hip_atomic_load(&tg[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    auto put = [&](int q, uint32_t v) {
+        if constexpr (LDS) s.tm[q] = v;
+        else __hip_atomic_store(&tg[q], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     auto ring = [&](int q) -> int {
         if constexpr (LDS) return s.ring[q];
         else return b.ring[off + q] - (int)off;
     };
+    int sb = 6;  // positions of an entry of minima: 1 << sb
+    if constexpr (!LDS) {
+        while ((uint32_t)(L - 1) >> sb >= (uint32_t)kLong) sb++;
+        for (int k = t; k < kLong; k += THREADS) s.tm[k] = 0xFFFFFFFEu;
+        __syncthreads();
+    }
     const int L64 = (L + 63) / 64 * 64;
     for (int q = t; q < L64; q += THREADS) {  // (whole waves)
         uint32_t v = 0xFFFFFFFFu;
@@ -652,18 +667,23 @@ __device__ inline void sim_long(const Bc& b, int p, uint32_t off, uint32_t len, 
             const int32_t was = b.m[off + q];
             if (was <= tau) v = min(v, (uint32_t)was << 1);
             if constexpr (LDS) s.ring[q] = (uint16_t)(b.ring[off + q] - (int32_t)off);
-            else __hip_atomic_store(&tg[q], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else put(q, v);
         }
-        if constexpr (LDS) {
-            s.tm[q] = v;
-            const uint32_t low = (uint32_t)wave_min((int)(v >> 1)) << 1;
-            if (lane == 0) s.bm[q >> 6] = low;
+        if constexpr (LDS) s.tm[q] = v;
+        const uint32_t low = (uint32_t)wave_min((int)(v >> 1)) << 1;
+        if (lane == 0) {
+            if constexpr (LDS) s.bm[q >> 6] = low;
+            else atomicMin(&s.tm[q >> sb], low);
         }
     }
     if constexpr (LDS) {
         for (int k = L64 / 64 + t; k < kLong / 64; k += THREADS) s.bm[k] = 0xFFFFFFFEu;
     } else {
-        __threadfence();
+        __syncthreads();
+        for (int k = t; k < kLong; k += THREADS) {  // (whole waves)
+            const uint32_t low = (uint32_t)wave_min((int)(s.tm[k] >> 1)) << 1;
+            if (lane == 0) s.bm[k >> 6] = low;
+        }
     }
     __syncthreads();
     if (t < 64) {
@@ -689,25 +709,22 @@ __device__ inline void sim_long(const Bc& b, int p, uint32_t off, uint32_t len, 
                 if constexpr (LDS) {
                     h = first_marked(s, P, cyc, st);
                 } else {
-                    constexpr int U = 4;
-                    const int n = cyc ? L - 1 : L - 1 - P;
-                    for (int c = 1; h < 0 && c <= n; c += 64 * U) {
-                        uint32_t v[U];
-#pragma unroll
-                        for (int u = 0; u < U; u++) {
-                            const int d = c + 64 * u + lane;
-                            int q = d <= n ? P + d : P;
-                            if (q >= L) q -= L;
-                            v[u] = get(q);
+                    // the first position in lo .. hi - 1 whose time is below st
+                    auto scan = [&](int lo, int hi) {
+                        for (int c = lo & ~63; c < hi; c += 64) {
+                            const int q = c + lane;
+                            if (const uint64_t hit = __ballot(q >= lo && q < hi && (get(q) >> 1) < st))
+                                return c + (int)__builtin_ctzll(hit);
                         }
-#pragma unroll
-                        for (int u = 0; u < U; u++) {
-                            const uint64_t hit = __ballot(c + 64 * u + lane <= n && (v[u] >> 1) < st);
-                            if (hit && h < 0) {
-                                h = P + c + 64 * u + (int)__builtin_ctzll(hit);
-                                if (h >= L) h -= L;
-                            }
-                        }
+                        return -1;
+                    };
+                    auto end = [&](int e) { return (int)min((uint32_t)L, (uint32_t)(e + 1) << sb); };
+                    const int own = P >> sb;
+                    h = scan(P + 1, end(own));
+                    if (h < 0) {
+                        const int blk = first_marked(s, own, cyc, st);
+                        if (blk >= 0) h = scan(blk << sb, end(blk));
+                        else if (cyc) h = scan(own << sb, P);
                     }
                 }
                 if (h < 0 && cyc) {
@@ -719,16 +736,17 @@ __device__ inline void sim_long(const Bc& b, int p, uint32_t off, uint32_t len, 
                 do {  // (uniform: every place of the node on this path)
                     const uint32_t v = get(q);
                     if (lane == 0 && (st << 1) < v) {
+                        put(q, st << 1);
                         if constexpr (LDS) {
-                            s.tm[q] = st << 1;
-                            if ((st << 1) < s.bm[q >> 6]) s.bm[q >> 6] = st << 1;
+                            s.bm[q >> 6] = min(s.bm[q >> 6], st << 1);
                         } else {
-                            __hip_atomic_store(&tg[q], st << 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            const int e = q >> sb;
+                            s.tm[e] = min(s.tm[e], st << 1);
+                            s.bm[e >> 6] = min(s.bm[e >> 6], st << 1);
                         }
                     }
                     q = ring(q);
                 } while (q != prev);
-                if constexpr (!LDS) __threadfence();
                 wave_settle();
             }
         }
