@@ -155,8 +155,9 @@ int dpx_stage_components(const uint8_t* d_graph, int width, int height, int32_t*
  * d_counts[3] receives the number of chains, of nodes and a status (0;
  * DPX_ENOMEM when max_nodes or max_chains is too small; DPX_EINVAL, with no
  * chains, when a link leaves the frame or has no reverse link: the graph
- * is not a resolved, symmetric similarity graph), readable once the stream
- * reaches this point. */
+ * is not a resolved, symmetric similarity graph; DPX_EHIP, with no chains,
+ * should the walks not settle within 2 width height + 1 rounds, which no graph
+ * is known to need), readable once the stream reaches this point. */
 int dpx_stage_border_chains(const uint8_t* d_graph, int width, int height, uint8_t* d_scratch,
                             int32_t* d_nodes, int max_nodes, int32_t* d_sizes, int max_chains,
                             int32_t* d_counts, void* stream);

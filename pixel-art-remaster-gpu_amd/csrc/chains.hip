@@ -883,10 +883,13 @@ __global__ __launch_bounds__(256) void k_bc_spread(Bc b, int r, int slot)
 }
 
 // The rounds that are left, in one block: on few paths a block's barrier
-// costs less than a launch.  Ends when no path waits: every round makes at
-// least the smallest walk that was not final so.
+// costs less than a launch.  Ends when no path waits: among the short paths
+// every round makes at least the smallest walk that is not final (for what the
+// long ones last did) so, and each evaluation of the long ones the smallest of
+// all.  Frames take a few dozen rounds; paths that still wait after max_rounds
+// leave no chains and a status.
 constexpr int kFinishBlock = 1024;
-__global__ __launch_bounds__(kFinishBlock) void k_bc_finish(Bc b, int slot)
+__global__ __launch_bounds__(kFinishBlock) void k_bc_finish(Bc b, int slot, uint32_t max_rounds)
 {
     __shared__ LongLds s;
     __shared__ int s_short, s_long, s_nodes;
@@ -902,7 +905,7 @@ __global__ __launch_bounds__(kFinishBlock) void k_bc_finish(Bc b, int slot)
             if (short_waits(b, p)) b.dshort[atomicAdd(&s_short, 1)] = p;
     __syncthreads();
     int n_short = s_short, n_long = s_long;
-    for (uint32_t round = 0; (n_short | n_long) && round <= 2 * b.N; round++) {  // (uniform)
+    for (uint32_t round = 0; (n_short | n_long) && round < max_rounds; round++) {  // (uniform)
         __syncthreads();
         if (t == 0) {
             s_nodes = s_short = 0;
@@ -926,6 +929,7 @@ __global__ __launch_bounds__(kFinishBlock) void k_bc_finish(Bc b, int slot)
         n_short = s_short;
         n_long = s_long;
     }
+    if (t == 0 && (n_short | n_long)) b.ctr[kStatus] = DPX_EHIP;
 }
 
 // The chain a node starts: its length (0: none), its place and its path's range.
@@ -1033,9 +1037,11 @@ __global__ __launch_bounds__(kNodeBlock) void k_bc_write(Bc b, const uint64_t* _
 
 }  // namespace
 
-extern "C" int dpx_stage_border_chains(const uint8_t* d_graph, int W, int H, uint8_t* d_scratch, int32_t* d_nodes,
-                                       int max_nodes, int32_t* d_sizes, int max_chains, int32_t* d_counts,
-                                       void* stream)
+// dpx_stage_border_chains with a bound on k_bc_finish's rounds (not part of
+// the interface: the test of what happens at the bound calls it).
+extern "C" int dpx_internal_border_chains(const uint8_t* d_graph, int W, int H, uint8_t* d_scratch, int32_t* d_nodes,
+                                          int max_nodes, int32_t* d_sizes, int max_chains, int32_t* d_counts,
+                                          void* stream, uint32_t max_rounds)
 {
     DPX_CHECK(d_graph && d_scratch && d_nodes && d_sizes && d_counts && W > 0 && H > 0, DPX_EINVAL,
               "bad arguments");
@@ -1123,7 +1129,7 @@ extern "C" int dpx_stage_border_chains(const uint8_t* d_graph, int W, int H, uin
         else hipLaunchKernelGGL(k_bc_sim<false>, sims, dim3(kSimBlock), 0, s, b, r, -1);
         hipLaunchKernelGGL(k_bc_spread, per_node, dim3(256), 0, s, b, r, slot);
     }
-    hipLaunchKernelGGL(k_bc_finish, dim3(1), dim3(kFinishBlock), 0, s, b, slot);
+    hipLaunchKernelGGL(k_bc_finish, dim3(1), dim3(kFinishBlock), 0, s, b, slot, max_rounds);
     hipLaunchKernelGGL(k_bc_count, per_block, dim3(kNodeBlock), 0, s, b, sums);
     hipLaunchKernelGGL(k_bc_sums, dim3(1), dim3(kNodeBlock), 0, s, b, sums, node_blocks, max_nodes, max_chains,
                        d_counts);
@@ -1131,6 +1137,15 @@ extern "C" int dpx_stage_border_chains(const uint8_t* d_graph, int W, int H, uin
                        d_counts);
     DPX_HIP(hipGetLastError());
     return DPX_OK;
+}
+
+extern "C" int dpx_stage_border_chains(const uint8_t* d_graph, int W, int H, uint8_t* d_scratch, int32_t* d_nodes,
+                                       int max_nodes, int32_t* d_sizes, int max_chains, int32_t* d_counts,
+                                       void* stream)
+{
+    // (W H is checked there; twice the nodes and one more, far beyond what any graph has been seen to take)
+    return dpx_internal_border_chains(d_graph, W, H, d_scratch, d_nodes, max_nodes, d_sizes, max_chains, d_counts, stream,
+                                      2u * (uint32_t)W * (uint32_t)H + 1u);
 }
 
 }  // namespace dpx
