@@ -120,7 +120,7 @@ __global__ void kt_info(const uint32_t* __restrict__ mask, int S, uint8_t* __res
 // kf_graph: similarity graph + trivial crossing removal
 // ---------------------------------------------------------------------------
 // One wave marches down the rows of a strip of 64 columns, one column per
-// lane, with the lane word (pixel class + YUV fields, see lane_ref) of the
+// lane, with the lane word (pixel class + YUV fields, see yuv_lanes) of the
 // row above in a register and no LDS, barrier or second pass:
 //   * a similarity test is two subtractions, one three-input logic operation
 //     and a compare; the right neighbours' words come through the DPP shift
@@ -150,15 +150,8 @@ __device__ inline void shift_in(uint32_t& v, uint64_t m)
     asm("v_addc_co_u32_e64 %0, %1, %0, %0, %2" : "+v"(v), "=s"(c) : "s"(m));
 }
 
-// Two lane words a, b are similar iff bit 8 of each 10-bit lane of a - b + t
-// + 256 and of b - a + t + 256 is set (a lane holds 6 .. 518, so none borrows
-// or carries; with d the fields' difference, bit 8 of the first is set iff -t
-// <= d <= 255 - t) and the classes are equal, which leaves 3 in the class bits
-// of both.
-constexpr uint32_t kSimilarBias = 3u << 30 | (256u + 5) << 20 | (256u + 7) << 10 | (256u + 6);
-constexpr uint32_t kSimilarTest = 3u << 30 | 1u << 28 | 1u << 18 | 1u << 8;
-
-// A row of lane words as the tests take it: l, l + bias and bias - l.
+// A row of lane words as the tests take it (see lane_similar): l, l + bias and
+// bias - l.
 struct LaneRow {
     uint32_t l, plus, minus;
 };
@@ -277,14 +270,7 @@ __device__ __forceinline__ void graph_strip(const DevItem& it, const GraphSplit 
         }
     };
 
-    // Lane words.  Colours of three bytes c0, c1, c2: n = 299 c0 + 587 c1 +
-    // 114 c2 as two byte dot products, luma's quotient as in luma() (the high
-    // half of a 24-bit product, whose low half is 704 n / 1000 for a multiple
-    // of 1000 and at least 4294968 otherwise: the multiples but 0, black, take
-    // luma()'s double expression); the packed word is put together in the lane
-    // word's 10-bit lanes at once, where negative U and V borrow from the
-    // lane above as they do in yuv_pack's bytes (a lane below zero there is
-    // below zero here, since |U|, |V| < 256).
+    // Lane words (see luma_sum and lane_fields for the steps).
     const uint32_t cls = col ? kLaneOpaque : 0u, cls_clear = col ? kLaneTransparent : 0u;
     const uint32_t order = (it.flags & DPX_RGB) ? 0x03000102u : 0x03020100u;
     const uint32_t clear_below = ((it.flags & DPX_ALPHA) && it.ch == 4) ? 1u << 24 : 0u;
@@ -299,10 +285,9 @@ __device__ __forceinline__ void graph_strip(const DevItem& it, const GraphSplit 
 #pragma unroll
             for (int q = 0; q < G; q++) {
                 if constexpr (PIXELS == kPixelsGeneral) v[q] = __builtin_amdgcn_perm(0u, v[q], order);
-                const uint32_t n = __builtin_amdgcn_udot4(
-                    v[q], 0x00724B2Bu, __builtin_amdgcn_udot4(v[q], 0x00000201u, 0u, false) << 8, false);
-                y[q] = (uint32_t)(((uint64_t)(n & 0xFFFFFFu) * 4294968u) >> 32);
-                whole[q] = __builtin_amdgcn_ballot_w64((n & 0xFFFFFFu) * 4294968u - 1u < 4294967u);
+                const uint32_t n = luma_sum(v[q]);
+                y[q] = luma_quotient(n);
+                whole[q] = __builtin_amdgcn_ballot_w64(luma_whole(n));
             }
             uint64_t any = 0;
 #pragma unroll
@@ -316,11 +301,7 @@ __device__ __forceinline__ void graph_strip(const DevItem& it, const GraphSplit 
             }
 #pragma unroll
             for (int q = 0; q < G; q++) {
-                const int u = (int)((float)((int)((v[q] >> 16) & 0xFFu) - (int)y[q]) * 0.492f);
-                const int vv = (int)((float)((int)(v[q] & 0xFFu) - (int)y[q]) * 0.877f);
-                uint32_t f = (y[q] << 10) + (uint32_t)u;
-                asm("" : "+v"(f));  // (keeps the sum two shift-and-adds)
-                f = (((f << 10) + (uint32_t)vv) & 0x0FF3FCFFu) | cls;
+                uint32_t f = lane_fields(v[q], y[q]) | cls;
                 if constexpr (PIXELS == kPixelsGeneral) f = v[q] < clear_below ? cls_clear : f;
                 v[q] = f;
             }

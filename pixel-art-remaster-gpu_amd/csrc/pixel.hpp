@@ -105,30 +105,63 @@ __host__ __device__ inline uint32_t yuv_lanes(uint32_t w)
     return ((w >> 16) & 0xFFu) << 20 | ((w >> 8) & 0xFFu) << 10 | (w & 0xFFu);
 }
 
-// |dY| <= 5, |dU| <= 7, |dV| <= 6 on the fields, all three lanes at once:
-// L = a - b + 256 + t stays inside its lane (7..517, so no lane borrows from
-// the next and the class bits subtract exactly, mod 4); a field is within
-// threshold iff 256 <= L <= 256 + 2t, i.e. bit 8 of L is set and M = L + 255
-// - 2t does not reach bit 9.  Equal classes leave bits 30-31 of L (and M)
-// clear.  A pair with one end outside the frame never passes; two ends
-// outside the frame do, and callers never ask for such a pair.
+// The lane word of a colour w = c0 | c1 << 8 | c2 << 16 (byte 3 is ignored) in
+// the steps kf_graph takes, four pixels at a time:
+//   n = luma_sum(w): 299 c0 + 587 c1 + 114 c2 in the low 24 bits, as two byte
+//     dot products, 43 c0 + 75 c1 + 114 c2 + 256 (c0 + 2 c1);
+//   y = luma_quotient(n), or where luma_whole(n) luma()'s double expression:
+//     the low half of the quotient's product is 704 n / 1000 < 2^18 for a
+//     multiple of 1000 and at least 4294968 otherwise, so the multiples but 0,
+//     black, are told from it;
+//   lane_fields(w, y): the packed word put together in the lanes at once,
+//     where negative U and V borrow from the lane above as they do in
+//     yuv_pack's bytes (a lane below zero there is below zero here, since |U|,
+//     |V| < 256).
+__host__ __device__ inline uint32_t luma_sum(uint32_t w)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_udot4(w, 0x00724B2Bu, __builtin_amdgcn_udot4(w, 0x00000201u, 0u, false) << 8, false);
+#else
+    const uint32_t c0 = w & 0xFFu, c1 = (w >> 8) & 0xFFu, c2 = (w >> 16) & 0xFFu;
+    return (c0 + 2u * c1) * 256u + 0x2Bu * c0 + 0x4Bu * c1 + 0x72u * c2;
+#endif
+}
+__host__ __device__ inline uint32_t luma_quotient(uint32_t n)
+{
+    return (uint32_t)(((uint64_t)(n & 0xFFFFFFu) * 4294968u) >> 32);
+}
+__host__ __device__ inline bool luma_whole(uint32_t n) { return (n & 0xFFFFFFu) * 4294968u - 1u < 4294967u; }
+__host__ __device__ inline uint32_t lane_fields(uint32_t w, uint32_t y)
+{
+    const int u = (int)((float)((int)((w >> 16) & 0xFFu) - (int)y) * 0.492f);
+    const int v = (int)((float)((int)(w & 0xFFu) - (int)y) * 0.877f);
+    uint32_t f = (y << 10) + (uint32_t)u;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm("" : "+v"(f));  // (keeps the sum two shift-and-adds)
+#endif
+    return ((f << 10) + (uint32_t)v) & 0x0FF3FCFFu;
+}
+
+// |dY| <= 5, |dU| <= 7, |dV| <= 6 on the fields, all three lanes at once: two
+// lane words a, b are similar iff bit 8 of each 10-bit lane of a - b + t + 256
+// and of b - a + t + 256 is set (a lane holds 6 .. 518, so none borrows or
+// carries; with d the fields' difference, bit 8 of the first is set iff -t <= d
+// <= 255 - t) and the classes are equal, which leaves 3 in the class bits of
+// both.  A pair with one end outside the frame never passes; two ends outside
+// the frame do, and callers never ask for such a pair.  kf_graph's row_edges is
+// this test on the words of two rows, in assembly.
+constexpr uint32_t kSimilarBias = 3u << 30 | (256u + 5) << 20 | (256u + 7) << 10 | (256u + 6);
+constexpr uint32_t kSimilarTest = 3u << 30 | 1u << 28 | 1u << 18 | 1u << 8;
+
 struct LaneRef {
-    uint32_t not_s;  // ~(a + B1): ~L = b + not_s
-    uint32_t m;      // a + B1 + B2: M = m - b
+    uint32_t plus, minus;  // a + bias and bias - a
 };
 
-__host__ __device__ inline LaneRef lane_ref(uint32_t la)
-{
-    const uint32_t B1 = (256u + 5) << 20 | (256u + 7) << 10 | (256u + 6);
-    const uint32_t B2 = (255u - 10) << 20 | (255u - 14) << 10 | (255u - 12);
-    uint32_t s = la + B1;
-    return LaneRef{ ~s, s + B2 };
-}
+__host__ __device__ inline LaneRef lane_ref(uint32_t la) { return LaneRef{ la + kSimilarBias, kSimilarBias - la }; }
 
 __host__ __device__ inline uint32_t lane_similar(const LaneRef& a, uint32_t lb)
 {
-    uint32_t bad = (0x10040100u & (a.not_s + lb)) | ((a.m - lb) & 0xE0080200u);
-    return bad == 0 ? 1u : 0u;
+    return ((a.plus - lb) & kSimilarTest & (a.minus + lb)) == kSimilarTest ? 1u : 0u;
 }
 
 __host__ __device__ inline int iabs(int a) { return a < 0 ? -a : a; }
