@@ -597,7 +597,11 @@ __host__ __device__ inline int mad24(int a, int b, int c)
 }
 
 // With `test` false (the caller knows the polygon to be strictly convex) no
-// vertex can lie in another three's triangle, and none is looked at.
+// vertex can lie in another three's triangle, and none is looked at.  That
+// reasoning is about the plane, so it takes coordinates whose products are not
+// cut off: with |x|, |y| <= kEarLimit a difference is below 2^15, and a cross
+// product of differences is at most 8 kEarLimit^2 < 2^31.
+constexpr int kEarLimit = 16383;
 template <int MAXN, class V, class Ear>
 __host__ __device__ inline int ear_clip_ring(const V* P, int stride, int n, bool test, Ear ear)
 {

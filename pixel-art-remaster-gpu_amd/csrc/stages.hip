@@ -366,7 +366,7 @@ __global__ __launch_bounds__(kTriBlock) void k_triangulate(dpx_point* __restrict
         for (int k = 0; k < PER; k++) {
             const int c = t / MAXN + k * (kTriBlock / MAXN);
             uint32_t w;
-            if (!pack_point((int)(p[k].x * 64.0f), (int)(p[k].y * 64.0f), 32767, &w)) s_any[c] = 1;
+            if (!pack_point((int)(p[k].x * 64.0f), (int)(p[k].y * 64.0f), kEarLimit, &w)) s_any[c] = 1;
             s_poly[q * kTriRun + c] = w;
         }
     }
