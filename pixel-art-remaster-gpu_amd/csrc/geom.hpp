@@ -15,6 +15,13 @@ namespace dpx {
 
 constexpr int kCellSize = 45;   // CELL_SIZE, kernel.cu:8
 constexpr int kMaxPts = 16;     // createCellFromPattern pushes at most 2 points per case
+// Triangles of a triangulated cell by its vertex count, at most as many as its
+// slots hold; 0 for the counts of a caller's diagram that are no polygon's (the
+// subtraction first would overflow for the least of them).
+__host__ __device__ inline int cell_triangles(int edge_count)
+{
+    return edge_count < 3 ? 0 : edge_count > kCellSize / 3 + 1 ? kCellSize / 3 : edge_count - 2;
+}
 constexpr int kMaxPoly = 32;    // subdivision emits at most 2 points per hull vertex
 
 // neighbour offsets of graph bit e (diff, graph_functions.cu:194-235)

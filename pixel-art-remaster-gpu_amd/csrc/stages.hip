@@ -526,7 +526,7 @@ __device__ __noinline__ uint32_t tri_sample_any(ImgView im, const dpx_point* __r
     for (int j = j1; j >= j0; j--)
         for (int i = i1; i >= i0; i--) {
             const size_t k = (size_t)j * im.W + (size_t)i;
-            const int nt = min(edge_count[k] - 2, kCellSize / 3);
+            const int nt = cell_triangles(edge_count[k]);
             const dpx_point* c = &diagram[k * kCellSize];
             const float fi = (float)i, fj = (float)j;
             const long long sx = px - (long long)i * unit, sy = py - (long long)j * unit;
@@ -641,7 +641,7 @@ __global__ __launch_bounds__(16 * TY) void k_tri(ImgView im, const dpx_point* __
                 if (t == 0) s_any = 1;
             } else {
                 for (int k = t; k < nc; k += NT)
-                    s_nt[k] = min(edge_count[(size_t)(bj + k / nci) * im.W + bi + k % nci] - 2, kTris);
+                    s_nt[k] = cell_triangles(edge_count[(size_t)(bj + k / nci) * im.W + bi + k % nci]);
                 __syncthreads();
                 int lo = 0, hi = 64;
                 bool wide = false;
@@ -791,7 +791,7 @@ __global__ __launch_bounds__(256) void k_tri_far(ImgView im, const dpx_point* __
     for (long long j = j1; j >= j0 && left; j--)
         for (long long i = i1; i >= i0 && left; i--) {
             const size_t k = (size_t)j * im.W + (size_t)i;
-            const int nt = min(edge_count[k] - 2, kCellSize / 3);
+            const int nt = cell_triangles(edge_count[k]);
             const dpx_point* c = &diagram[k * kCellSize];
             const float fi = (float)i, fj = (float)j;
             uint32_t hit = 0;
