@@ -39,16 +39,16 @@ struct DevItem {
 
 // Summary of a cell's coverage rows at scale S: bit 0 = it covers every
 // sample of its own square; bit 1 + (dy+1)*3 + (dx+1) = it covers a sample of
-// the neighbouring square at (dx, dy).
-__host__ __device__ inline uint32_t coverage_info(const uint32_t* rows, int S)
+// the neighbouring square at (dx, dy).  The rows are those of samples y0 .. y0 +
+// n - 1, their bits the samples from x0.
+__host__ __device__ inline uint32_t coverage_info(const uint32_t* rows, int S, int x0, int y0, int n)
 {
-    const int kmin = mask_kmin(S), mw = mask_w(S);
-    const int c0 = -kmin;  // bit of the own square's first column
+    const int c0 = -x0;  // bit of the own square's first column
     const uint32_t own = ((1u << S) - 1u) << c0;
     uint32_t info = 0;
     bool full = true;
-    for (int r = 0; r < mw; r++) {
-        int ky = kmin + r;
+    for (int r = 0; r < n; r++) {
+        int ky = y0 + r;
         int dy = ky < 0 ? -1 : (ky >= S ? 1 : 0);
         uint32_t row = rows[r];
         if (dy == 0 && (row & own) != own) full = false;
@@ -72,19 +72,19 @@ __host__ __device__ constexpr size_t cell_table_bytes(int S)
     return S > kMaxCellScale ? 0 : (size_t)kKeys * 9 * (S <= kMaxCellScale16 ? 2 : 8);
 }
 
-// The rows of the nine masks of a cell with coverage rows `row(r)`: put(j,
-// ky, bits), those without any left out.
-template <int S, class R, class F>
+// The rows of the nine masks of a cell with coverage rows `row(r)`, samples Y0 ..
+// of N, their bits the samples from X0: put(j, ky, bits), those without any
+// left out.
+template <int S, int X0, int Y0, int N, class R, class F>
 __host__ __device__ inline void cell_mask_rows(R row, F put)
 {
-    constexpr int kmin = mask_kmin(S), mw = mask_w(S);
 #pragma unroll
     for (int j = 0; j < 9; j++) {
-        const int dy = 1 - j / 3, dx = 1 - j % 3, sh = -dx * S - kmin;
+        const int dy = 1 - j / 3, dx = 1 - j % 3, sh = -dx * S - X0;
 #pragma unroll
         for (int ky = 0; ky < S; ky++) {
-            const int r = ky - dy * S - kmin;
-            if (r < 0 || r >= mw) continue;
+            const int r = ky - dy * S - Y0;
+            if (r < 0 || r >= N) continue;
             put(j, ky, (sh >= 0 ? (row(r) >> sh) : (row(r) << -sh)) & ((1u << S) - 1u));
         }
     }
@@ -407,7 +407,8 @@ __global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const D
                                                  uint32_t* __restrict__ rows)
 {
     DPX_TILE_NAMES(TX);
-    constexpr int MW = mask_w(S), KMIN = mask_kmin(S), RW = rows_words(S);
+    constexpr int X0 = cover_x0(S), Y0 = cover_y0(S), COLS = cover_w(S), ROWS = cover_h(S), RW = rows_words(S);
+    static_assert(COLS <= 32, "a row of samples is a word");
     constexpr int PITCH = 257;  // of the rows: adjacent rows of a cell in adjacent banks
     __shared__ int s_nblk;
     __shared__ uint32_t s_g32[GY * RWW];
@@ -420,7 +421,7 @@ __global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const D
     // its smoothed polygon at most 16, within the cells around (-64 .. 127)
     __shared__ uint16_t s_poly[16 * 256];
     // sample row r of column t at [r * PITCH + t], then its masks and summary; first the walk window
-    constexpr int COV = (MW + 1) * PITCH, WALK_WORDS = WALK ? WalkWindow<TX>::BYTES / 4 : 0;
+    constexpr int COV = (ROWS + 1 > RW ? ROWS + 1 : RW) * PITCH, WALK_WORDS = WALK ? WalkWindow<TX>::BYTES / 4 : 0;
     // What is needed until the polygons are made lies where the rows come
     // after them (the walk window is read meanwhile and keeps it apart): a
     // block more fits each CU.
@@ -511,7 +512,7 @@ __global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const D
     __syncthreads();
     if (t < nlist) {
 #pragma unroll
-        for (int r = 0; r < MW; r++) C[PITCH * r] = 0;
+        for (int r = 0; r < ROWS; r++) C[PITCH * r] = 0;
         // seen from its pixel's centre almost every cell goes round once
         // (no clipping is needed to know that it is cut wholly); the others
         // are clipped, their vertices counter-clockwise as ear_clip takes them
@@ -524,8 +525,8 @@ __global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const D
                 }
             s_clip[atomicAdd(&s_nclip, 1)] = (uint8_t)t;
         }
-        wsum = poly_rows_cross<MW>(P, 256, m, 2 * S, KMIN,
-                                   [&](int r, uint32_t mask) { atomicXor(&C[PITCH * r], mask); });
+        wsum = poly_rows_cross<ROWS, COLS>(P, 256, m, 2 * S, X0, Y0,
+                                           [&](int r, uint32_t mask) { atomicXor(&C[PITCH * r], mask); });
         s_m[t] = (uint8_t)m;
     }
     __syncthreads();
@@ -537,38 +538,38 @@ __global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const D
     if (t < nlist) {
         int bits = 0;
 #pragma unroll
-        for (int r = 0; r < MW; r++) bits += __builtin_popcount(C[PITCH * r]);
+        for (int r = 0; r < ROWS; r++) bits += __builtin_popcount(C[PITCH * r]);
         if (s_m[t] == 0 || wsum != bits) {
             // not cut wholly, or a winding other than 0 and 1 (none in the
             // synthetic workloads): the rows of each ear as it is cut
-            uint32_t cov[MW];
+            uint32_t cov[ROWS];
 #pragma unroll
-            for (int r = 0; r < MW; r++) cov[r] = 0;
+            for (int r = 0; r < ROWS; r++) cov[r] = 0;
             ear_clip_ring<16>(P, 256, m, true, [&](uint16_t A, uint16_t B, uint16_t E) {
                 // units of 1/(128 S) of a cell; counter-clockwise (an ear's cross is positive)
-                tri_rows_or<MW>(vert_x(A) * 2 * S, vert_y(A) * 2 * S, vert_x(B) * 2 * S, vert_y(B) * 2 * S,
-                                vert_x(E) * 2 * S, vert_y(E) * 2 * S, KMIN, cov);
+                tri_rect_or<ROWS, COLS>(vert_x(A) * 2 * S, vert_y(A) * 2 * S, vert_x(B) * 2 * S, vert_y(B) * 2 * S,
+                                        vert_x(E) * 2 * S, vert_y(E) * 2 * S, X0, Y0, cov);
             });
 #pragma unroll
-            for (int r = 0; r < MW; r++) C[PITCH * r] = cov[r];
+            for (int r = 0; r < ROWS; r++) C[PITCH * r] = cov[r];
         }
-        uint32_t cov[MW];
+        uint32_t cov[ROWS];
 #pragma unroll
-        for (int r = 0; r < MW; r++) cov[r] = C[PITCH * r];
-        const uint32_t info = coverage_info(cov, S);
+        for (int r = 0; r < ROWS; r++) cov[r] = C[PITCH * r];
+        const uint32_t info = coverage_info(cov, S, X0, Y0, ROWS);
         if constexpr (S <= kMaxCellScale) {
             uint32_t word[RW] = {};
-            cell_mask_rows<S>([&](int r) { return cov[r]; },
-                              [&](int j, int ky, uint32_t bits) {
-                                  const int at = S <= kMaxCellScale16 ? 16 * j + ky * S : 8 * (j * S + ky);
-                                  word[at / 32] |= bits << (at % 32);
-                              });
+            cell_mask_rows<S, X0, Y0, ROWS>([&](int r) { return cov[r]; },
+                                            [&](int j, int ky, uint32_t bits) {
+                                                const int at = S <= kMaxCellScale16 ? 16 * j + ky * S : 8 * (j * S + ky);
+                                                word[at / 32] |= bits << (at % 32);
+                                            });
             constexpr int at = S <= kMaxCellScale16 ? 16 * 9 : 8 * 9 * S;
             word[at / 32] |= (info & 0xFFu) << (at % 32);
 #pragma unroll
             for (int r = 0; r < RW; r++) C[PITCH * r] = word[r];
         } else {
-            C[PITCH * MW] = info;
+            C[PITCH * ROWS] = info;
         }
     }
     __syncthreads();
@@ -595,6 +596,9 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
 {
     DPX_TILE_NAMES(TX);
     constexpr int MW = mask_w(S), KMIN = mask_kmin(S), RW = rows_words(S);
+    // the grid of smoothed cells' rows; the table's are shifted to its columns
+    constexpr int SY0 = cover_y0(S), ROWS = cover_h(S), X0 = SUB ? cover_x0(S) : KMIN;
+    static_assert(KMIN >= X0 && last_sample(S, 80) - X0 < 32, "a hull's samples stay in the word");
     __shared__ uint32_t s_aux32[SUB ? 1 : AY * RWW];
     __shared__ uint32_t s_p32[SUB ? 1 : (GY + 1) * RWW];  // decisions of crossed blocks, by origin
     __shared__ uint16_t s_blk[SUB ? 1 : (GY + 1) * RDB];  // crossed blocks: origin byte index in the window
@@ -605,7 +609,7 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     __shared__ uint16_t s_key[RCX * RCY];
     __shared__ uint8_t s_info[RCX * RCY];  // coverage summary bits 0..4 (simple_cell)
     __shared__ uint32_t s_col[RCX * RCY];
-    __shared__ uint32_t s_src[SUB ? RCX * RCY : 1];  // smoothed candidates: word offset of their rows in the item's
+    __shared__ uint32_t s_src[SUB ? RCX * RCY : 1];  // smoothed candidates: word offset of their masks in the item's (from 9x: their cell)
     __shared__ uint16_t s_list[RTX * RTY];  // own cells that need the candidate search
     __shared__ int s_nlist;
     // resolved pixels of the first listed cells, so that every own
@@ -633,8 +637,12 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
     const DevItem it = items[at.item];
     const int x0 = at.tx * RTX, y0 = at.ty * RTY;
     const uint8_t* aux = gaux + it.g_off;
-    // (an item's coverage is less than 2^32 words, checked on the host; a batch's may be more)
+    // (an item's coverage is less than 2^32 words up to 8x, checked on the host; from 9x, and a batch's, it may be more)
     const uint32_t* item_rows = SUB ? cell_rows + it.rows_off / 4 : nullptr;
+    auto smoothed_cell = [&](uint32_t src) {
+        if constexpr (S <= kMaxCellScale) return item_rows + src;
+        else return item_rows + (size_t)src * RW;
+    };
     const int ay0 = y0 - 2;  // first snapshot row
 
     if (t == 0) {
@@ -719,9 +727,10 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
                 // an internal one (node 90) keeps its hull: the table's
                 uint32_t src = 0xFFFFFFFFu;
                 if ((key & 0xFFu) != 90) {
-                    src = ((uint32_t)y * (uint32_t)it.W + (uint32_t)x) * RW;
-                    constexpr int at = S > kMaxCellScale ? 32 * MW : S <= kMaxCellScale16 ? 16 * 9 : 8 * 9 * S;
-                    info = (uint8_t)((item_rows[src + at / 32] >> (at % 32)) & 0x1Fu);
+                    constexpr int at = S > kMaxCellScale ? 32 * ROWS : S <= kMaxCellScale16 ? 16 * 9 : 8 * 9 * S;
+                    src = (uint32_t)y * (uint32_t)it.W + (uint32_t)x;
+                    if constexpr (S <= kMaxCellScale) src *= RW;
+                    info = (uint8_t)((smoothed_cell(src)[at / 32] >> (at % 32)) & 0x1Fu);
                 } else {
                     info = info_table[key] & 0x1Fu;
                 }
@@ -802,14 +811,19 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
 #pragma unroll
             for (int dx = 1; dx >= -1; dx--) {
                 int k = (uy + 1 + dy) * RCX + (ux + 1 + dx);
-                int r = ky - dy * S - KMIN;
                 uint32_t row = 0;
                 const bool before_own = dy < 0 || (dy == 0 && dx < 0);
-                if (!(own_full && before_own) && r >= 0 && r < MW && s_key[k] != kNoCell) {
+                if (!(own_full && before_own) && s_key[k] != kNoCell) {
+                    const int r = ky - dy * S - KMIN;
                     if constexpr (SUB) {
                         const uint32_t src = s_src[k];
-                        row = src != 0xFFFFFFFFu ? item_rows[src + r] : mask_table[(uint32_t)s_key[k] * MW + r];
-                    } else {
+                        const int rs = ky - dy * S - SY0;
+                        if (src != 0xFFFFFFFFu) {
+                            if (rs >= 0 && rs < ROWS) row = smoothed_cell(src)[rs];
+                        } else if (r >= 0 && r < MW) {
+                            row = mask_table[(uint32_t)s_key[k] * MW + r] << (KMIN - X0);
+                        }
+                    } else if (r >= 0 && r < MW) {
                         row = mask_table[(uint32_t)s_key[k] * MW + r];
                     }
                 }
@@ -830,7 +844,7 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
         uint32_t seen = 0, won[9];
 #pragma unroll
         for (int j = 0; j < 9; j++) {
-            const int sh = (j % 3 - 1) * S - KMIN;
+            const int sh = (j % 3 - 1) * S - X0;
             const uint32_t bits = (sh >= 0 ? (rows[j] >> sh) : (rows[j] << -sh)) & FULL;
             won[j] = bits & ~seen;
             seen |= bits;
@@ -916,7 +930,7 @@ __global__ __launch_bounds__(256) void kf_raster(const DevItem* __restrict__ ite
                     const uint8_t* src = cell_table + ((key * 9 + j) * PARTS + h) * TB;
                     if constexpr (SUB) {
                         if (s_src[k] != 0xFFFFFFFFu)
-                            src = reinterpret_cast<const uint8_t*>(item_rows + s_src[k]) + j * (PARTS == 1 ? 2 : S) + 4 * h;
+                            src = reinterpret_cast<const uint8_t*>(smoothed_cell(s_src[k])) + j * (PARTS == 1 ? 2 : S) + 4 * h;
                     }
                     __builtin_memcpy(&m[j], src, TB);
                 }

@@ -95,8 +95,9 @@ __global__ void kt_cell(const uint32_t* __restrict__ mask, uint8_t* __restrict__
     if (key >= kKeys) return;
     const uint32_t* rows = mask + (size_t)key * mask_w(S);
     uint64_t m[9] = {};
-    cell_mask_rows<S>([&](int r) { return rows[r]; },
-                      [&](int j, int ky, uint32_t bits) { m[j] |= (uint64_t)bits << (ky * (TB == 2 ? S : 8)); });
+    cell_mask_rows<S, mask_kmin(S), mask_kmin(S), mask_w(S)>(
+        [&](int r) { return rows[r]; },
+        [&](int j, int ky, uint32_t bits) { m[j] |= (uint64_t)bits << (ky * (TB == 2 ? S : 8)); });
     for (int j = 0; j < 9; j++) __builtin_memcpy(cell + (size_t)(key * 9 + j) * TB, &m[j], TB);
 }
 
@@ -112,7 +113,7 @@ __global__ void kt_info(const uint32_t* __restrict__ mask, int S, uint8_t* __res
 {
     int key = blockIdx.x * blockDim.x + threadIdx.x;
     if (key >= kKeys) return;
-    info[key] = (uint8_t)coverage_info(mask + (size_t)key * mask_w(S), S);
+    info[key] = (uint8_t)coverage_info(mask + (size_t)key * mask_w(S), S, mask_kmin(S), mask_kmin(S), mask_w(S));
 }
 
 

@@ -735,16 +735,18 @@ __host__ __device__ inline uint32_t tri_row_bits(int ax, int ay, int bx, int by,
 // sy = 128 (kmin + r) + 64), ORed into cov[r].  Along the rows an edge's
 // column bound moves by a fixed rational step, so each bound is kept as a
 // quotient and remainder and advanced by one exact step per row instead of
-// a division per row.  Same bits as tri_row_bits on every row.
-template <int MW>
-__host__ __device__ inline void tri_rows_or(int ax, int ay, int bx, int by, int cx, int cy, int kmin, uint32_t* cov)
+// a division per row.  Same bits as tri_row_bits on every row.  tri_rect_or:
+// on a grid of ROWS rows from y0 and COLS columns from x0.
+template <int ROWS, int COLS>
+__host__ __device__ inline void tri_rect_or(int ax, int ay, int bx, int by, int cx, int cy, int x0, int y0,
+                                            uint32_t* cov)
 {
     const int ymin = min(ay, min(by, cy)), ymax = max(ay, max(by, cy));
-    const int sy0 = 128 * kmin + 64;
+    const int sx0 = 128 * x0 + 64, sy0 = 128 * y0 + 64;
     // per edge: dy > 0 bounds hi, dy < 0 bounds lo, dy == 0 admits a range
     // of rows.  q, rem: floor of the bound's numerator over D = 128 |dy|.
     int q[3], rem[3], qs[3], rs[3], D[3], kind[3];  // kind: 1 hi, -1 lo, 0 horizontal
-    int ylo = sy0, yhi = sy0 + 128 * (MW - 1);       // rows the horizontal edges admit (sample y)
+    int ylo = sy0, yhi = sy0 + 128 * (ROWS - 1);     // rows the horizontal edges admit (sample y)
     const int px_[3] = { ax, bx, cx }, py_[3] = { ay, by, cy };
 #pragma unroll
     for (int e = 0; e < 3; e++) {
@@ -760,17 +762,17 @@ __host__ __device__ inline void tri_rows_or(int ax, int ay, int bx, int by, int 
             else yhi = ylo - 1;                      // (a point: nothing)
             continue;
         }
-        // numerator at row 0: N = dx (sy0 - py) + dy (px - sy0); hi uses N - 1, lo uses N
-        const int N0 = dx * (sy0 - py) + dy * (px - sy0) - (dy > 0 ? 1 : 0);
+        // numerator at row 0: N = dx (sy0 - py) + dy (px - sx0); hi uses N - 1, lo uses N
+        const int N0 = dx * (sy0 - py) + dy * (px - sx0) - (dy > 0 ? 1 : 0);
         q[e] = floor_div(N0, D[e]);
         rem[e] = N0 - q[e] * D[e];
         qs[e] = floor_div(128 * dx, D[e]);
         rs[e] = 128 * dx - qs[e] * D[e];
     }
 #pragma unroll
-    for (int r = 0; r < MW; r++) {
+    for (int r = 0; r < ROWS; r++) {
         const int sy = sy0 + 128 * r;
-        int lo = 0, hi = MW - 1;
+        int lo = 0, hi = COLS - 1;
 #pragma unroll
         for (int e = 0; e < 3; e++) {
             if (kind[e] > 0) hi = min(hi, q[e]);
@@ -786,6 +788,12 @@ __host__ __device__ inline void tri_rows_or(int ax, int ay, int bx, int by, int 
         if (sy >= ymin && sy <= ymax && sy >= ylo && sy <= yhi && lo <= hi)
             cov[r] |= ((2u << hi) - 1u) & ~((1u << lo) - 1u);
     }
+}
+
+template <int MW>
+__host__ __device__ inline void tri_rows_or(int ax, int ay, int bx, int by, int cx, int cy, int kmin, uint32_t* cov)
+{
+    tri_rect_or<MW, MW>(ax, ay, bx, by, cx, cy, kmin, kmin, cov);
 }
 
 // The coverage rows of a counter-clockwise polygon that ear clipping has
@@ -810,10 +818,11 @@ __host__ __device__ inline void tri_rows_or(int ax, int ay, int bx, int by, int 
 // are visited (a smoothed cell's 8 to 16 edges cross one or two each, of 10
 // rows at 4x and 18 at 8x), the crossing's column from the exact numerator
 // by a reciprocal and one step: toggle(r, mask) receives each.
-template <int MW, class V, class Toggle>
-__host__ __device__ inline int poly_rows_cross(const V* P, int stride, int m, int S2, int kmin, Toggle toggle)
+// The grid has ROWS rows from y0 and COLS columns from x0.
+template <int ROWS, int COLS, class V, class Toggle>
+__host__ __device__ inline int poly_rows_cross(const V* P, int stride, int m, int S2, int x0, int y0, Toggle toggle)
 {
-    const int s0 = 128 * kmin + 64;  // the first sample row, and column
+    const int sx0 = 128 * x0 + 64, sy0 = 128 * y0 + 64;  // the first sample column and row
     int wsum = 0;
     V A = P[stride * (m - 1)];
     for (int k = 0; k < m; k++) {
@@ -829,9 +838,9 @@ __host__ __device__ inline int poly_rows_cross(const V* P, int stride, int m, in
         py *= S2;
         const int dx = qx * S2 - px, dy = qy * S2 - py;
         // rows sy with py <= sy < qy
-        int r = (py - s0 + 127) >> 7, end = (py + dy - s0 + 127) >> 7;
+        int r = (py - sy0 + 127) >> 7, end = (py + dy - sy0 + 127) >> 7;
         r = r < 0 ? 0 : r;
-        end = end > MW ? MW : end;
+        end = end > ROWS ? ROWS : end;
         if (r >= end) continue;
         const int D = 128 * dy;
 #ifdef __HIP_DEVICE_COMPILE__
@@ -842,13 +851,13 @@ __host__ __device__ inline int poly_rows_cross(const V* P, int stride, int m, in
         // columns left of the crossing: 0 .. floor(N / D); an upward edge's
         // covered side (N = e - 1 above 0) and a downward one's uncovered
         // side end at the same column
-        int N = dx * (s0 + 128 * r - py) + dy * (px - s0) - 1;
+        int N = dx * (sy0 + 128 * r - py) + dy * (px - sx0) - 1;
         for (; r < end; r++) {
             int q = (int)floorf((float)N * inv);  // within 1 of the quotient
             const int rem = N - q * D;
             if (rem < 0) q--;
             else if (rem >= D) q++;
-            const int cols = q < -1 ? 0 : q >= MW - 1 ? MW : q + 1;
+            const int cols = q < -1 ? 0 : q >= COLS - 1 ? COLS : q + 1;
             if (cols > 0) {
                 toggle(r, cols >= 32 ? 0xFFFFFFFFu : (1u << cols) - 1u);
                 wsum += sign * cols;
@@ -862,7 +871,7 @@ __host__ __device__ inline int poly_rows_cross(const V* P, int stride, int m, in
 template <int MW, class V>
 __host__ __device__ inline int poly_rows_xor(const V* P, int stride, int m, int S2, int kmin, uint32_t* cov)
 {
-    return poly_rows_cross<MW>(P, stride, m, S2, kmin, [&](int r, uint32_t mask) { cov[r] ^= mask; });
+    return poly_rows_cross<MW, MW>(P, stride, m, S2, kmin, kmin, [&](int r, uint32_t mask) { cov[r] ^= mask; });
 }
 
 }  // namespace dpx
