@@ -411,29 +411,29 @@ __global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const D
     static_assert(COLS <= 32, "a row of samples is a word");
     constexpr int PITCH = 257;  // of the rows: adjacent rows of a cell in adjacent banks
     __shared__ int s_nblk;
-    __shared__ uint32_t s_g32[GY * RWW];
-    __shared__ uint16_t s_list[RTX * RTY];
+    __shared__ uint8_t s_list[RTX * RTY];
     __shared__ int s_bin[16];  // own cells to smooth per hull size
     __shared__ int s_nlist, s_nclip;
     __shared__ uint8_t s_clip[RTX * RTY];  // columns whose polygon is clipped
-    __shared__ uint8_t s_m[RTX * RTY];     // vertices of a column's polygon; 0 once its clipping has failed
+    __shared__ uint8_t s_m[RTX * RTY];     // vertices of a column's polygon; 0 once its clipping has failed; at last its summary
     // vertex k of column t at [k * 256 + t]; a hull has at most 8 vertices,
     // its smoothed polygon at most 16, within the cells around (-64 .. 127)
     __shared__ uint16_t s_poly[16 * 256];
-    // sample row r of column t at [r * PITCH + t], then its masks and summary; first the walk window
-    constexpr int COV = (ROWS + 1 > RW ? ROWS + 1 : RW) * PITCH, WALK_WORDS = WALK ? WalkWindow<TX>::BYTES / 4 : 0;
+    // sample row r of column t at [r * PITCH + t], then its masks; first the walk window
+    constexpr int COV = (S > kMaxCellScale || ROWS > RW ? ROWS : RW) * PITCH, WALK_WORDS = WALK ? WalkWindow<TX>::BYTES / 4 : 0;
     // What is needed until the polygons are made lies where the rows come
     // after them (the walk window is read meanwhile and keeps it apart): a
     // block more fits each CU.
     constexpr int HULL_WORDS = RCX * RCY * (int)(sizeof(HullBits) / 4), AUX_WORDS = AY * RWW, P_WORDS = (GY + 1) * RWW;
-    constexpr int EARLY = HULL_WORDS + AUX_WORDS + P_WORDS + ((GY + 1) * RDB + 1) / 2;
+    constexpr int G_WORDS = GY * RWW, EARLY = HULL_WORDS + AUX_WORDS + P_WORDS + G_WORDS + ((GY + 1) * RDB + 1) / 2;
     constexpr int LATE = COV > WALK_WORDS ? COV : WALK_WORDS;
     __shared__ __align__(8) uint32_t s_cov[WALK ? LATE + EARLY + 1 : LATE > EARLY ? LATE : EARLY];
     uint32_t* s_early = s_cov + (WALK ? (LATE + 1) / 2 * 2 : 0);
     HullBits* s_hull = reinterpret_cast<HullBits*>(s_early);
     uint32_t* s_aux32 = s_early + HULL_WORDS;
     uint32_t* s_p32 = s_aux32 + AUX_WORDS;
-    uint16_t* s_blk = reinterpret_cast<uint16_t*>(s_p32 + P_WORDS);
+    uint32_t* s_g32 = s_p32 + P_WORDS;
+    uint16_t* s_blk = reinterpret_cast<uint16_t*>(s_g32 + G_WORDS);
     const uint8_t* s_g = reinterpret_cast<const uint8_t*>(s_g32);
 
     const int t = threadIdx.x;
@@ -485,7 +485,7 @@ __global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const D
         if (t == 15) s_nlist = acc;
     }
     __syncthreads();
-    if (my_n >= 0) s_list[s_bin[15 - my_n] + my_rank] = (uint16_t)t;
+    if (my_n >= 0) s_list[s_bin[15 - my_n] + my_rank] = (uint8_t)t;
     __syncthreads();
     const int nlist = s_nlist;
     if (nlist == 0) return;  // (uniform)
@@ -569,7 +569,7 @@ __global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const D
 #pragma unroll
             for (int r = 0; r < RW; r++) C[PITCH * r] = word[r];
         } else {
-            C[PITCH * ROWS] = info;
+            s_m[t] = (uint8_t)info;
         }
     }
     __syncthreads();
@@ -578,7 +578,8 @@ __global__ __launch_bounds__(256, smooth_blocks(S, WALK)) void kf_smooth(const D
     for (int k = t; k < nlist * RW; k += 256) {
         const int c = k / RW, r = k - c * RW, own = s_list[c];
         const uint32_t cell = (uint32_t)(y0 + own / RTX) * (uint32_t)it.W + (uint32_t)(x0 + own % RTX);
-        dst[(size_t)cell * RW + r] = s_cov[PITCH * r + c];
+        if constexpr (S > kMaxCellScale) dst[(size_t)cell * RW + r] = r == ROWS ? s_m[c] : s_cov[PITCH * r + c];
+        else dst[(size_t)cell * RW + r] = s_cov[PITCH * r + c];
     }
 }
 
