@@ -477,8 +477,8 @@ __global__ __launch_bounds__(256) void k_export_vbo(ImgView im, const dpx_point*
 // for the frame's raster and for the GLUT window (display()
 // callbacks.cpp:39-72, renderCuda simpleVBO.cpp:185-440): a sample takes the
 // colour of the highest-index cell (the last one drawn) with a triangle that
-// covers it.  Cells reach at most 0.34 past their unit square, so the cells
-// around the sample's own are the candidates.
+// covers it.  Cells reach at most three quarters of a cell past their unit
+// square, so the cells around the sample's own are the candidates.
 //
 // All coordinates are whole numbers of a unit such that a cell is `unit` of
 // them: 1/(128 scale) of a cell for the raster, 1/(512 sc) for the window
@@ -551,13 +551,19 @@ __device__ __noinline__ uint32_t tri_sample_any(ImgView im, const dpx_point* __r
 // coverage rule in k (covered: all three above 0), so that a sample's test of
 // a triangle is six multiply-adds; and how far the cells reach beyond their
 // squares, which keeps most pixels to one to four of the cells around them.
-// A vertex within half a cell of its cell and a sample within three cells
-// keep every term in 31 bits and the factors in 24; a cell of a caller's
-// diagram beyond that, and scales with more cells, take tri_sample_any.
+// A vertex within a smoothed cell's reach, and a sample that lies up to two
+// cells and a pixel from its candidates, keep every term in 31 bits and the
+// factors in 24; a cell of a caller's diagram beyond that, and scales with more
+// cells, take tri_sample_any.  (With half a cell for the reach, dithers of
+// nearly similar colours took that in most blocks: the raster of 256x224 at 8x
+// 546 us, so 151, the window at 8x 719, so 96.)
 // Bound by the instructions of the tests; straight from memory in 64 bits
 // the 1200x800 window of a smoothed 256x224 frame took 221 us, so 44.
 constexpr int kTris = kCellSize / 3;
-constexpr int kTriLow = -32, kTriHigh = 96;  // 1/64 units
+constexpr int kTriLow = std::min(kReachXLow, kReachYLow), kTriHigh = std::max(kReachXHigh, kReachYHigh);  // 1/64 units
+constexpr long long kTriUnitMost = 512 * 3200, kTriStep = 8 * 6400;  // of the window, the larger ones
+static_assert((kTriHigh - kTriLow) * (2 * (2 * kTriUnitMost + kTriStep) + 2 * kTriHigh * kTriUnitMost / 64) < 1LL << 31 &&
+              2 * kTriUnitMost + kTriStep < 1 << 23, "an edge function and its factors");
 struct TriEdge {
     uint32_t d;  // dx | dy << 16
     int k;
