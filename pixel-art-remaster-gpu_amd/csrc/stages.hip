@@ -11,6 +11,8 @@
 #include <string.h>
 
 #include <algorithm>
+#include <numeric>
+#include <type_traits>
 
 #include "common.hpp"
 #include "geom.hpp"
@@ -762,26 +764,33 @@ __global__ __launch_bounds__(16 * TY) void k_tri(ImgView im, const dpx_point* __
     *reinterpret_cast<uint32_t*>(out + (size_t)row * out_stride + (size_t)X * 4) = tri_average<NS>(col);
 }
 
-// Views that put so many cells into a block that they do not fit LDS (scales
-// below 1): a thread per pixel, the cells around all of its samples read
-// once from the diagram, each triangle tested against every sample that no
-// cell has covered yet.
-template <int NS>
+// A thread per pixel, the cells around all of its samples read once from the
+// diagram, each triangle tested against every sample that no cell has covered
+// yet.  For views that put so many cells into a block that they do not fit LDS
+// (scales below 1), and for one sample a pixel up to 1x, where a tile would set
+// up two cells' triangles for each pixel that it tests (256x224 at 1x: the
+// raster 39 us, so 31, the window 46, so 30).  SMALL: units of at most
+// kTriSmallUnit a cell and places below 2^26, so that they are 32-bit, and so
+// are the tests of triangles within four cells of their own.
+constexpr int kTriSmallUnit = 4096, kTriSmallVertex = 256;  // (coordinates below 511 * 64 apart: 2 * 32704^2 < 2^31)
+constexpr int kTriBatch = 4;
+template <int NS, bool SMALL>
 __global__ __launch_bounds__(256) void k_tri_far(ImgView im, const dpx_point* __restrict__ diagram,
                                                  const int32_t* __restrict__ edge_count, TriGeom v,
                                                  uint8_t* __restrict__ out, int out_stride)
 {
+    using Place = std::conditional_t<SMALL, int, long long>;
     const int X = blockIdx.x * 16 + (threadIdx.x & 15), Y = blockIdx.y * 16 + (threadIdx.x >> 4);
     if (X >= v.W || Y >= v.H) return;
-    const long long unit = v.unit;
-    long long px[NS], py[NS], i0 = 0, i1 = 0, j0 = 0, j1 = 0;
+    const Place unit = v.unit, u = v.unit / 64;
+    Place px[NS], py[NS], i0 = 0, i1 = 0, j0 = 0, j1 = 0;
     uint32_t col[NS];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
-        px[s] = (long long)v.step * X + v.ox[s];
-        py[s] = (long long)v.step * Y + v.oy[s];
+        px[s] = (Place)v.step * X + (Place)v.ox[s];
+        py[s] = (Place)v.step * Y + (Place)v.oy[s];
         col[s] = 0xFF000000u;  // clear colour (0,0,0,1), main.cpp:260
-        const long long ci = floor_div(px[s], unit), cj = floor_div(py[s], unit);
+        const Place ci = floor_div(px[s], unit), cj = floor_div(py[s], unit);
         if (s == 0 || ci < i0) i0 = ci;
         if (s == 0 || ci > i1) i1 = ci;
         if (s == 0 || cj < j0) j0 = cj;
@@ -794,26 +803,46 @@ __global__ __launch_bounds__(256) void k_tri_far(ImgView im, const dpx_point* __
     j1 = j1 + 1 > im.H - 1 ? im.H - 1 : j1 + 1;
     const int cc = colour_channels(im);
     uint32_t left = (1u << NS) - 1u;
-    for (long long j = j1; j >= j0 && left; j--)
-        for (long long i = i1; i >= i0 && left; i--) {
+    for (Place j = j1; j >= j0 && left; j--)
+        for (Place i = i1; i >= i0 && left; i--) {
             const size_t k = (size_t)j * im.W + (size_t)i;
             const int nt = cell_triangles(edge_count[k]);
             const dpx_point* c = &diagram[k * kCellSize];
             const float fi = (float)i, fj = (float)j;
             uint32_t hit = 0;
-            for (int t = 0; t < nt && (left & ~hit); t++) {
-                long long w[6];
+            for (int t0 = 0; t0 < nt && (left & ~hit); t0 += kTriBatch) {
+                // (a batch's loads before its first test: a triangle at a time
+                // waits a memory latency for each)
+                dpx_point p[3 * kTriBatch];
 #pragma unroll
-                for (int q = 0; q < 3; q++) {
-                    const dpx_point p = c[3 * t + q];
-                    w[2 * q] = (long long)(int)((p.x - fi) * 64.0f) * (v.unit / 64);
-                    w[2 * q + 1] = (long long)(int)((p.y - fj) * 64.0f) * (v.unit / 64);
+                for (int q = 0; q < 3 * kTriBatch; q++) p[q] = c[min(3 * t0 + q, 3 * nt - 1)];
+#pragma unroll
+                for (int b = 0; b < kTriBatch; b++) {
+                    if (t0 + b >= nt || !(left & ~hit)) break;
+                    int w[6], most = 0;
+#pragma unroll
+                    for (int q = 0; q < 3; q++) {
+                        w[2 * q] = (int)((p[3 * b + q].x - fi) * 64.0f);
+                        w[2 * q + 1] = (int)((p[3 * b + q].y - fj) * 64.0f);
+                    }
+                    auto test = [&](auto one) {
+                        using T = decltype(one);
+#pragma unroll
+                        for (int s = 0; s < NS; s++)
+                            if (((left & ~hit) >> s) & 1u)
+                                if (tri_covers<T>(w[0] * (T)u, w[1] * (T)u, w[2] * (T)u, w[3] * (T)u, w[4] * (T)u,
+                                                  w[5] * (T)u, (T)(px[s] - i * unit), (T)(py[s] - j * unit)))
+                                    hit |= 1u << s;
+                    };
+                    if constexpr (SMALL) {
+#pragma unroll
+                        for (int q = 0; q < 6; q++) most = max(most, max(w[q], -1 - w[q]));
+                        if (most < kTriSmallVertex) test(0);
+                        else test(0LL);
+                    } else {
+                        test(0LL);
+                    }
                 }
-#pragma unroll
-                for (int s = 0; s < NS; s++)
-                    if (((left & ~hit) >> s) & 1u)
-                        if (tri_covers(w[0], w[1], w[2], w[3], w[4], w[5], px[s] - i * unit, py[s] - j * unit))
-                            hit |= 1u << s;
             }
             if (hit) {
                 const uint32_t rgba = cell_rgba(load_px(im, (int)i, (int)j), cc);
@@ -827,9 +856,19 @@ __global__ __launch_bounds__(256) void k_tri_far(ImgView im, const dpx_point* __
     *reinterpret_cast<uint32_t*>(out + (size_t)row * out_stride + (size_t)X * 4) = tri_average<NS>(col);
 }
 
-void launch_tri(const ImgView& im, const dpx_point* diagram, const int32_t* edge_count, const TriGeom& v, int samples,
+void launch_tri(const ImgView& im, const dpx_point* diagram, const int32_t* edge_count, TriGeom v, int samples,
                 uint8_t* out, int out_stride, hipStream_t stream)
 {
+    // the coarsest units in which everything is whole (a vertex lies at a 64th of a cell)
+    long long g = std::gcd((long long)(v.unit / 64), (long long)v.step), far_off = 0;
+    for (int s = 0; s < samples; s++) g = std::gcd(g, std::gcd(v.ox[s], v.oy[s]));
+    v.unit /= (int)g;
+    v.step /= (int)g;
+    for (int s = 0; s < samples; s++) {
+        v.ox[s] /= g;
+        v.oy[s] /= g;
+        far_off = std::max({ far_off, std::abs(v.ox[s]), std::abs(v.oy[s]) });
+    }
     // cells that n output pixels reach on one axis: their own, a part at each
     // end and one around each side
     auto reach = [&](int n) { return ((long long)n * v.step - 1) / v.unit + 4; };
@@ -840,10 +879,11 @@ void launch_tri(const ImgView& im, const dpx_point* diagram, const int32_t* edge
     const int ty = tall ? 16 : 4, cap = v.quads ? 0 : (int)std::min(reach(16) * reach(ty), 1LL << 20);
     const size_t lds = v.quads ? 0 : lds_of(ty);
     const dim3 grid((unsigned)((v.W + 15) / 16), (unsigned)((v.H + ty - 1) / ty));
-    if (lds > 60 * 1024) {
+    const bool small = v.unit <= kTriSmallUnit && far_off + (long long)v.step * std::max(v.W, v.H) < 1LL << 26;
+    if (lds > 60 * 1024 || (samples == 1 && v.unit <= v.step && !v.quads)) {
         const dim3 far((unsigned)((v.W + 15) / 16), (unsigned)((v.H + 15) / 16));
-        hipLaunchKernelGGL(samples == 4 ? k_tri_far<4> : k_tri_far<1>, far, dim3(256), 0, stream, im, diagram,
-                           edge_count, v, out, out_stride);
+        auto fn = samples == 4 ? (small ? k_tri_far<4, true> : k_tri_far<4, false>) : small ? k_tri_far<1, true> : k_tri_far<1, false>;
+        hipLaunchKernelGGL(fn, far, dim3(256), 0, stream, im, diagram, edge_count, v, out, out_stride);
         return;
     }
     auto fn = samples == 4 ? (tall ? k_tri<4, 16> : k_tri<4, 4>) : (tall ? k_tri<1, 16> : k_tri<1, 4>);
