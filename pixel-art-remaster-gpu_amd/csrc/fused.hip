@@ -676,16 +676,23 @@ dim3 tile_grid(const std::vector<DevItem>& dev, int TX, int TY, int* grid3d, std
 // (item, strip).
 dim3 strip_grid(const std::vector<DevItem>& dev, int max_rows, int* grid3d, std::vector<uint2>* map)
 {
-    const uint32_t n0 = graph_split(dev[0].W, dev[0].H, max_rows).strips;
+    std::vector<uint32_t> strips(dev.size());
+    uint32_t total = 0;
     bool same = dev.size() <= 65535;
-    for (const DevItem& d : dev) same = same && graph_split(d.W, d.H, max_rows).strips == n0;
+    for (size_t k = 0; k < dev.size(); k++) {
+        const bool as_before = k && dev[k].W == dev[k - 1].W && dev[k].H == dev[k - 1].H;
+        strips[k] = as_before ? strips[k - 1] : graph_split(dev[k].W, dev[k].H, max_rows).strips;
+        same = same && strips[k] == strips[0];
+        total += strips[k];
+    }
     map->clear();
     *grid3d = same ? 1 : 0;
-    if (same) return dim3(n0, 1, (unsigned)dev.size());
+    if (same) return dim3(strips[0], 1, (unsigned)dev.size());
+    map->resize(total);
+    uint2* at = map->data();
     for (size_t k = 0; k < dev.size(); k++)
-        for (uint32_t q = 0, n = graph_split(dev[k].W, dev[k].H, max_rows).strips; q < n; q++)
-            map->push_back(make_uint2((unsigned)k, q));
-    return dim3((unsigned)map->size(), 1, 1);
+        for (uint32_t q = 0; q < strips[k]; q++) *at++ = make_uint2((unsigned)k, q);
+    return dim3(total, 1, 1);
 }
 
 }  // namespace
@@ -1336,31 +1343,29 @@ struct NaPut {
     uint32_t gslot;  // in the grouped item array
     uint32_t gpos;   // gslot - the group's first slot (the raster launch's items)
     uint32_t gstrip, rtile;
+    uint32_t strips;
 };
 constexpr int kNaPutChunk = 32;
 struct NaPutArgs {
-    uint32_t n;
-    int grows;  // rows of the graph launch's blocks
     NaPut it[kNaPutChunk];
 };
 static_assert(sizeof(NaPutArgs) <= 4000, "kernel arguments stay under 4 KB");
 
+// A block per item.  (One block that took the items in turn: 17 us a launch of
+// 32, and 21 when each item's strips were counted here.)
 __global__ __launch_bounds__(256) void k_na_put(NaPutArgs a, DevItem* __restrict__ items,
                                                 DevItem* __restrict__ group_items, uint2* __restrict__ gmap,
                                                 uint2* __restrict__ rmap)
 {
-    for (uint32_t i = 0; i < a.n; i++) {
-        const NaPut& p = a.it[i];
-        if (threadIdx.x == 0) {
-            items[p.index] = p.d;
-            group_items[p.gslot] = p.d;
-        }
-        const uint32_t gs = graph_split(p.d.W, p.d.H, a.grows).strips;
-        for (uint32_t t = threadIdx.x; t < gs; t += blockDim.x) gmap[p.gstrip + t] = make_uint2(p.index, t);
-        const uint32_t rx = (uint32_t)(p.d.W + kNaTX - 1) / kNaTX, ry = (uint32_t)(p.d.H + kNaTY - 1) / kNaTY;
-        for (uint32_t t = threadIdx.x; t < rx * ry; t += blockDim.x)
-            rmap[p.rtile + t] = make_uint2(p.gpos, (t / rx) << 16 | (t % rx));
+    const NaPut& p = a.it[blockIdx.x];
+    if (threadIdx.x == 0) {
+        items[p.index] = p.d;
+        group_items[p.gslot] = p.d;
     }
+    for (uint32_t t = threadIdx.x; t < p.strips; t += blockDim.x) gmap[p.gstrip + t] = make_uint2(p.index, t);
+    const uint32_t rx = (uint32_t)(p.d.W + kNaTX - 1) / kNaTX, ry = (uint32_t)(p.d.H + kNaTY - 1) / kNaTY;
+    for (uint32_t t = threadIdx.x; t < rx * ry; t += blockDim.x)
+        rmap[p.rtile + t] = make_uint2(p.gpos, (t / rx) << 16 | (t % rx));
 }
 
 constexpr int kNaMaxDevices = 64;
@@ -1460,11 +1465,11 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
     uint32_t gnext[2 * (kMaxScale + 1)] = {}, gtnext[2 * (kMaxScale + 1)] = {};
     NaPutArgs args;
     memset(&args, 0, sizeof(args));
-    args.grows = grows;
     uint64_t goff = 0;
     uint32_t gt = 0;
+    int n_put = 0;
     for (int k = 0; k < n_items; k++) {
-        NaPut& p = args.it[args.n++];
+        NaPut& p = args.it[n_put++];
         (void)make_dev_item(items[k], k, d_out, goff, p.d);  // (validated in pass 1)
         const int g = 2 * p.d.scale + p.d.subdivide;
         p.index = (uint32_t)k;
@@ -1472,12 +1477,13 @@ extern "C" int dpx_batch_run_noalloc(const uint8_t* d_in, uint8_t* d_out, const 
         p.gslot = gslot0[g] + p.gpos;
         p.gstrip = gt;
         p.rtile = gtile0[g] + gtnext[g];
-        gt += graph_split(p.d.W, p.d.H, grows).strips;
+        p.strips = graph_split(p.d.W, p.d.H, grows).strips;
+        gt += p.strips;
         gtnext[g] += (uint32_t)(((p.d.W + kNaTX - 1) / kNaTX) * ((p.d.H + kNaTY - 1) / kNaTY));
         goff += align_up((size_t)p.d.W * p.d.H, 256);
-        if (args.n == kNaPutChunk || k == n_items - 1) {
-            hipLaunchKernelGGL(k_na_put, dim3(1), dim3(256), 0, stream, args, d_items, d_gitems, d_gmap, d_rmap);
-            args.n = 0;
+        if (n_put == kNaPutChunk || k == n_items - 1) {
+            hipLaunchKernelGGL(k_na_put, dim3(n_put), dim3(256), 0, stream, args, d_items, d_gitems, d_gmap, d_rmap);
+            n_put = 0;
         }
     }
     hipLaunchKernelGGL(kf_graph, dim3((unsigned)graph_strips), dim3(64), 0, stream, d_items, d_gmap, 0,
