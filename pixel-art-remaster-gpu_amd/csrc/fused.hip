@@ -393,6 +393,7 @@ __global__ __launch_bounds__(64) void kf_graph(const DevItem* __restrict__ items
     const DevItem it = items[at.item];
     const uint32_t strip = (uint32_t)at.ty << 16 | (uint32_t)at.tx;
     const GraphSplit sp = graph_split(it.W, it.H, max_rows);
+    if (strip >= sp.strips) return;  // (an item of fewer strips than the launch has for each)
     if (it.flags & DPX_INDEXED) {
         // the lane words of the 256 palette entries
         const uint32_t order = (it.flags & DPX_RGB) ? 0x03000102u : 0x03020100u;
@@ -664,30 +665,37 @@ dim3 tile_grid(const std::vector<DevItem>& dev, int TX, int TY, int* grid3d, std
     map->clear();
     *grid3d = same ? 1 : 0;
     if (same) return dim3(tx0, ty0, (unsigned)dev.size());
+    size_t total = 0;
+    for (const DevItem& d : dev) total += (size_t)((unsigned)(d.W + TX - 1) / TX) * ((unsigned)(d.H + TY - 1) / TY);
+    map->resize(total);
+    uint2* at = map->data();
     for (size_t k = 0; k < dev.size(); k++) {
         const unsigned tx = (unsigned)(dev[k].W + TX - 1) / TX, ty = (unsigned)(dev[k].H + TY - 1) / TY;
         for (unsigned y = 0; y < ty; y++)
-            for (unsigned x = 0; x < tx; x++) map->push_back(make_uint2((unsigned)k, y << 16 | x));
+            for (unsigned x = 0; x < tx; x++) *at++ = make_uint2((unsigned)k, y << 16 | x);
     }
-    return dim3((unsigned)map->size(), 1, 1);
+    return dim3((unsigned)total, 1, 1);
 }
 
-// The same for kf_graph's strips: (strips, 1, items), or 1-D with a map to
-// (item, strip).
+// The same for kf_graph's strips: (strips, 1, items) when all items have nearly
+// as many as the most, else 1-D with a map to (item, strip).  The waves past an
+// item's last strip end at once; an eighth of them costs less than a map, which
+// is uploaded whenever the items change (64 frames of 248 to 256 columns at 2x,
+// other items each call: 78 us with a map; five of 640 and 639 columns:
+// 59).
 dim3 strip_grid(const std::vector<DevItem>& dev, int max_rows, int* grid3d, std::vector<uint2>* map)
 {
     std::vector<uint32_t> strips(dev.size());
-    uint32_t total = 0;
-    bool same = dev.size() <= 65535;
+    uint32_t total = 0, most = 0;
     for (size_t k = 0; k < dev.size(); k++) {
         const bool as_before = k && dev[k].W == dev[k - 1].W && dev[k].H == dev[k - 1].H;
         strips[k] = as_before ? strips[k - 1] : graph_split(dev[k].W, dev[k].H, max_rows).strips;
-        same = same && strips[k] == strips[0];
+        most = std::max(most, strips[k]);
         total += strips[k];
     }
     map->clear();
-    *grid3d = same ? 1 : 0;
-    if (same) return dim3(strips[0], 1, (unsigned)dev.size());
+    *grid3d = dev.size() <= 65535 && (uint64_t)most * dev.size() <= (uint64_t)total + total / 8 ? 1 : 0;
+    if (*grid3d) return dim3(most, 1, (unsigned)dev.size());
     map->resize(total);
     uint2* at = map->data();
     for (size_t k = 0; k < dev.size(); k++)

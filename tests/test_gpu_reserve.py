@@ -20,7 +20,8 @@ def batch(D, torch, sizes, S):
 
 
 # the raster tile grid is the same for a batch's items, the number of strips is not
-@pytest.mark.parametrize("sizes", [[(640, 480)] * 4 + [(639, 480)], [(60 - k % 9, 31) for k in range(3000)]])
+@pytest.mark.parametrize("sizes", [[(640, 480)] * 4 + [(639, 480)], [(60 - k % 9, 31) for k in range(3000)],
+                                   [(64, 860)] + [(49, 860)] * 39])  # (the last needs a map of 13,900 strips)
 def test_reserved_context_does_not_wait(gpu, D, O, sizes):
     torch = gpu
     S = 2
