@@ -148,8 +148,9 @@ int dpx_stage_components(const uint8_t* d_graph, int width, int height, int32_t*
 /* border chains of a resolved graph: extractBorderPoints cc_functions.cu:348-503
  * (its CClist / CCsizes outputs).  Chain k is d_nodes[sum of d_sizes[0..k-1] ..]
  * of d_sizes[k] node indices j*width+i, chains in the order the row-major scan
- * starts them.  d_scratch: width*height bytes, 4-byte aligned for frames of
- * more than about 620,000 nodes.  Working memory of about 340 bytes per node
+ * starts them.  d_scratch is kept for callers of earlier versions and is not
+ * used, but still checked: not null, 4-byte aligned for frames of more than
+ * 622,336 nodes.  Working memory of about 340 bytes per node
  * is allocated and freed in stream order (hipMallocAsync / hipFreeAsync on
  * `stream`).
  * d_counts[3] receives the number of chains, of nodes and a status (0;

@@ -109,38 +109,32 @@ struct TileAt {
     int item, tx, ty;
 };
 
-// With RUN > 1 the blocks are permuted in groups of 8 * RUN: the hardware
-// hands consecutive blocks to the 8 XCDs in turn, and within a group XCD x
-// is given the RUN consecutive tiles x * RUN .. x * RUN + RUN - 1 (a row of
-// horizontally adjacent tiles), so the input and graph lines that adjacent
-// tiles share are fetched into one XCD's L2 once, not into several.  Blocks
-// past the last whole group keep their place.
+// The blocks are permuted in groups of 8 * RUN: the hardware hands consecutive
+// blocks to the 8 XCDs in turn, and within a group XCD x is given the RUN
+// consecutive tiles x * RUN .. x * RUN + RUN - 1 (a row of horizontally
+// adjacent tiles), so the input and graph lines that adjacent tiles share are
+// fetched into one XCD's L2 once, not into several.  Blocks past the last
+// whole group keep their place.
 template <int RUN>
 __device__ inline TileAt locate_tile(const uint2* __restrict__ tile_map, int grid3d)
 {
-    if constexpr (RUN == 1) {
-        if (grid3d) return TileAt{ (int)blockIdx.z, (int)blockIdx.x, (int)blockIdx.y };
-        const uint2 m = tile_map[blockIdx.x];
-        return TileAt{ (int)m.x, (int)(m.y & 0xFFFFu), (int)(m.y >> 16) };
-    } else {
-        const uint32_t n = gridDim.x * gridDim.y * gridDim.z;
-        uint32_t b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-        if (b < n / (8 * RUN) * (8 * RUN)) {
-            const uint32_t w = b % (8 * RUN);
-            b += (w % 8) * RUN + w / 8 - w;
-        }
-        if (grid3d) {
-            const uint32_t plane = gridDim.x * gridDim.y, r = b % plane;
-            return TileAt{ (int)(b / plane), (int)(r % gridDim.x), (int)(r / gridDim.x) };
-        }
-        const uint2 m = tile_map[b];
-        return TileAt{ (int)m.x, (int)(m.y & 0xFFFFu), (int)(m.y >> 16) };
+    const uint32_t n = gridDim.x * gridDim.y * gridDim.z;
+    uint32_t b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    if (b < n / (8 * RUN) * (8 * RUN)) {
+        const uint32_t w = b % (8 * RUN);
+        b += (w % 8) * RUN + w / 8 - w;
     }
+    if (grid3d) {
+        const uint32_t plane = gridDim.x * gridDim.y, r = b % plane;
+        return TileAt{ (int)(b / plane), (int)(r % gridDim.x), (int)(r / gridDim.x) };
+    }
+    const uint2 m = tile_map[b];
+    return TileAt{ (int)m.x, (int)(m.y & 0xFFFFu), (int)(m.y >> 16) };
 }
 
 // ---------------------------------------------------------------------------
-// kf_raster: heuristic crossing resolution, cells (+ subdivision) and the
-// gather raster of a tile of cells
+// kf_raster: heuristic crossing resolution, cells and the gather raster of a
+// tile of cells
 // ---------------------------------------------------------------------------
 // Raster tiles of TX x (256 / TX) cells, one own cell per thread of a
 // 256-thread block (32x8 by default; 16x16 and 64x4 are the other shapes an
@@ -161,14 +155,10 @@ constexpr uint16_t kNoCell = 0xFFFF;
 
 // LDS windows of the raster tile hold graph bytes in rows of WW 32-bit
 // words; word w of a row holds x = x0 - 8 + 4w .. x0 - 5 + 4w.  Words
-// 1..DW (x0 - 4 .. x0 + X + 3) carry data, words 0 and DW + 1 stay zero.  Candidate cells
-// (halo 1) need the resolved bytes of their left and right neighbours for
-// their keys: resolved rows at halo 1; with subdivision the hulls at halo 2
-// are needed as well: resolved rows at halo 2.  Resolving a byte reads the
-// snapshot rows above and below it.
-// Resolved rows y0 - 1 .. y0 + Y (GY rows: candidate cells need their left
-// and right neighbours' bytes for their keys); resolving them reads one more
-// snapshot row on each side (AY rows).
+// 1..DW (x0 - 4 .. x0 + X + 3) carry data, words 0 and DW + 1 stay zero.
+// Resolved rows y0 - 1 .. y0 + Y (GY rows: the candidate cells' rows, whose
+// keys take the bytes left and right of them too); resolving them reads one
+// more snapshot row on each side (AY rows).
 #define DPX_TILE_NAMES(TX)                                                                                 \
     using TS = TileShape<TX>;                                                                              \
     constexpr int RTX = TS::X, RTY = TS::Y, RCX = TS::CX, RCY = TS::CY, RWW = TS::WW, RWB = TS::WB;        \
@@ -176,8 +166,8 @@ constexpr uint16_t kNoCell = 0xFFFF;
     (void)RTX; (void)RTY; (void)RCX; (void)RCY; (void)RWW; (void)RWB; (void)GY; (void)AY; (void)RDW; (void)RDB
 
 // Per-cell coverage of smoothed cells (kf_smooth -> kf_raster<S, true>): up to
-// 8x the nine cell masks and the coverage summary, from 9x MW words of sample
-// rows and one of summary; cell (x, y) of an item at word (y * W + x) *
+// 8x the nine cell masks and the coverage summary, from 9x cover_h(S) words of
+// sample rows and one of summary; cell (x, y) of an item at word (y * W + x) *
 // rows_words(S) of its range.
 __host__ __device__ constexpr int rows_words(int S) { return (int)cell_row_words(S); }
 

@@ -43,8 +43,9 @@
 // the ranking's launches in front of them; bytes and arithmetic are small
 // (640x480: 272 k links of 12 B).  Measured, against one wave that took the
 // walks in scan order (a microsecond a walk): dithered 640x480 frames 6.3 ->
-// 0.55 ms, those with a face of thousands of abandoned walks 9-13 -> 3.3-3.9
-// ms; 256x224 game frames 0.61-1.64 -> 0.30-0.81 ms; 64x48 0.29 -> 0.16 ms.
+// 0.4-1.2 ms, one in eight, with a face of thousands of abandoned walks, 9-13 ->
+// 3.1-3.9 ms; 256x224 game frames 0.60-1.64 -> 0.27-0.80 ms; 64x48 0.29 -> 0.16;
+// game frames of 1280x960 39-99 -> 4-42 ms, dithered ones 45-50 -> 1.5-1.6.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -64,7 +65,7 @@ constexpr uint32_t kStartBit = 0x80000000u; // flag beside a position's node: th
 constexpr int kShort = 512;                 // positions of a path that one wave holds in registers
 constexpr int kLong = 8192;                 // positions of a path that fit a block's LDS
 constexpr int kSimBlock = 512;
-// Frames of more nodes need an aligned scratch (include/depixel.h).
+// Frames of more nodes are refused without an aligned scratch (include/depixel.h), though none is used.
 constexpr uint32_t kScratchUnalignedNodes = 622336;
 constexpr int kGridRounds = 8;  // rounds as launches over the machine; k_bc_finish does the rest
 

@@ -1,32 +1,32 @@
 // fused.hip -- the batched path: many frames or sprites of uneven size
-// through two fused kernels.
+// through two fused kernels, three with subdivision.
 //
-//   kf_graph   strip of 64 columns of a row block, one wave: lane words (YUV fields + class) once
-//              per pixel, similarity in four directions (the other four by
-//              symmetry) with block flags for the trivial crossing removal
-//              -> snapshot graph (1 B/px)
-//   kf_raster  tile of 32x8 cells: heuristic crossing resolution on the
-//              snapshot (crossed blocks listed and decided once), cell keys
-//              (and, with subdivision, hulls, smoothed polygons and their
-//              coverage) in LDS; cells whose S*S pixels are all their own
-//              colour are simple, the rest are listed and resolved row by
-//              row (up to 7x: cell by cell) against the 3x3 candidate cells
-//              in draw order into an LDS pixel buffer; then every row of
-//              the tile's output is stored once, simple and resolved pixels
-//              by the same store instructions.
+//   kf_graph   strip of 62 columns of a row block, one wave: lane words (YUV
+//              fields + class) once per pixel, similarity in four directions
+//              (the other four by symmetry) and the trivial crossing removal
+//              on row masks in scalar registers -> snapshot graph (1 B/px)
+//   kf_raster  tile of 32x8 cells (or 16x16, 64x4): heuristic crossing
+//              resolution on the snapshot (crossed blocks listed and decided
+//              once), cell keys and coverage summaries in LDS; cells whose S*S
+//              pixels are all their own colour are simple, the rest are
+//              listed and resolved (cell by cell at 1x to 7x, row by row from
+//              8x) against the 3x3 candidate cells in draw order; then every
+//              row of the tile's output is stored once, simple and resolved
+//              pixels by the same store instructions.
 //
 // Coverage of an unsmoothed cell depends only on its 12-bit key and the
 // scale, so it is precomputed once per scale into a table of sample-row
 // bitmasks (kt_mask): bit b of row r of key k says whether sample
 // (kmin+b, kmin+r) of the cell's local sample grid is covered, kmin =
-// -(S/2)-1, MW = 2S+2 rows and columns (local [-0.5, 1.5] of the cell); into
-// a summary byte per key (kt_info, coverage_info's low bits); and at 1x to 8x into
-// each key's sample mask of each neighbour cell (kt_cell).
+// -(S/2)-1, MW = 2S+2 rows and columns (a hull lies within -0.25 .. 1.25 of
+// the cell); into a summary byte per key (kt_info, coverage_info's low bits);
+// and at 1x to 8x into each key's sample mask of each neighbour cell (kt_cell).
 //
-// With subdivision, kf_smooth runs between the two: it resolves the
-// crossings of each tile, smooths and ear-clips its non-internal cells
-// (polygons in LDS, each own cell once) and writes their coverage rows; the
-// raster (kf_raster<S, true>) then reads the resolved graph and those rows.
+// With subdivision, kf_smooth runs between the two: it resolves the crossings
+// of each tile, smooths its non-internal cells (polygons in LDS, each own
+// cell once) and writes their coverage, as cell masks up to 8x and as sample
+// rows from 9x; the raster (kf_raster<S, true>) then reads the resolved graph
+// and that coverage, and resolves no crossings.
 #include <dlfcn.h>
 #include <stdio.h>
 #include <stdlib.h>

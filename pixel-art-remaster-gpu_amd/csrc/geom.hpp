@@ -508,17 +508,6 @@ __host__ __device__ inline int ear_clip(const int* x, const int* y, int n, uint8
     return ntri;
 }
 
-// ear_clip on at most MAXN <= 16 vertices in counter-clockwise order, for
-// one lane of a wave: vertex k at P[stride * k], packed.  ear(A, B, C)
-// receives each triangle as it is cut; returns the number of vertices left (2
-// when the polygon is cut wholly).  The vertices stay where they are: a mask
-// holds those not cut off yet, and the three at hand move along it (after an
-// ear the walk goes on at its third corner, else at its second, which is
-// where ear_clip's index stands in its shortened list).  The test of the
-// other vertices is unrolled over registers, two multiply-adds an edge: a
-// loop over a list in LDS costs a read, two unpackings and three comparisons
-// of indices a vertex more.  Products are taken modulo 2^32, as ear_clip's
-// are; coordinates are 16 bits.
 __host__ __device__ inline int mad24(int a, int b, int c);
 
 // Vertices packed x | y << 16 (16 bits each) or x | y << 8 (8 bits each).
@@ -603,6 +592,18 @@ __host__ __device__ inline int mad24(int a, int b, int c)
 #endif
 }
 
+// ear_clip on at most MAXN <= 16 vertices in counter-clockwise order, for
+// one lane of a wave: vertex k at P[stride * k], packed.  ear(A, B, C)
+// receives each triangle as it is cut; returns the number of vertices left (2
+// when the polygon is cut wholly).  The vertices stay where they are: a mask
+// holds those not cut off yet, and the three at hand move along it (after an
+// ear the walk goes on at its third corner, else at its second, which is
+// where ear_clip's index stands in its shortened list).  The test of the
+// other vertices is unrolled over registers, two multiply-adds an edge: a
+// loop over a list in LDS costs a read, two unpackings and three comparisons
+// of indices a vertex more.  Products are taken modulo 2^32, as ear_clip's
+// are; coordinates are 16 bits.
+//
 // With `test` false (the caller knows the polygon to be strictly convex) no
 // vertex can lie in another three's triangle, and none is looked at.  That
 // reasoning is about the plane, so it takes coordinates whose products are not
