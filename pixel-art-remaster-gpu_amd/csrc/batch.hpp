@@ -379,9 +379,9 @@ __device__ inline void tile_resolved_load(const DevItem& it, const uint8_t* __re
 // triangles cut so far are the cell), runs for the few polygons for which
 // that is not plain, gathered into the first lanes.  The cells are listed by
 // the size of their hull, so that the lanes of a wave end together.  16 frames
-// of 640x480 at 8x: 290 us (606 with every row of every edge visited, every
+// of 640x480 at 8x: 293 us (606 with every row of every edge visited, every
 // cell clipped, and hulls and colours read per vertex); 64 of 251x223 at 4x:
-// 128 (334).
+// 127 (334).
 // ---------------------------------------------------------------------------
 // Blocks a CU, for which the registers are allotted: as many as their LDS
 // leaves room for (a wave waits for two thirds of its time, most of it at

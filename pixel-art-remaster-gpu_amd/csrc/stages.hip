@@ -560,7 +560,7 @@ __device__ __noinline__ uint32_t tri_sample_any(ImgView im, const dpx_point* __r
 // nearly similar colours took that in most blocks: the raster of 256x224 at 8x
 // 546 us, so 151, the window at 8x 719, so 96.)
 // Bound by the instructions of the tests; straight from memory in 64 bits
-// the 1200x800 window of a smoothed 256x224 frame took 221 us, so 44.
+// the 1200x800 window of a smoothed 256x224 frame took 221 us, so 40.
 constexpr int kTris = kCellSize / 3;
 constexpr int kTriLow = std::min(kReachXLow, kReachYLow), kTriHigh = std::max(kReachXHigh, kReachYHigh);  // 1/64 units
 constexpr long long kTriUnitMost = 512 * 3200, kTriStep = 8 * 6400;  // of the window, the larger ones
